@@ -45,12 +45,6 @@ struct Layer {
 
 constexpr int kPad = 8;   // zero positions after the nz bins
 
-__global__ void k_add(float* __restrict__ dst, const float* __restrict__ src, size_t n)
-{
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) dst[i] += src[i];
-}
-
 // u[i] = (lnk[idx[i]] - mu) * inv_sigma (idx null: identity)
 __global__ void k_norm_u(const float* __restrict__ lnk, const uint32_t* __restrict__ idx,
                          float* __restrict__ u, int n, float mu, float inv_sigma)
@@ -76,7 +70,9 @@ struct NetImpl {
   size_t nparam = 0;
   float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   uint16_t *wt = nullptr, *wb = nullptr;
-  unet::FilmLayer* d_film = nullptr;       // scale offsets for max_b samples
+  unet::WeightLayer* d_wl = nullptr;       // the layers' weights
+  unet::FilmLayer* d_film = nullptr;       // scale offsets for film_b samples
+  int film_b = 0;
   unet::FilmLayer* d_film_inf = nullptr;   // ... for inf_b samples
   size_t scale_per_sample = 0;       // sum of the layers' Cout
   // training / evaluation buffers for max_b samples
@@ -85,6 +81,7 @@ struct NetImpl {
   float *scale = nullptr, *dpre = nullptr, *xb = nullptr, *tb = nullptr, *ub = nullptr;
   float *lossb = nullptr, *hist = nullptr;
   uint32_t* idx = nullptr;
+  size_t idx_cap = 0;
   int hist_cap = 0;
   // inference buffers (the batch engine) for inf_b samples
   int inf_b = 0;
@@ -143,16 +140,14 @@ void free_net(NetImpl* n)
                    n->hist, n->iscale, n->data.x, n->data.y, n->data.u})
     (void)hipFree(p);
   (void)hipFree(n->wt); (void)hipFree(n->wb); (void)hipFree(n->idx); (void)hipFree(n->d_film);
-  (void)hipFree(n->d_film_inf);
+  (void)hipFree(n->d_film_inf); (void)hipFree(n->d_wl);
   (void)hipFree(n->data.count);
   free_bufs(n->pre); free_bufs(n->out); free_bufs(n->dy); free_bufs(n->iout);
 }
 
 int refresh_bf16(NetImpl* n)
 {
-  for (const Layer& l : n->layers)
-    NN_CHECK(unet::bf16_copies(n->w + l.w_off, n->wt + l.w_off, n->wb + l.w_off, l.cout, l.taps,
-                               l.cin, n->s));
+  NN_CHECK(unet::bf16_copies(n->w, n->wt, n->wb, n->d_wl, (int)n->layers.size(), n->s));
   return 0;
 }
 
@@ -187,9 +182,11 @@ int forward(NetImpl* n, const float* x, const float* u, const uint32_t* dyn_b, i
   return 0;
 }
 
-// The FiLM table for B samples per layer (scale offsets soff * B).
-int upload_film(NetImpl* n, int B, unet::FilmLayer* dst)
+// The FiLM table for B samples per layer (scale offsets soff * B); held: the
+// count dst holds the table for.
+int upload_film(NetImpl* n, int B, unet::FilmLayer* dst, int* held)
 {
+  if (*held == B) return 0;
   std::vector<unet::FilmLayer> fl(n->layers.size());
   size_t soff = 0;
   for (size_t k = 0; k < n->layers.size(); ++k) {
@@ -201,6 +198,7 @@ int upload_film(NetImpl* n, int B, unet::FilmLayer* dst)
   NN_CHECK(hipMemcpyAsync(dst, fl.data(), fl.size() * sizeof(unet::FilmLayer),
                           hipMemcpyHostToDevice, n->s));
   NN_CHECK(hipStreamSynchronize(n->s));
+  *held = B;
   return 0;
 }
 
@@ -234,7 +232,7 @@ int alloc_train(NetImpl* n, int B)
 int loss_grad(NetImpl* n, int B, bool grad)
 {
   hipStream_t s = n->s;
-  if (upload_film(n, B, n->d_film) ||
+  if (upload_film(n, B, n->d_film, &n->film_b) ||
       forward(n, n->xb, n->ub, nullptr, B, n->d_film, n->out, n->scale, grad ? &n->pre : nullptr,
               s))
     return -1;
@@ -243,16 +241,14 @@ int loss_grad(NetImpl* n, int B, bool grad)
                       n->cpad, n->zn, n->cout, 1.f / n->out_scale, B, s));
   if (!grad) return 0;
   NN_CHECK(hipMemsetAsync(n->g, 0, n->nparam * 4, s));
-  for (size_t k = 0; k + 1 < L; ++k)
-    NN_CHECK(hipMemsetAsync(n->dy[k], 0, act_size(n->layers[k], B) * 4, s));
+  // the layer whose output gradient also flows into layer k through its skip
+  std::vector<int> skip_to(L, -1);
+  for (size_t k = 0; k < L; ++k)
+    if (n->layers[k].skip >= 0) skip_to[n->layers[k].skip] = (int)k;
   size_t soff = n->scale_per_sample;
   for (size_t kk = L; kk-- > 0;) {
     const Layer& l = n->layers[kk];
     soff -= l.cout;
-    const size_t na = act_size(l, B);
-    if (l.skip >= 0)
-      hipLaunchKernelGGL(k_add, dim3((unsigned)((na + 255) / 256)), dim3(256), 0, s,
-                         n->dy[l.skip], n->dy[kk], na);
     NN_CHECK(unet::film_bwd(n->dy[kk], n->pre[kk], n->scale + soff * B, n->ub, n->dpre,
                             n->g + l.a_off, B, l.zout, l.cout, s));
     const float* in = kk == 0 ? n->xb : n->out[kk - 1];
@@ -260,12 +256,13 @@ int loss_grad(NetImpl* n, int B, bool grad)
                        l.dil, l.mode};
     NN_CHECK(unet::wgrad(wa, s));
     if (kk == 0) continue;
-    // d(input) = conv^T(dpre), added into the previous layer's output gradient
+    // the previous layer's output gradient: conv^T(dpre), plus that of the
+    // layer it skips to (processed before, its gradient still in place)
     unet::ConvArgs a{};
     a.in = n->dpre;
     a.w = n->wb + l.w_off;
     a.out = n->dy[kk - 1];
-    a.skip = n->dy[kk - 1];
+    a.skip = skip_to[kk - 1] >= 0 ? n->dy[skip_to[kk - 1]] : nullptr;
     a.B = B; a.Zin = l.zout; a.Zout = l.zin; a.Cin = l.cout; a.Cout = l.cin;
     a.taps = l.taps; a.dil = l.dil;
     a.mode = l.mode == unet::kSame ? unet::kSameFlip
@@ -277,12 +274,12 @@ int loss_grad(NetImpl* n, int B, bool grad)
   return 0;
 }
 
-// x (host or device) [B][zn_in][cin] rows into xb [B][Z0][cin] (zero padding)
+// x (host or device) [B][zn_in][cin] rows into xb [B][Z0][cin] (its padding
+// rows are zero from its allocation on)
 int stage_inputs(NetImpl* n, const float* x, const float* lnk, const float* y, int B,
                  hipMemcpyKind kind)
 {
   const size_t row = (size_t)n->nz * n->cin;
-  NN_CHECK(hipMemsetAsync(n->xb, 0, (size_t)B * n->Z0 * n->cin * 4, n->s));
   NN_CHECK(hipMemcpy2DAsync(n->xb, (size_t)n->Z0 * n->cin * 4, x, row * 4, row * 4, B, kind, n->s));
   if (y)
     NN_CHECK(hipMemcpyAsync(n->tb, y, (size_t)B * n->zn * n->cout * 4, kind, n->s));
@@ -325,7 +322,8 @@ int net_reserve_infer(NetImpl* n, int B)
     n->iout.push_back(p);
   }
   NN_CHECK(hipMalloc(&n->iscale, n->scale_per_sample * B * 4));
-  return upload_film(n, B, n->d_film_inf);
+  int held = 0;
+  return upload_film(n, B, n->d_film_inf, &held);
 }
 
 int net_data(NetImpl* n, NetData* out)
@@ -371,10 +369,19 @@ int hps_nn_create(hps_nn** out, uint32_t nr, uint32_t nz, const uint32_t* widths
   for (float** p : {&n->w, &n->g, &n->m, &n->v}) ok = ok && hipMalloc(p, np) == hipSuccess;
   ok = ok && hipMalloc(&n->wt, n->nparam * 2) == hipSuccess &&
        hipMalloc(&n->wb, n->nparam * 2) == hipSuccess &&
+       hipMalloc(&n->d_wl, n->layers.size() * sizeof(unet::WeightLayer)) == hipSuccess &&
        hipMalloc(&n->d_film, n->layers.size() * sizeof(unet::FilmLayer)) == hipSuccess &&
        hipMalloc(&n->d_film_inf, n->layers.size() * sizeof(unet::FilmLayer)) == hipSuccess &&
        hipMalloc(&n->data.count, 4) == hipSuccess && hipMemset(n->data.count, 0, 4) == hipSuccess;
   if (!ok) { free_net(n); delete h; return fail_msg("surrogate allocation failed"); }
+  std::vector<unet::WeightLayer> wl;
+  for (const Layer& l : n->layers) wl.push_back({l.cout, l.taps, l.cin, 0, l.w_off});
+  if (hipMemcpy(n->d_wl, wl.data(), wl.size() * sizeof(unet::WeightLayer),
+                hipMemcpyHostToDevice) != hipSuccess) {
+    free_net(n);
+    delete h;
+    return fail_msg("surrogate initialisation failed");
+  }
   // He-style initialisation scaled for a deep linear network: each layer
   // keeps the signal variance (std = 1/sqrt(taps * Cin)); FiLM coefficients 0
   std::vector<float> p(n->nparam, 0.f);
@@ -579,7 +586,7 @@ int hps_nn_predict(hps_nn* h, const float* x, const float* lnk, uint32_t count, 
     const int B = (int)std::min<uint32_t>((uint32_t)n->max_b, count - c0);
     if (stage_inputs(n, x + (size_t)c0 * n->nz * n->cin, lnk + c0, nullptr, B,
                      hipMemcpyHostToDevice) ||
-        upload_film(n, B, n->d_film) ||
+        upload_film(n, B, n->d_film, &n->film_b) ||
         forward(n, n->xb, n->ub, nullptr, B, n->d_film, n->out, n->scale, nullptr, n->s))
       return -1;
     // rows of the node positions, channels of the field, times the output scale
@@ -631,24 +638,35 @@ int hps_nn_train(hps_nn* h, uint32_t first, uint32_t count, uint32_t steps, uint
     NN_CHECK(hipMalloc(&n->hist, (size_t)steps * 4));
     n->hist_cap = (int)steps;
   }
-  if (!n->idx) NN_CHECK(hipMalloc(&n->idx, (size_t)n->max_b * 4));
-  const size_t rx = (size_t)n->nz * n->cin, ry = (size_t)n->zn * n->cout;
+  // the sample indices of up to kPickSteps steps go up together
+  constexpr uint32_t kPickSteps = 1024;
+  const size_t picks = (size_t)std::min(steps, kPickSteps) * batch;
+  if (picks > n->idx_cap) {
+    (void)hipFree(n->idx);
+    n->idx = nullptr;
+    n->idx_cap = 0;
+    NN_CHECK(hipMalloc(&n->idx, picks * 4));
+    n->idx_cap = picks;
+  }
   std::mt19937 rng(seed);
   std::uniform_int_distribution<uint32_t> pick(first, first + count - 1);
-  std::vector<uint32_t> idx(batch);
+  std::vector<uint32_t> idx;
   const int B = (int)batch;
+  unet::BatchArgs ba{};
+  ba.x = n->data.x; ba.y = n->data.y; ba.u = n->data.u;
+  ba.xb = n->xb; ba.tb = n->tb; ba.ub = n->ub;
+  ba.B = B; ba.row_x = n->nz * n->cin; ba.stride_x = n->Z0 * n->cin; ba.row_y = n->zn * n->cout;
+  ba.mu = n->u_mu; ba.inv_sigma = 1.f / n->u_sigma;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (uint32_t st = 0; st < steps; ++st) {
-    for (auto& i : idx) i = pick(rng);
-    NN_CHECK(hipMemcpyAsync(n->idx, idx.data(), batch * 4, hipMemcpyHostToDevice, n->s));
-    // inputs: the nz bin rows into the zero-padded Z0 rows
-    NN_CHECK(hipMemsetAsync(n->xb, 0, (size_t)B * n->Z0 * n->cin * 4, n->s));
-    NN_CHECK(unet::gather(n->data.x, n->idx, n->tb, B, (int)rx, n->s));   // staging in tb
-    NN_CHECK(hipMemcpy2DAsync(n->xb, (size_t)n->Z0 * n->cin * 4, n->tb, rx * 4, rx * 4, B,
-                              hipMemcpyDeviceToDevice, n->s));
-    NN_CHECK(unet::gather(n->data.y, n->idx, n->tb, B, (int)ry, n->s));
-    hipLaunchKernelGGL(k_norm_u, dim3((B + 255) / 256), dim3(256), 0, n->s, n->data.u, n->idx,
-                       n->ub, B, n->u_mu, 1.f / n->u_sigma);
+    if (st % kPickSteps == 0) {
+      NN_CHECK(hipStreamSynchronize(n->s));
+      idx.resize((size_t)std::min(steps - st, kPickSteps) * batch);
+      for (auto& i : idx) i = pick(rng);
+      NN_CHECK(hipMemcpy(n->idx, idx.data(), idx.size() * 4, hipMemcpyHostToDevice));
+    }
+    ba.idx = n->idx + (size_t)(st % kPickSteps) * batch;
+    NN_CHECK(unet::stage(ba, n->s));
     if (loss_grad(n, B, true)) return -1;
     ++n->step;
     // cosine decay from lr to lr_end over the call

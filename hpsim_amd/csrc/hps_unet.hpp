@@ -22,7 +22,7 @@ constexpr int kWgradChunk = 256;     // positions per weight-gradient task
 
 struct ConvArgs {
   const float* in;          // [B][Zin][Cin]
-  const uint16_t* w;        // BF16 [Cout][taps][Cin]
+  const uint16_t* w;        // BF16 [Cout][taps][Cin] in operand order (k_bf16)
   float* pre;               // optional: the product before scale and skip
   float* out;               // [B][Zout][Cout]
   const float* scale;       // optional [B][Cout]
@@ -45,6 +45,21 @@ struct FilmLayer {
   size_t s_off;             // this layer's scales [max_b][cout] in the scale buffer
 };
 
+// one layer's weights in the flat parameter vector
+struct WeightLayer {
+  int cout, taps, cin, pad_;
+  size_t w_off;
+};
+
+// a training batch gathered from the dataset by sample index
+struct BatchArgs {
+  const float *x, *y, *u;   // dataset rows: row_x and row_y floats, log aspects
+  const uint32_t* idx;      // [B] samples
+  float *xb, *tb, *ub;      // [B][stride_x], [B][row_y], [B] (standardised)
+  int B, row_x, stride_x, row_y;
+  float mu, inv_sigma;
+};
+
 hipError_t conv(const ConvArgs& a, hipStream_t s);
 hipError_t wgrad(const WgradArgs& a, hipStream_t s);
 hipError_t film(const float* params, const FilmLayer* layers, int nlayers, const float* u,
@@ -57,8 +72,9 @@ hipError_t loss(const float* y, const float* tgt, float* dy, float* l, int Z0, i
                 int cout, float inv_scale, int B, hipStream_t s);
 hipError_t adam(float* w, const float* g, float* m, float* v, int n, float lr_t, float b1,
                 float b2, float eps, hipStream_t s);
-hipError_t bf16_copies(const float* w, uint16_t* wt, uint16_t* wb, int Cout, int taps, int Cin,
-                       hipStream_t s);
+hipError_t bf16_copies(const float* params, uint16_t* wt, uint16_t* wb, const WeightLayer* layers,
+                       int nlayers, hipStream_t s);
+hipError_t stage(const BatchArgs& a, hipStream_t s);
 hipError_t gather(const float* src, const uint32_t* idx, float* dst, int n, int row,
                   hipStream_t s);
 

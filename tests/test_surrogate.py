@@ -116,6 +116,44 @@ def test_gpu_network_matches_reference_forward_and_gradient():
             assert e < 2e-2, (r, e)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("nr,nz,widths,nbot,B", [
+    (16, 64, (16, 16, 16, 16), 1, 1),        # one channel tile, 72 positions: a partial tile
+    (32, 128, (48, 64, 96, 96), 4, 33),      # two position tiles per workgroup, odd sample count
+    (64, 64, (144, 16, 144, 32), 2, 5)])     # the widest layers, the most product steps
+def test_gpu_network_layer_shapes_match_reference(nr, nz, widths, nbot, B):
+    """Forward pass and gradient at the edges of the layer kernels' tiles.
+    Weights are BF16 on both sides; activations carry 17 bits (two BF16
+    terms) on the GPU forward, 9 bits in the weight gradient's left operand:
+    1e-4 forward, 1e-2 gradient as in the test above."""
+    from hpsim_amd.surrogate import Network
+    net = Network(nr=nr, nz=nz, widths=widths, nbot=nbot, max_batch=B, seed=9)
+    table, n = _table(nr, net.cpad, widths, nbot)
+    net.set_norm(1.0, 0.0, 1.0)
+    rng = np.random.default_rng(21)
+    p = net.params()
+    film = np.zeros(n, bool)
+    for r in table:
+        film[r[7]:r[7] + 3 * r[2]] = True
+    p[film] = rng.normal(0, 0.2, film.sum()).astype(np.float32)
+    net.set_params(p)
+    x = rng.normal(0, 1, (B, nz, nr)).astype(np.float32)
+    u = rng.normal(0, 0.6, B).astype(np.float32)
+    y = rng.normal(0, 1, (B, nz + 1, 2 * (nr + 1))).astype(np.float32)
+    pr = p.astype(np.float64)
+    pr[~film] = R.bf16(p[~film])
+    xr = np.zeros((B, net.Z0, nr))
+    xr[:, :nz] = x
+    want = R.forward(pr, table, xr, u.astype(np.float64))[:, :nz + 1, :2 * (nr + 1)]
+    got = net.predict(x, u)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-4
+    loss, g = net.loss_grad(x, u, y)
+    rl, rg = R.loss_and_grad(pr, table, xr, u.astype(np.float64), y.astype(np.float64), nz + 1,
+                             2 * (nr + 1))
+    assert np.allclose(loss, rl, rtol=1e-4)
+    assert np.linalg.norm(g - rg) / np.linalg.norm(rg) < 1e-2
+
+
 def _train_small(steps=20000):
     """A small network trained on the grouped SCHEFF solves of two short
     tracking runs (scan members and beams of the accelerating lattice)."""
