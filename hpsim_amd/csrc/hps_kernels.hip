@@ -112,85 +112,94 @@ __device__ __forceinline__ double block_max(double v, double* buf, int t)
   return r;
 }
 
-// Thread t's entries c = t + 256 k, k < K, of the cross-chunk trees below
-// (mpad = 256 K, or K = 1 and mpad <= 256): the Q partial sums folded by the
-// upper levels of the halving tree, the integer counts C[c] of c < nch (C
-// may be null), and, when M is given, the largest M[c] of c < nch (-inf if
-// none; a NaN entry is never taken).  Every load is issued before the first
-// addition, so the K * (Q + 2) loads share one round trip.
-template <int Q, int K>
-__device__ __forceinline__ void fold_entries(const double* P, const uint32_t* C, const double* M,
-                                             uint32_t mpad, uint32_t nch, int t, double (&v)[Q],
-                                             uint32_t& cnt, double& mx)
+// --- cross-chunk trees ------------------------------------------------------
+//
+// A quantity's chunk partials P[0, mpad) (zero padded to mpad, a power of two
+// of at most 4,096) are summed by one wavefront: lane l holds the entries
+// l + 64 m, folds them over m as the upper levels of the halving tree, and the
+// lanes' values meet in shuffles.  The waves of the one workgroup take
+// different quantities, so the sums need no LDS and no barrier among
+// themselves; what bounds them is the memory round trip, so the loads of up
+// to 16 entries a lane are issued before the first addition.
+
+// sum of the tree over P (valid in lane 0)
+template <int M>
+__device__ __forceinline__ double wave_tree(const double* P, uint32_t mpad, int l)
 {
-  const bool in = K > 1 || (uint32_t)t < mpad;
-  double r[Q][K];
-  uint32_t n[K];
-  double m[K];
+  // entries m = g + kG k of batch g fold over k (the upper levels), then the
+  // batches over g: (0 + 2) + (1 + 3) of four, 0 + 1 of two
+  constexpr int kN = M < 16 ? M : 16, kG = M / kN;
+  static_assert(kG <= 4, "at most 4,096 entries");
+  const auto batch = [&](int g) {
+    double r[kN];
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const uint32_t c = (uint32_t)t + kBlock * k;
+    for (int k = 0; k < kN; ++k)
+      r[k] = (M > 1 || (uint32_t)l < mpad) ? gld(P, l + 64 * (g + kG * k)) : 0.0;
 #pragma unroll
-    for (int q = 0; q < Q; ++q) r[q][k] = in ? gld(P, (size_t)q * mpad + c) : 0.0;
-    n[k] = (C && in) ? gld(C, c) : 0u;
-    m[k] = (M && in) ? gld(M, c) : -__builtin_huge_val();
-  }
+    for (int h = kN / 2; h >= 1; h /= 2) {
 #pragma unroll
-  for (int q = 0; q < Q; ++q) {
-#pragma unroll
-    for (int h = K / 2; h >= 1; h /= 2) {
-#pragma unroll
-      for (int k = 0; k < h; ++k) r[q][k] = r[q][k] + r[q][k + h];
+      for (int k = 0; k < h; ++k) r[k] = r[k] + r[k + h];
     }
-    v[q] = r[q][0];
+    return r[0];
+  };
+  double s;
+  if constexpr (kG == 1) {
+    s = batch(0);
+  } else {
+    constexpr int kH = kG / 2;
+    double v[2] = {0.0, 0.0};
+#pragma unroll 1
+    for (int j = 0; j < kG; ++j) {   // 0, kH, 1, kH + 1: one batch's registers at a time
+      const double x = batch((j & 1) * kH + (j >> 1));
+      if ((j & 1) == 0) v[1] = x;
+      else v[0] = j == 1 ? v[1] + x : v[0] + (v[1] + x);
+    }
+    s = v[0];
   }
-  cnt = 0;
-  mx = -__builtin_huge_val();
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const bool live = (uint32_t)t + kBlock * k < nch;
-    cnt += live ? n[k] : 0u;
-    if (live && m[k] > mx) mx = m[k];
+  for (int o = 32; o >= 1; o >>= 1) s = s + __shfl_down(s, o, 64);
+  return s;
+}
+
+__device__ __forceinline__ double wave_tree_sum(const double* P, uint32_t mpad, int l)
+{
+  switch (mpad > 64 ? mpad / 64 : 1u) {
+    case 1: return wave_tree<1>(P, mpad, l);
+    case 2: return wave_tree<2>(P, mpad, l);
+    case 4: return wave_tree<4>(P, mpad, l);
+    case 8: return wave_tree<8>(P, mpad, l);
+    case 16: return wave_tree<16>(P, mpad, l);
+    case 32: return wave_tree<32>(P, mpad, l);
+    default: return wave_tree<64>(P, mpad, l);
   }
 }
 
-// Cross-chunk trees of Q quantities stored P[q * mpad + c] (zero padded to
-// mpad, a power of two) and the sum of the integer counts C[0, nch).  Thread
-// t first folds its entries t + 256k in registers (the upper levels of the
-// halving tree), then one block tree finishes.  Every thread gets the
-// results; with M given, *own_max receives the largest M[c] over the
-// thread's own entries c < nch.  mpad <= 4096 (16 entries per thread).
-template <int Q>
-__device__ void final_reduce(const double* P, const uint32_t* C, uint32_t mpad, uint32_t nch,
-                             double* red, uint32_t* ured, double* mred, int t, double (&out)[Q],
-                             uint32_t& cnt_out, const double* M = nullptr,
-                             double* own_max = nullptr)
+// sum of the counts C[0, n) (valid in lane 0)
+__device__ __forceinline__ uint32_t wave_count(const uint32_t* C, uint32_t n, int l)
 {
-  double v[Q];
-  uint32_t cnt;
-  double own;
-  switch (mpad > (uint32_t)kBlock ? mpad / kBlock : 1u) {
-    case 1: fold_entries<Q, 1>(P, C, M, mpad, nch, t, v, cnt, own); break;
-    case 2: fold_entries<Q, 2>(P, C, M, mpad, nch, t, v, cnt, own); break;
-    case 4: fold_entries<Q, 4>(P, C, M, mpad, nch, t, v, cnt, own); break;
-    case 8: fold_entries<Q, 8>(P, C, M, mpad, nch, t, v, cnt, own); break;
-    default: fold_entries<Q, 16>(P, C, M, mpad, nch, t, v, cnt, own); break;
-  }
-  if (own_max) *own_max = own;
-  double mx = 0.0;
-  block_reduce<Q>(v, cnt, mx, red, ured, mred, t);
-  __shared__ double bcast[kMaxQ];
-  __shared__ uint32_t bcnt;
-  if (t == 0) {
+  uint32_t v = 0;
+#pragma unroll 16
+  for (uint32_t c = l; c < n; c += 64) v += gld(C, c);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) bcast[q] = v[q];
-    bcnt = cnt;
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_down(v, o, 64);
+  return v;
+}
+
+// largest of M[0, n), from v0 up (a NaN entry is never taken; valid in lane 0)
+__device__ __forceinline__ double wave_max(const double* M, uint32_t n, double v0, int l)
+{
+  double v = v0;
+#pragma unroll 8
+  for (uint32_t c = l; c < n; c += 64) {
+    const double u = gld(M, c);
+    if (u > v) v = u;
   }
-  __syncthreads();
 #pragma unroll
-  for (int q = 0; q < Q; ++q) out[q] = bcast[q];
-  cnt_out = bcnt;
-  __syncthreads();
+  for (int o = 32; o >= 1; o >>= 1) {
+    const double u = __shfl_down(v, o, 64);
+    if (u > v) v = u;
+  }
+  return v;
 }
 
 __device__ __forceinline__ bool is_good(uint32_t loss, uint32_t lloss)
@@ -373,45 +382,55 @@ struct RedSmem {
 __device__ void chunk_flag_stats_wave(const BeamArrays& b, uint32_t c, double thr, int lane,
                                       const Partials& pr)
 {
-  constexpr int kSlots = kBlock / 64;
-  double acc[kSlots][kScQ];
+  static_assert(kBlock == 256, "the folds below are written for 256 canonical lanes");
   uint32_t cnt = 0;
   double mx = -__builtin_huge_val();
-#pragma unroll
-  for (int sl = 0; sl < kSlots; ++sl) {
-#pragma unroll
-    for (int q = 0; q < kScQ; ++q) acc[sl][q] = 0.0;
+  // canonical lanes lane + 64 sl: the sums of one sl from its four particles,
+  // all loaded (at clamped indexes) before the first is used
+  const auto slot = [&](int sl, double (&acc)[kScQ]) {
+    double phi[kPerLane], x[kPerLane], y[kPerLane], w[kPerLane];
+    uint32_t loss[kPerLane], lloss[kPerLane];
 #pragma unroll
     for (int j = 0; j < (int)kPerLane; ++j) {
       const uint32_t i = c * kChunk + j * kBlock + sl * 64 + lane;
-      double phi = 0.0, x = 0.0, y = 0.0, w = 0.0;
-      uint32_t loss = 1, lloss = 0;
-      if (i < b.n) {
-        phi = b.phi[i]; x = b.x[i]; y = b.y[i]; w = b.w[i]; loss = b.loss[i]; lloss = b.lloss[i];
-        if (phi > thr) {
-          if (lloss != 1) b.lloss[i] = 1;
-          lloss = 1;
-        }
-        if (lloss == 0) mx = ::fmax(mx, phi);
+      const uint32_t k = i < b.n ? i : b.n - 1;
+      phi[j] = gld(b.phi, k); x[j] = gld(b.x, k); y[j] = gld(b.y, k); w[j] = gld(b.w, k);
+      loss[j] = gld(b.loss, k); lloss[j] = gld(b.lloss, k);
+    }
+#pragma unroll
+    for (int q = 0; q < kScQ; ++q) acc[q] = 0.0;
+#pragma unroll
+    for (int j = 0; j < (int)kPerLane; ++j) {
+      const uint32_t i = c * kChunk + j * kBlock + sl * 64 + lane;
+      const bool in = i < b.n;
+      if (in && phi[j] > thr) {
+        if (lloss[j] != 1) gst(b.lloss, i, 1u);
+        lloss[j] = 1;
       }
-      const bool g = (i < b.n) && is_good(loss, lloss);
-      const double vphi = g ? phi : 0.0, vx = g ? x : 0.0, vy = g ? y : 0.0, vw = g ? w : 0.0;
-      acc[sl][0] = acc[sl][0] + vphi;
-      acc[sl][1] = acc[sl][1] + vx;
-      acc[sl][2] = acc[sl][2] + vx * vx;
-      acc[sl][3] = acc[sl][3] + vy;
-      acc[sl][4] = acc[sl][4] + vy * vy;
-      acc[sl][5] = acc[sl][5] + vw;
+      if (in && lloss[j] == 0) mx = ::fmax(mx, phi[j]);
+      const bool g = in && is_good(loss[j], lloss[j]);
+      const double vphi = g ? phi[j] : 0.0, vx = g ? x[j] : 0.0, vy = g ? y[j] : 0.0,
+                   vw = g ? w[j] : 0.0;
+      acc[0] = acc[0] + vphi;
+      acc[1] = acc[1] + vx;
+      acc[2] = acc[2] + vx * vx;
+      acc[3] = acc[3] + vy;
+      acc[4] = acc[4] + vy * vy;
+      acc[5] = acc[5] + vw;
       cnt += g ? 1u : 0u;
     }
-  }
-  static_assert(kSlots == 4, "the fold below is written for 256 canonical lanes");
-  double v[kScQ];
+  };
+  // (lane L + lane L+128) + (lane L+64 + lane L+192): levels 128 and 64
+  double v[kScQ], h[kScQ];
+#pragma unroll 1
+  for (int j = 0; j < 4; ++j) {   // slots 0, 2, 1, 3
+    double u[kScQ];
+    slot((j & 1) * 2 + (j >> 1), u);
 #pragma unroll
-  for (int q = 0; q < kScQ; ++q) {
-    const double l0 = acc[0][q] + acc[2][q];   // level 128: lane L += lane L+128
-    const double l1 = acc[1][q] + acc[3][q];   //            lane L+64 += lane L+192
-    v[q] = l0 + l1;                            // level 64
+    for (int q = 0; q < kScQ; ++q) {
+      if ((j & 1) == 0) h[q] = u[q];
+      else v[q] = j == 1 ? h[q] + u[q] : v[q] + (h[q] + u[q]);
+    }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
@@ -422,9 +441,9 @@ __device__ void chunk_flag_stats_wave(const BeamArrays& b, uint32_t c, double th
   }
   if (lane == 0) {
 #pragma unroll
-    for (int q = 0; q < kScQ; ++q) pr.sums[q * pr.mpad + c] = v[q];
-    pr.cnt[c] = cnt;
-    pr.pmax[c] = mx;
+    for (int q = 0; q < kScQ; ++q) gst(pr.sums, q * pr.mpad + c, v[q]);
+    gst(pr.cnt, c, cnt);
+    gst(pr.pmax, c, mx);
   }
 }
 
@@ -914,87 +933,107 @@ __global__ __launch_bounds__(kWideBlock) void k_segment_wide(SegArgs a)
 // workgroup, makes the partials visible: the aperture loss count and
 // centroid (UpdateLoss + UpdateAvgXY), or the longitudinal-loss update and
 // good moments of the space-charge statistics.
+//
+// kFinalBlock threads: the first eight waves reduce a quantity each; all
+// sixteen rescan chunks.
+constexpr uint32_t kFinalBlock = 1024;
+constexpr uint32_t kRescan = 256;   // chunks of one rescan round
+
 __device__ __forceinline__ void seg_final_body(const SegArgs& a)
 {
-  __shared__ RedSmem sm;
-  __shared__ uint32_t rescan_list[64];
+  __shared__ double sum[kScQ];
+  __shared__ double pm;
+  __shared__ uint32_t good;
+  __shared__ uint32_t rescan_list[kRescan];
   __shared__ uint32_t rescan_n;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, l = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const BeamArrays& b = a.b;
   const Partials& pr = a.pr;
+  hps_beam_stats* st = a.st;
   if (a.stats == STAT_APERTURE) {
-    double s[2];
-    uint32_t nloss;
-    final_reduce<2>(pr.sums, pr.cnt, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, s, nloss);
+    if (wave < 2) {
+      const double v = wave_tree_sum(pr.sums + (size_t)wave * pr.mpad, pr.mpad, l);
+      if (l == 0) sum[wave] = v;
+    } else if (wave == 2) {
+      const uint32_t n = wave_count(pr.cnt, pr.nch, l);
+      if (l == 0) good = n;
+    }
+    __syncthreads();
     if (t == 0) {
-      hps_beam_stats* st = a.st;
+      const uint32_t nloss = good;
       st->num_loss = nloss;
       const double surv = (double)(uint32_t)(b.n - nloss);
-      st->x_avg = s[0] / surv;
-      st->y_avg = s[1] / surv;
+      st->x_avg = sum[0] / surv;
+      st->y_avg = sum[1] / surv;
     }
     return;
   }
 
   // STAT_SC: the longitudinal-loss update of Beam::UpdateLongitudinalLoss
   // (beam.cpp:776-782), then the good moments of beam.cpp:1008-1014.
-  hps_beam_stats* st = a.st;
   const uint32_t num_loss = st->num_loss;
-  // the chunk maxima are loaded together with the partials (one round trip)
-  double s[kScQ];
-  uint32_t g1;
-  double pm;
-  final_reduce<kScQ>(pr.sums, pr.cnt, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, s, g1,
-                     pr.pmax, &pm);
-  const double avg1 = g1 > 0 ? s[0] / (double)g1 : -99999;
-  const double thr = avg1 + TWOPI + PI;
-  // Chunks where a not-yet-flagged particle is beyond the threshold get their
-  // lloss flags set and their partials recomputed (rare: once per particle).
-  if (t == 0) rescan_n = 0;
-  __syncthreads();
-  if (pm > thr) atomicAdd(&rescan_n, 1u);
-  __syncthreads();
-  bool any = false;
-  for (uint32_t it = 0; rescan_n != 0 && it < pr.nch / 64 + 2; ++it) {
-    __syncthreads();
-    if (t == 0) rescan_n = 0;
-    __syncthreads();
-    for (uint32_t cc = t; cc < pr.nch; cc += kBlock) {
-      if (pr.pmax[cc] > thr) {
-        const uint32_t slot = atomicAdd(&rescan_n, 1u);
-        if (slot < 64) rescan_list[slot] = cc;
-      }
+  const auto moments = [&]() {
+    if (wave < kScQ) {
+      const double v = wave_tree_sum(pr.sums + (size_t)wave * pr.mpad, pr.mpad, l);
+      if (l == 0) sum[wave] = v;
+    } else if (wave == kScQ) {
+      const uint32_t n = wave_count(pr.cnt, pr.nch, l);
+      if (l == 0) good = n;
+    } else if (wave == kScQ + 1) {
+      const double m = wave_max(pr.pmax, pr.nch, -__builtin_huge_val(), l);
+      if (l == 0) pm = m;
     }
     __syncthreads();
-    const uint32_t nfound = rescan_n;
-    if (nfound == 0) break;
-    any = true;
-    const uint32_t take = nfound < 64 ? nfound : 64;
-    for (uint32_t r = (uint32_t)t / 64; r < take; r += kBlock / 64)
-      chunk_flag_stats_wave(b, rescan_list[r], thr, t & 63, pr);
+  };
+  moments();
+  const double avg1 = good > 0 ? sum[0] / (double)good : -99999;
+  const double thr = avg1 + TWOPI + PI;
+  // Chunks where a not-yet-flagged particle is beyond the threshold get their
+  // lloss flags set and their partials recomputed (rare: once per particle),
+  // a chunk per wave.  Beams that spill out of the bucket have tens to
+  // hundreds of such chunks at a kick point, hence the sixteen waves.
+  if (pm > thr) {
+    for (uint32_t it = 0; it < pr.nch / kRescan + 2; ++it) {
+      __syncthreads();
+      if (t == 0) rescan_n = 0;
+      __syncthreads();
+      for (uint32_t cc = t; cc < pr.nch; cc += kFinalBlock) {
+        if (gld(pr.pmax, cc) > thr) {
+          const uint32_t slot = atomicAdd(&rescan_n, 1u);
+          if (slot < kRescan) rescan_list[slot] = cc;
+        }
+      }
+      __syncthreads();
+      const uint32_t nfound = rescan_n;
+      if (nfound == 0) break;
+      const uint32_t take = nfound < kRescan ? nfound : kRescan;
+      for (uint32_t r = (uint32_t)wave; r < take; r += kFinalBlock / 64)
+        chunk_flag_stats_wave(b, rescan_list[r], thr, l, pr);
+    }
     __syncthreads();
+    moments();
   }
-  uint32_t g2 = g1;
-  if (any)
-    final_reduce<kScQ>(pr.sums, pr.cnt, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, s, g2);
   if (t == 0) {
+    const uint32_t g2 = good;
     st->num_good = g2;
-    st->phi_avg_good = g2 > 0 ? s[0] / (double)g2 : -99999;
+    st->phi_avg_good = g2 > 0 ? sum[0] / (double)g2 : -99999;
     const double surv = (double)(uint32_t)(b.n - num_loss);
-    const double xavg = s[1] / surv, x2avg = s[2] / surv, yavg = s[3] / surv, y2avg = s[4] / surv;
+    const double xavg = sum[1] / surv, x2avg = sum[2] / surv, yavg = sum[3] / surv,
+                 y2avg = sum[4] / surv;
     st->x_avg_good = xavg;
     st->x_sig_good = ::sqrt(x2avg - xavg * xavg);
     st->y_avg_good = yavg;
     st->y_sig_good = ::sqrt(y2avg - yavg * yavg);
-    st->w_avg_good = g2 > 0 ? s[5] / (double)g2 : -99999;
+    st->w_avg_good = g2 > 0 ? sum[5] / (double)g2 : -99999;
   }
 }
 
 
-__global__ __launch_bounds__(kBlock) void k_seg_final(SegArgs a) { seg_final_body(a); }
+__global__ __launch_bounds__(kFinalBlock) void k_seg_final(SegArgs a) { seg_final_body(a); }
 
 // one workgroup per simulation of a batch
-__global__ __launch_bounds__(kBlock) void k_seg_final_batch(const SegArgs* recs,
+__global__ __launch_bounds__(kFinalBlock) void k_seg_final_batch(const SegArgs* recs,
                                                             const uint64_t* roff)
 {
   const SegArgs a = period_recs(recs, roff)[blockIdx.x];
@@ -1191,9 +1230,11 @@ __global__ __launch_bounds__(kBlock) void k_phase_wave_batch(const PhaseArgs* re
 // device, and the cleared charge histogram
 // when it decides to remesh.  Thread 0 reads every input into registers
 // before it writes any output.
+constexpr uint32_t kPhaseFinalBlock = 512;
+
 __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
 {
-  __shared__ RedSmem sm;
+  __shared__ double sum[4];   // the three sums, the largest r^2
   __shared__ int remesh;
   __shared__ uint32_t nbins;
   const int t = threadIdx.x;
@@ -1217,25 +1258,24 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
     phi_sig_good = st->phi_sig_good;
     ss = sc->st;
   }
-  double s[3] = {0.0, 0.0, 0.0};
-  if (a.do_sums) {
-    uint32_t dummy;
-    final_reduce<3>(a.pr.sums, nullptr, a.pr.mpad, a.pr.nch, sm.red, sm.ured, sm.mred, t, s,
-                    dummy);
+  // waves 0..2: the relative-phase sums; wave 3: Beam::UpdateMaxRPhi
+  // (beam.cu:829-851), the largest r^2 about the last all-particle centroid
+  // over loss == 0, for the adjacent-bunch mesh, from the segment's chunk
+  // maxima, or directly for beams of at most two particles (no segment
+  // statistics).
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
+  if (wave < 3) {
+    const double v =
+        a.do_sums ? wave_tree_sum(a.pr.sums + (size_t)wave * a.pr.mpad, a.pr.mpad, l) : 0.0;
+    if (l == 0) sum[wave] = v;
+  } else if (wave == 3) {
+    const double v = a.rmax == 1 ? wave_max(a.pr.rmax2, a.pr.nch, 0.0, l) : 0.0;
+    if (l == 0) sum[3] = v;
   }
-  // Beam::UpdateMaxRPhi (beam.cu:829-851): the largest r^2 about the last
-  // all-particle centroid over loss == 0, for the adjacent-bunch mesh; from
-  // the segment's chunk maxima, or directly for beams of at most two
-  // particles (no segment statistics).
-  double r2max = 0.0;
-  if (a.rmax == 1) {
-    double v = 0.0;
-    for (uint32_t c = t; c < a.pr.nch; c += kBlock) {
-      const double u = a.pr.rmax2[c];
-      v = v < u ? u : v;
-    }
-    r2max = block_max(v, sm.mred, t);
-  } else if (a.rmax == 2 && t == 0) {
+  __syncthreads();
+  const double s[3] = {sum[0], sum[1], sum[2]};
+  double r2max = sum[3];
+  if (a.rmax == 2 && t == 0) {
     const double xa = st->x_avg, ya = st->y_avg;
     for (uint32_t i = 0; i < b.n; ++i) {
       if (b.loss[i] != 0) continue;
@@ -1322,12 +1362,12 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
   }
   __syncthreads();
   if (remesh)
-    for (uint32_t i = t; i < nbins; i += kBlock) a.bins[i] = 0;
+    for (uint32_t i = t; i < nbins; i += kPhaseFinalBlock) gst(a.bins, i, (int64_t)0);
 }
 
-__global__ __launch_bounds__(kBlock) void k_phase_final(PhaseArgs a) { phase_final_body(a); }
+__global__ __launch_bounds__(kPhaseFinalBlock) void k_phase_final(PhaseArgs a) { phase_final_body(a); }
 
-__global__ __launch_bounds__(kBlock) void k_phase_final_batch(const PhaseArgs* recs,
+__global__ __launch_bounds__(kPhaseFinalBlock) void k_phase_final_batch(const PhaseArgs* recs,
                                                               const uint64_t* roff)
 {
   const PhaseArgs a = period_recs(recs, roff)[blockIdx.x];
@@ -1821,22 +1861,16 @@ __global__ __launch_bounds__(kBlock) void k_sums(BeamArrays b, const double* pa,
 }
 
 // Cross-chunk trees of k_sums in one workgroup.
-__global__ __launch_bounds__(kBlock) void k_sums_final(Partials pr)
+__global__ __launch_bounds__(512) void k_sums_final(Partials pr)
 {
-  __shared__ RedSmem sm;
-  const int t = threadIdx.x;
-  double s[5];
-  uint32_t c0, c1, c2;
-  final_reduce<5>(pr.sums, pr.cnt, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, s, c0);
-  double d1[1], d2[1];
-  final_reduce<1>(pr.sums, pr.cnt + pr.mpad, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, d1, c1);
-  final_reduce<1>(pr.sums, pr.cnt + 2 * pr.mpad, pr.mpad, pr.nch, sm.red, sm.ured, sm.mred, t, d2, c2);
-  if (t == 0) {
-#pragma unroll
-    for (int q = 0; q < 5; ++q) pr.out[q] = s[q];
-    pr.out_cnt[0] = c0;
-    pr.out_cnt[1] = c1;
-    pr.out_cnt[2] = c2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (wave < 5) {
+    const double v = wave_tree_sum(pr.sums + (size_t)wave * pr.mpad, pr.mpad, l);
+    if (l == 0) pr.out[wave] = v;
+  } else {
+    const int k = wave - 5;
+    const uint32_t n = wave_count(pr.cnt + (size_t)k * pr.mpad, pr.nch, l);
+    if (l == 0) pr.out_cnt[k] = n;
   }
 }
 
@@ -1949,14 +1983,14 @@ hipError_t launch_segment_batch(const SegArgs* recs, const uint32_t* map, uint32
 
 hipError_t launch_seg_final(const SegArgs& a, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_seg_final, dim3(1), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_seg_final, dim3(1), dim3(kFinalBlock), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_seg_final_batch(const SegArgs* recs, uint32_t nmem, const uint64_t* roff,
                                   hipStream_t s)
 {
-  hipLaunchKernelGGL(k_seg_final_batch, dim3(nmem), dim3(kBlock), 0, s, recs, roff);
+  hipLaunchKernelGGL(k_seg_final_batch, dim3(nmem), dim3(kFinalBlock), 0, s, recs, roff);
   return hipGetLastError();
 }
 
@@ -1972,7 +2006,7 @@ hipError_t launch_phase(const PhaseArgs& a, hipStream_t s)
 
 hipError_t launch_phase_final(const PhaseArgs& a, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_phase_final, dim3(1), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_phase_final, dim3(1), dim3(kPhaseFinalBlock), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1994,7 +2028,7 @@ hipError_t launch_phase_batch(const PhaseArgs* recs, const uint32_t* map, uint32
 hipError_t launch_phase_final_batch(const PhaseArgs* recs, uint32_t nmem, const uint64_t* roff,
                                     hipStream_t s)
 {
-  hipLaunchKernelGGL(k_phase_final_batch, dim3(nmem), dim3(kBlock), 0, s, recs, roff);
+  hipLaunchKernelGGL(k_phase_final_batch, dim3(nmem), dim3(kPhaseFinalBlock), 0, s, recs, roff);
   return hipGetLastError();
 }
 
@@ -2195,7 +2229,7 @@ hipError_t launch_sums(BeamArrays b, const double* a, const double* bb, int filt
 {
   const uint32_t nch = (b.n + kChunk - 1) / kChunk;
   hipLaunchKernelGGL(k_sums, dim3(nch), dim3(kBlock), 0, s, b, a, bb, filter, pr, rel_ref);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(kBlock), 0, s, pr);
+  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(512), 0, s, pr);
   return hipGetLastError();
 }
 

@@ -172,6 +172,19 @@ def test_cross_chunk_tree_widths_bit_exact(num):
         assert gs[k] == os_[k], (k, gs[k], os_[k])
 
 
+@pytest.mark.parametrize("num", [65_537, 100_000])
+def test_cross_chunk_tree_of_two_entries_per_lane_bit_exact(num):
+    """65 and 98 chunks: partials padded to 128, two entries per lane of the
+    wavefront that sums a quantity, with longitudinal losses."""
+    import math
+    wl = H.workload(0, num=num, periods=3, sc=True)
+    wl.beam.sig_phi = math.radians(70.0)
+    ob, _, _ = H.run_oracle(wl)
+    gb, _, _ = H.run_gpu(wl)
+    err = H.compare_arrays(gb.arrays(), ob.arrays())
+    assert err is None, err
+
+
 @pytest.mark.parametrize("num", [4096, 600000])
 def test_aperture_elements_and_rotation_steerer(num):
     """Aperture elements (their centroid and loss-count statistics), a
