@@ -287,7 +287,6 @@ struct hps_spch {
   double* fld1 = nullptr;
   double* fld2 = nullptr;
   int64_t* bins = nullptr;
-  double* part = nullptr;    // split partial sums of the field (kFieldMaxSplit tables)
   size_t max_lds = 0;        // LDS bytes per workgroup on this device
 };
 
@@ -803,13 +802,12 @@ constexpr uint32_t kMaxAdjBunch = 1024;
 
 static int spch_alloc_tables(hps_spch* s)
 {
-  (void)hipFree(s->fld1); (void)hipFree(s->fld2); (void)hipFree(s->bins); (void)hipFree(s->part);
-  s->fld1 = nullptr; s->fld2 = nullptr; s->bins = nullptr; s->part = nullptr;
+  (void)hipFree(s->fld1); (void)hipFree(s->fld2); (void)hipFree(s->bins);
+  s->fld1 = nullptr; s->fld2 = nullptr; s->bins = nullptr;
   const uint32_t nr = s->cfg.nx, nz = s->cfg.nz;
   const size_t n1 = (size_t)(nr + 1) * nr * nz * 2, n2 = (size_t)(nz + 1) * (nr + 1) * 2;
   HPS_CHECK(hipMalloc(&s->fld1, n1 * 8));
   HPS_CHECK(hipMalloc(&s->fld2, n2 * 8));
-  HPS_CHECK(hipMalloc(&s->part, kFieldMaxSplit * n2 * 8));
   HPS_CHECK(hipMalloc(&s->bins, (size_t)nr * nz * 8));
   HPS_CHECK(hipMemset(s->fld1, 0, n1 * 8));
   HPS_CHECK(hipMemset(s->fld2, 0, n2 * 8));
@@ -858,7 +856,6 @@ int hps_spch_create(hps_spch** out, uint32_t nr, uint32_t nz, double interval, u
   }
   if (spch_alloc_tables(s) || spch_push_cfg(s)) {   // these set the error message
     (void)hipFree(s->dev); (void)hipFree(s->fld1); (void)hipFree(s->fld2); (void)hipFree(s->bins);
-    (void)hipFree(s->part);
     delete s;
     return -1;
   }
@@ -871,7 +868,6 @@ int hps_spch_destroy(hps_spch* s)
   if (!s) return 0;
   (void)hipStreamSynchronize(s->stream);
   (void)hipFree(s->dev); (void)hipFree(s->fld1); (void)hipFree(s->fld2); (void)hipFree(s->bins);
-  (void)hipFree(s->part);
   delete s;
   return 0;
 }
@@ -1398,8 +1394,8 @@ extern "C" int hps_sim_simulate(hps_sim* m, int32_t start, int32_t end)
                                deposit_ok, st);
       default: {
         FieldArgs f;
-        f.sc = sc->dev; f.bins = sc->bins; f.fld1 = sc->fld1; f.fld2 = sc->fld2; f.part = sc->part;
-        return launch_field(f, sc->cfg.nx, sc->cfg.nz, sc->max_lds, st);
+        f.sc = sc->dev; f.bins = sc->bins; f.fld1 = sc->fld1; f.fld2 = sc->fld2;
+        return launch_field(f, sc->cfg.nx, sc->cfg.nz, st);
       }
     }
   };
@@ -1797,16 +1793,16 @@ static int tune_gemm(hps_batch* bt, uint32_t nr, uint32_t nz, uint32_t B, hipStr
 // do the full work) and keeps the fastest in bt->field_shape.  Needs eager
 // launches; each candidate overwrites the field tables with the same values.
 static int tune_field(hps_batch* bt, const FieldArgs* d_field, uint32_t nmem, uint32_t nr,
-                      uint32_t nz, size_t max_lds, hipStream_t s)
+                      uint32_t nz, hipStream_t s)
 {
   const uint32_t n = field_batch_shapes();
   std::vector<hipEvent_t> ev(2 * n);
   for (auto& e : ev) HPS_CHECK(hipEventCreate(&e));
   // one untimed launch first (instruction caches, table residency)
-  HPS_CHECK(launch_field_batch(d_field, nmem, nr, nz, max_lds, field_batch_default_shape(nr, nmem), s));
+  HPS_CHECK(launch_field_batch(d_field, nmem, nr, nz, UINT32_MAX, s));
   for (uint32_t k = 0; k < n; ++k) {
     HPS_CHECK(hipEventRecord(ev[2 * k], s));
-    HPS_CHECK(launch_field_batch(d_field, nmem, nr, nz, max_lds, k, s));
+    HPS_CHECK(launch_field_batch(d_field, nmem, nr, nz, k, s));
     HPS_CHECK(hipEventRecord(ev[2 * k + 1], s));
   }
   HPS_CHECK(hipEventSynchronize(ev[2 * n - 1]));
@@ -2130,7 +2126,7 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
   // per launch the records of its step
   const uint32_t nr = sc_on ? m0->sc->cfg.nx : 0, nz = sc_on ? m0->sc->cfg.nz : 0;
   if (bt->field_key[0] != nr || bt->field_key[1] != nz || bt->field_key[2] != (uint32_t)B)
-    bt->field_shape = bt->autotune ? UINT32_MAX : field_batch_default_shape(nr, (uint32_t)B);
+    bt->field_shape = bt->autotune ? UINT32_MAX : field_batch_default_shape(nr, nz, (uint32_t)B);
   std::vector<uint32_t> build_map;
   std::vector<uint32_t> nchs(B);
   for (size_t k = 0; k < B; ++k) nchs[k] = bt->sims[k]->b->pr.nch;
@@ -2154,7 +2150,6 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
         build_map.push_back(((uint32_t)k << kBatchLocalBits) | c);
       FieldArgs& f = field[k];
       f.sc = m->sc->dev; f.bins = m->sc->bins; f.fld1 = m->sc->fld1; f.fld2 = m->sc->fld2;
-      f.part = m->sc->part;
     }
   }
   const bool gemm = sc_on && bt->field_mode == 1;
@@ -2317,10 +2312,9 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
         if (bt->autotune && bt->field_shape == UINT32_MAX) {
           // first rebuild of this batch shape: time every field launch shape
           // on the live tables (each gives the same bits) and keep the fastest
-          if (tune_field(bt, d_field, (uint32_t)B, nr, nz, m0->sc->max_lds, s)) return -1;
+          if (tune_field(bt, d_field, (uint32_t)B, nr, nz, s)) return -1;
         }
-        HPS_CHECK(launch_field_batch(d_field, (uint32_t)B, nr, nz, m0->sc->max_lds,
-                                     bt->field_shape, s));
+        HPS_CHECK(launch_field_batch(d_field, (uint32_t)B, nr, nz, bt->field_shape, s));
         break;
       }
     }

@@ -110,11 +110,7 @@ struct FieldArgs {
   const int64_t* bins;
   const double* fld1;
   double* fld2;
-  double* part;     // kFieldMaxSplit * (nz+1)*(nr+1) double2: split partial sums
 };
-// The field sum may split its partial sums over up to this many workgroup
-// sets (a lone simulation, to use more CUs); part holds their results.
-constexpr uint32_t kFieldMaxSplit = 8;
 
 // Batched launches cover the blocks of several simulations in one grid; a
 // block map entry packs the simulation (high bits) and its local block.
@@ -143,8 +139,7 @@ uint32_t deposit_blocks_batch(uint32_t n, uint32_t nr, uint32_t nz);
 hipError_t launch_sc_build(ScDev* sc, double* fld1, uint32_t nr, uint32_t nz, BeamArrays b,
                            const hps_beam_stats* st, int64_t* bins, bool deposit,
                            hipStream_t s);
-hipError_t launch_field(const FieldArgs& a, uint32_t nr, uint32_t nz, size_t max_lds,
-                        hipStream_t s);
+hipError_t launch_field(const FieldArgs& a, uint32_t nr, uint32_t nz, hipStream_t s);
 uint32_t greens_blocks(uint32_t nr, uint32_t nz);
 
 // Batched forms: recs holds one argument record per simulation (the segment
@@ -179,9 +174,9 @@ hipError_t launch_probe(int fn, const double* x, const double* y, double* out, u
 // larger value: the default for the batch size); every shape gives the same
 // bits, so a caller may time them and keep the fastest.
 uint32_t field_batch_shapes();
-uint32_t field_batch_default_shape(uint32_t nr, uint32_t nmem);
+uint32_t field_batch_default_shape(uint32_t nr, uint32_t nz, uint32_t nmem);
 hipError_t launch_field_batch(const FieldArgs* recs, uint32_t nmem, uint32_t nr, uint32_t nz,
-                              size_t max_lds, uint32_t shape, hipStream_t s);
+                              uint32_t shape, hipStream_t s);
 
 // Grouped field solve of a batch (hps_field_gemm.hip): per-member record,
 // device state, launch shapes.

@@ -10,7 +10,7 @@
 //   k_phase    per-chunk relative-phase moments; k_phase_final finishes them
 //              and runs the Scheff::Start control logic on the device (no
 //              host round trip per kick).
-//   k_sc_build / k_field   the SCHEFF rebuild (Green's table and charge
+//   k_sc_build / k_field_wave   the SCHEFF rebuild (Green's table and charge
 //              deposit in one launch, then the field sum), run only when the
 //              control step asks for a remesh (flag in device memory).
 // Reductions follow one canonical order (see kChunk): lane sums of 4
@@ -1617,204 +1617,191 @@ __global__ __launch_bounds__(kDepositBlock) void k_sc_build_batch(const BuildArg
 // partials.  Field point (zp, rp) reads the Green's entry at dz = zs - zp
 // (zs >= zp, E_z sign -1) or zp - zs - 1 (zs < zp).
 //
-// The P partials may be split by residue over S workgroup sets (S a power of
-// two dividing P): set s holds the partials p = s, s + S, ...; its halving
-// tree runs the levels o >= S (which pair partials of the same residue) and
-// stores the level-S value; k_field_combine runs the levels o < S.
+// A wave computes K consecutive rows zp0 .. zp0 + K - 1 of 64 / P radii rp
+// (wave's lanes = P partials x 64 / P radii).  Along zs the K rows need the
+// Green's entries of K consecutive offsets d = zs - zp, so a K-deep window of
+// (E_r, signed E_z) values stays in registers and each step takes one new
+// entry and one charge for 2 K products.  The window slot of offset d is d
+// mod K (zp0 is a multiple of K), so with the zs loop unrolled by K every
+// slot index is a compile-time constant.
 //
-// A group of P / S lanes computes K consecutive rows zp0 .. zp0 + K - 1 of
-// one rp: lane j holds partial s + j S of all K points.  Along zs the K
-// points need the Green's entries of K consecutive offsets d = zs - zp, so a
-// K-deep window of (E_r, signed E_z) values stays in registers and each step
-// loads one new entry and one charge.  The window slot of offset d is d mod K
-// (zp0 is a multiple of K), so with the zs loop unrolled by K every slot
-// index is a compile-time constant.  kLds: the workgroup's columns (rings of
-// its residue) of the rp slice of the table and of the bins are staged in
-// LDS first.
+// All lanes of the wave share zp0, hence d: the row an entry is read from and
+// the sign of its E_z are scalar, and the vector unit does little but the 2 K
+// products.  Lanes of one wave on different rows of one radius cost as many
+// vector instructions for index and sign as for the products, and every
+// workgroup staged the whole table slice of its radius in LDS first (32 x 128:
+// 96 KB per workgroup of four waves, two memory round trips before the first
+// product; 64 x 256: sixteen-byte pieces of every line, eight splits and a
+// combine launch).  The entries now come straight from L2, coalesced, kDepth
+// row blocks ahead of their use; only the charges, shared by all waves, are
+// staged.  Workgroups are dealt so that those of neighbouring radii share an
+// XCD's L2.  Against the staged form: 300,007 particles on 64 x 256 148 ->
+// 109 us a kick point, seven FP64 members on 32 x 128 field 46 -> 24 us.
 struct FieldGeom {
-  uint32_t P, S, groups_per_wg, wgs_per_set;
+  uint32_t P;        // partials
+  uint32_t blocks;   // row blocks of K rows
+  uint32_t units;    // waves with work: groups of 64 / P radii x row blocks
+  uint32_t per_xcd;  // workgroups dealt to an XCD
 };
 
-template <int K, bool kLds>
-__device__ __forceinline__ void field_win_body(const FieldArgs& f, uint32_t nr, uint32_t nz,
-                                               const FieldGeom& fg, uint32_t blk, double* lds)
+template <int K, int kDepth>
+__device__ __forceinline__ void field_wave_body(const FieldArgs& f, uint32_t nr, uint32_t nz,
+                                                const FieldGeom& fg, uint32_t blk, double* lq)
 {
-  const ScDev* sc = f.sc;
-  if (!sc->remesh) return;
-  const uint32_t S = fg.S, G = fg.P / S;
-  const uint32_t per_rp = S * fg.wgs_per_set;
-  const uint32_t rp = blk / per_rp;
-  const uint32_t set = (blk % per_rp) / fg.wgs_per_set;
-  const uint32_t wg = blk % fg.wgs_per_set;
+  if (!f.sc->remesh) return;
+  // charges, kStage in flight per thread
+  constexpr uint32_t kStage = 8;
   const uint32_t fld_sz = nr * nz;
-  // columns of this set: rings rs = set + c S, c < nc
-  const uint32_t nc = set < nr ? (nr - set + S - 1) / S : 0;
-  const double2* gsrc = reinterpret_cast<const double2*>(f.fld1) + (size_t)rp * fld_sz;
-  const double2* g = gsrc;
-  const double* lb = nullptr;
-  uint32_t gstride = nr;
-  if (kLds) {
-    double2* lg = reinterpret_cast<double2*>(lds);   // [nz][nc] (E_r, E_z)
-    double* lq = lds + 2 * (size_t)nz * nc;           // [nz][nc] charge
-    // kStage entries per thread are loaded before any is stored: one memory
-    // round trip per kStage entries instead of one per entry.  Indexes past
-    // the slice are clamped to its last entry, so every load and store is
-    // unconditional (the clamped stores write that entry's own values).
-    constexpr uint32_t kStage = 8;
-    const uint32_t total = nz * nc;
-    for (uint32_t i0 = threadIdx.x; i0 < total; i0 += kStage * blockDim.x) {
-      double2 gv[kStage];
-      int64_t qv[kStage];
+  for (uint32_t i0 = threadIdx.x; i0 < fld_sz; i0 += kStage * blockDim.x) {
+    int64_t qv[kStage];
 #pragma unroll
-      for (uint32_t u = 0; u < kStage; ++u) {
-        const uint32_t i = ::min(i0 + u * blockDim.x, total - 1);
-        const uint32_t src = (i / nc) * nr + set + (i % nc) * S;
-        const double* e = reinterpret_cast<const double*>(gsrc) + 2 * (size_t)src;
-        gv[u] = make_double2(gld(e, 0), gld(e, 1));
-        qv[u] = gld(f.bins, src);
-      }
+    for (uint32_t u = 0; u < kStage; ++u) qv[u] = gld(f.bins, ::min(i0 + u * blockDim.x, fld_sz - 1));
 #pragma unroll
-      for (uint32_t u = 0; u < kStage; ++u) {
-        const uint32_t i = ::min(i0 + u * blockDim.x, total - 1);
-        lg[i] = gv[u];
-        lq[i] = (double)qv[u] * 0x1p-36;
-      }
-    }
-    __syncthreads();
-    g = lg;
-    lb = lq;
-    gstride = nc;
+    for (uint32_t u = 0; u < kStage; ++u)
+      lq[::min(i0 + u * blockDim.x, fld_sz - 1)] = (double)qv[u] * 0x1p-36;
   }
-  const uint32_t j = threadIdx.x % G;
-  const uint32_t block = wg * fg.groups_per_wg + threadIdx.x / G;
-  const int zp0 = (int)(block * K);
-  if (zp0 > (int)nz) return;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wg = (blk & 7u) * fg.per_xcd + (blk >> 3);
+  const uint32_t unit = wg * (blockDim.x >> 6) + wave;
+  const uint32_t P = fg.P, lane = threadIdx.x & 63u;
+  const uint32_t j = lane & (P - 1);
+  const uint32_t rp0 = unit / fg.blocks * (64 / P);   // the wave's radii rp0 ...
+  const uint32_t rp = rp0 + lane / P;
+  const int zp0 = (int)(unit % fg.blocks) * K;
   const int inz = (int)nz;
-  // column of ring rs in the (staged or global) table
-  auto col = [&](uint32_t rs) -> uint32_t { return kLds ? (rs - set) / S : rs; };
-  // window entry for offset d of ring rs; offsets of the zs loop always
-  // index the table (|d| < nz for rows zp <= nz), only the prefill of rows
-  // past nz needs the bound
-  auto entry = [&](int d, uint32_t c) -> double2 {
-    const int t = d >= 0 ? d : -d - 1;
-    double2 v = g[(uint32_t)t * gstride + c];
-    if (d >= 0) v.y = -v.y;
-    return v;
-  };
-  auto entry_bounded = [&](int d, uint32_t c) -> double2 {
-    const int t = d >= 0 ? d : -d - 1;
-    return t < inz ? entry(d, c) : make_double2(0.0, 0.0);
-  };
-  auto charge = [&](int zs, uint32_t c) -> double {
-    const uint32_t bi = (uint32_t)zs * gstride + c;
-    return kLds ? lb[bi] : (double)f.bins[bi] * 0x1p-36;
-  };
+  __syncthreads();
+  if (unit >= fg.units) return;
+  // the wave's part of the table as a buffer: entries at a lane offset (radius
+  // and ring) plus a scalar row offset
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const uint32_t nrad = ::min(nr + 1 - rp0, 64 / P);
+  const __amdgpu_buffer_rsrc_t tab = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<double*>(f.fld1) + 2 * (size_t)rp0 * fld_sz, 0, (int)(16 * nrad * fld_sz), 0x00020000);
+  const uint32_t lane0 = 16 * ((rp <= nr ? rp : nr) - rp0) * fld_sz;
+  const int rb = 16 * (int)nr, last = (inz - 1) * rb;   // bytes of a row, offset of the last
   double tx[K], ty[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) { tx[k] = 0.0; ty[k] = 0.0; }
-  for (uint32_t rs = set + j * S; rs < nr; rs += fg.P) {
-    const uint32_t c = col(rs);
-    double2 w[K];
-    w[0] = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int k = 1; k < K; ++k) w[K - k] = entry_bounded(-zp0 - k, c);
-    int zs0 = 0;
-    for (; zs0 + K <= inz; zs0 += K) {
+  for (uint32_t rs = j; rs < nr; rs += P) {
+    const int at = (int)(lane0 + 16 * rs);
+    const auto entry = [&](int so) -> double2 {
+      const u4 v = __builtin_amdgcn_raw_buffer_load_b128(tab, at, ::min(so, last), 0);
+      return make_double2(double_of((uint64_t)v.y << 32 | v.x), double_of((uint64_t)v.w << 32 | v.z));
+    };
+    // the entries (E_z unsigned) of source rows zs0 .. zs0 + K - 1 against row
+    // zp0: both multiples of K, so all behind or all ahead; rows past the
+    // table repeat its last and are not used
+    const auto load = [&](double2 (&e)[K], int zs0) {
+      const bool ahead = zs0 >= zp0;
+      int so = (ahead ? zs0 - zp0 : zp0 - 1 - zs0) * rb;
 #pragma unroll
       for (int u = 0; u < K; ++u) {
-        w[u] = entry(zs0 + u - zp0, c);
-        const double q = charge(zs0 + u, c);
+        e[u] = entry(so);
+        so += ahead ? rb : -rb;
+      }
+    };
+    // Ring of kDepth + 1 row blocks: block b sits in ring[b % R], its
+    // predecessor (the older half of the window) in the slot before, and when
+    // b is done that slot takes block b + kDepth.
+    constexpr int R = kDepth + 1;
+    double2 ring[R][K];
+    ring[R - 1][0] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int k = 1; k < K; ++k) {   // offsets -zp0 - k: entry zp0 + k - 1, none past the table
+      ring[R - 1][K - k] = entry((zp0 + k - 1) * rb);
+      if (zp0 + k > inz) ring[R - 1][K - k] = make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int h = 0; h < kDepth; ++h) load(ring[h], h * K);
+    // the products of block b = zs0 / K in ring[h], n of its K rows
+    double c[R][K];
+    const auto block = [&](int zs0, int h, int n) {
+      const uint64_t flip = zs0 >= zp0 ? 0x8000000000000000ull : 0ull;   // sources ahead
+      const int hp = (h + R - 1) % R;
+#pragma unroll
+      for (int u = 0; u < K; ++u) {
+        if (u >= n) continue;
+        ring[h][u].y = double_of(bits_of(ring[h][u].y) ^ flip);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-          const double2 v = w[(u - k + K) % K];
-          tx[k] = ::fma(q, v.x, tx[k]);
-          ty[k] = ::fma(q, v.y, ty[k]);
+          const double2 v = k <= u ? ring[h][u - k] : ring[hp][K + u - k];
+          tx[k] = ::fma(c[h][u], v.x, tx[k]);
+          ty[k] = ::fma(c[h][u], v.y, ty[k]);
+        }
+      }
+    };
+    // charges of a whole block, read from LDS one block ahead (past the last
+    // whole block it is read again, unused)
+    const auto charges = [&](int zs0, int h) {
+      const double* q = lq + (uint32_t)::min(zs0, inz - K) * nr + rs;
+#pragma unroll
+      for (int u = 0; u < K; ++u) c[h][u] = q[(uint32_t)u * nr];
+    };
+    int zs0 = 0;
+    if (R * K <= inz) {
+      charges(0, 0);
+      for (; zs0 + R * K <= inz; zs0 += R * K) {
+#pragma unroll
+        for (int h = 0; h < R; ++h) {
+          charges(zs0 + (h + 1) * K, (h + 1) % R);
+          block(zs0 + h * K, h, K);
+          load(ring[(h + R - 1) % R], zs0 + (h + kDepth) * K);
         }
       }
     }
-    if (zs0 < inz) {
 #pragma unroll
-      for (int u = 0; u < K; ++u) {
-        if (zs0 + u < inz) {
-          w[u] = entry(zs0 + u - zp0, c);
-          const double q = charge(zs0 + u, c);
+    for (int h = 0; h < R; ++h) {
+      const int z = zs0 + h * K, n = ::min(K, inz - z);
+      if (n <= 0) break;
 #pragma unroll
-          for (int k = 0; k < K; ++k) {
-            const double2 v = w[(u - k + K) % K];
-            tx[k] = ::fma(q, v.x, tx[k]);
-            ty[k] = ::fma(q, v.y, ty[k]);
-          }
-        }
-      }
+      for (int u = 0; u < K; ++u)
+        if (u < n) c[h][u] = lq[(uint32_t)(z + u) * nr + rs];
+      block(z, h, n);
+      if (h == 0) load(ring[R - 1], zs0 + kDepth * K);
     }
   }
-  // levels o = P/2 .. S of the tree: lane offsets G/2 .. 1 inside the group
-  for (uint32_t o = G / 2; o >= 1; o >>= 1) {
+  // halving tree over the partials
+  for (uint32_t o = P / 2; o >= 1; o >>= 1) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const double ox = __shfl_down(tx[k], o, (int)G);
-      const double oy = __shfl_down(ty[k], o, (int)G);
+      const double ox = __shfl_down(tx[k], o, (int)P);
+      const double oy = __shfl_down(ty[k], o, (int)P);
       tx[k] = tx[k] + ox;
       ty[k] = ty[k] + oy;
     }
   }
-  if (j == 0) {
-    const uint32_t nout = (nz + 1) * (nr + 1);
-    double* dst = S == 1 ? f.fld2 : f.part + 2 * (size_t)set * nout;
+  if (j == 0 && rp <= nr) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int zp = zp0 + k;
       if (zp <= inz) {
         const size_t o = (size_t)zp * (nr + 1) + rp;
-        dst[2 * o] = tx[k];
-        dst[2 * o + 1] = ty[k];
+        gst(f.fld2, 2 * o, tx[k]);
+        gst(f.fld2, 2 * o + 1, ty[k]);
       }
     }
   }
 }
 
-template <int K, bool kLds>
-__global__ __launch_bounds__(1024) void k_field_win(FieldArgs f, uint32_t nr, uint32_t nz,
-                                                    FieldGeom fg)
+constexpr uint32_t kFieldMaxWaves = 9;
+constexpr size_t kCuLds = 160 * 1024;
+
+template <int K, int kDepth>
+__global__ __launch_bounds__(64 * kFieldMaxWaves) void k_field_wave(FieldArgs f, uint32_t nr,
+                                                                    uint32_t nz, FieldGeom fg)
 {
   extern __shared__ double lds[];
-  field_win_body<K, kLds>(f, nr, nz, fg, blockIdx.x, lds);
+  field_wave_body<K, kDepth>(f, nr, nz, fg, blockIdx.x, lds);
 }
 
 // per simulation of a batch: blocks [m * per, (m + 1) * per)
-template <int K, bool kLds>
-__global__ __launch_bounds__(1024) void k_field_win_batch(const FieldArgs* recs, uint32_t per,
-                                                          uint32_t nr, uint32_t nz, FieldGeom fg)
+template <int K, int kDepth>
+__global__ __launch_bounds__(64 * kFieldMaxWaves) void k_field_wave_batch(
+    const FieldArgs* recs, uint32_t per, uint32_t nr, uint32_t nz, FieldGeom fg)
 {
   extern __shared__ double lds[];
   const FieldArgs f = recs[blockIdx.x / per];
-  field_win_body<K, kLds>(f, nr, nz, fg, blockIdx.x % per, lds);
-}
-
-// Levels o = S/2 .. 1 of the field tree over the split results.
-__global__ __launch_bounds__(kBlock) void k_field_combine(FieldArgs f, uint32_t nout, uint32_t S)
-{
-  if (!f.sc->remesh) return;
-  const uint32_t o = blockIdx.x * kBlock + threadIdx.x;
-  if (o >= nout) return;
-  double ax[kFieldMaxSplit], ay[kFieldMaxSplit];
-#pragma unroll
-  for (uint32_t l = 0; l < kFieldMaxSplit; ++l) {
-    ax[l] = l < S ? f.part[2 * ((size_t)l * nout + o)] : 0.0;
-    ay[l] = l < S ? f.part[2 * ((size_t)l * nout + o) + 1] : 0.0;
-  }
-#pragma unroll
-  for (uint32_t h = kFieldMaxSplit / 2; h >= 1; h >>= 1) {
-    if (h < S) {
-#pragma unroll
-      for (uint32_t l = 0; l < h; ++l) {
-        ax[l] = ax[l] + ax[l + h];
-        ay[l] = ay[l] + ay[l + h];
-      }
-    }
-  }
-  f.fld2[2 * (size_t)o] = ax[0];
-  f.fld2[2 * (size_t)o + 1] = ay[0];
+  field_wave_body<K, kDepth>(f, nr, nz, fg, blockIdx.x % per, lds);
 }
 
 // --- getter reductions ---------------------------------------------------------
@@ -2106,53 +2093,38 @@ hipError_t launch_sc_build_batch(const BuildArgs* recs, const uint32_t* map, uin
 
 namespace {
 
-// Launch shape of the field sum.
+// Launch shape of the field sum: rows per wave and waves per workgroup.
 struct FieldShape {
-  bool lds;
   int K;
   FieldGeom g;
   uint32_t threads, blocks;
-  size_t lds_bytes;
 };
 
-FieldShape field_shape_k(uint32_t nr, uint32_t nz, size_t max_lds, int K, uint32_t S,
-                         uint32_t max_threads)
+FieldShape field_shape(uint32_t nr, uint32_t nz, int K, uint32_t waves)
 {
   FieldShape f{};
   uint32_t P = 1;
   while (P < nr && P < 64) P <<= 1;
-  if (S > P) S = P;
-  f.g.P = P;
-  f.g.S = S;
+  const uint32_t radii = 64 / P;
   f.K = K;
-  const uint32_t G = P / S;
-  const uint32_t nblk = (nz + 1 + K - 1) / K;
-  uint32_t threads = nblk * G;
-  threads = (threads + 63) / 64 * 64;
-  if (threads > max_threads) threads = max_threads;
-  f.threads = threads;
-  f.g.groups_per_wg = threads / G;
-  f.g.wgs_per_set = (nblk + f.g.groups_per_wg - 1) / f.g.groups_per_wg;
-  f.blocks = (nr + 1) * S * f.g.wgs_per_set;
-  const uint32_t nc = (nr + S - 1) / S;   // columns of the widest set
-  f.lds_bytes = (size_t)24 * nz * nc;
-  f.lds = f.lds_bytes <= max_lds;
-  if (!f.lds) f.lds_bytes = 0;
+  f.g.P = P;
+  f.g.blocks = (nz + 1 + K - 1) / K;
+  f.g.units = (nr + 1 + radii - 1) / radii * f.g.blocks;
+  f.g.per_xcd = ((f.g.units + waves - 1) / waves + 7) / 8;
+  f.threads = 64 * waves;
+  f.blocks = 8 * f.g.per_xcd;
   return f;
 }
 
-// A batch has workgroups enough with the deepest window and all partials in
-// one workgroup.  A lone simulation uses small (256-thread) workgroups with
-// all partials, so that the rows spread over more CUs and no combine step is
-// needed, when its table slice fits in LDS (32 x 128: 11.7 ms/step of field
-// time against 13.2 for the 8-set split plus combine); otherwise it splits
-// its partials over sets (each set stages only its rings).
-FieldShape field_shape(uint32_t nr, uint32_t nz, size_t max_lds, uint32_t nsim)
+// The launch shapes (every shape computes the same canonical sums): K = 8 / 4
+// / 2 rows, 9 / 4 / 2 waves.
+constexpr uint32_t kFieldShapes = 9;
+constexpr uint32_t kFieldWaves[] = {9, 4, 2};
+static_assert(kFieldWaves[0] <= kFieldMaxWaves, "launch bounds");
+
+FieldShape field_shape_of(uint32_t nr, uint32_t nz, uint32_t idx)
 {
-  if (nsim * (nr + 1) >= 1024) return field_shape_k(nr, nz, max_lds, 8, 1, 1024);
-  const FieldShape f = field_shape_k(nr, nz, max_lds, 4, 1, 256);
-  if (f.lds) return f;
-  return field_shape_k(nr, nz, max_lds, 4, kFieldMaxSplit, 1024);
+  return field_shape(nr, nz, 8 >> (idx / 3), kFieldWaves[idx % 3]);
 }
 
 template <bool kBatch>
@@ -2160,68 +2132,53 @@ hipError_t launch_field_shape(const FieldShape& f, const FieldArgs* recs, const 
                               uint32_t nsim, uint32_t nr, uint32_t nz, hipStream_t s)
 {
   const dim3 grid(f.blocks * nsim), block(f.threads);
-#define HPS_FIELD_LAUNCH(KK, LL)                                                              \
-  if (kBatch)                                                                                 \
-    hipLaunchKernelGGL((k_field_win_batch<KK, LL>), grid, block, f.lds_bytes, s, recs,        \
-                       f.blocks, nr, nz, f.g);                                                \
-  else                                                                                        \
-    hipLaunchKernelGGL((k_field_win<KK, LL>), grid, block, f.lds_bytes, s, one, nr, nz, f.g);
-  if (f.K == 8) {
-    if (f.lds) { HPS_FIELD_LAUNCH(8, true) } else { HPS_FIELD_LAUNCH(8, false) }
-  } else if (f.K == 4) {
-    if (f.lds) { HPS_FIELD_LAUNCH(4, true) } else { HPS_FIELD_LAUNCH(4, false) }
-  } else if (f.K == 2) {
-    if (f.lds) { HPS_FIELD_LAUNCH(2, true) } else { HPS_FIELD_LAUNCH(2, false) }
-  } else {
-    if (f.lds) { HPS_FIELD_LAUNCH(1, true) } else { HPS_FIELD_LAUNCH(1, false) }
-  }
+  const size_t lds = (size_t)nr * nz * sizeof(double);
+#define HPS_FIELD_LAUNCH(KK, DD)                                                                \
+  if (kBatch)                                                                                   \
+    hipLaunchKernelGGL((k_field_wave_batch<KK, DD>), grid, block, lds, s, recs, f.blocks, nr,   \
+                       nz, f.g);                                                                \
+  else                                                                                          \
+    hipLaunchKernelGGL((k_field_wave<KK, DD>), grid, block, lds, s, one, nr, nz, f.g);
+  if (f.K == 8) { HPS_FIELD_LAUNCH(8, 1) }
+  else if (f.K == 4) { HPS_FIELD_LAUNCH(4, 3) }
+  else { HPS_FIELD_LAUNCH(2, 7) }
 #undef HPS_FIELD_LAUNCH
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_field(const FieldArgs& a, uint32_t nr, uint32_t nz, size_t max_lds,
-                        hipStream_t s)
+uint32_t field_batch_shapes() { return kFieldShapes; }
+
+// Eight rows a wave spend 84 % of the vector instructions on products, four
+// 80 %, but a table with fewer than one wave of eight rows per SIMD is bound
+// by the length of a wave's chain, which four rows halve (65,536 particles on
+// 32 x 128: 42.3 us a kick point with K = 4, 43.8 with 8, 44.4 with 2; seven
+// members: 153.0 with 8, 153.4 with 4, 166.7 with 2).  Where the charges take
+// more than half of the LDS a CU holds one workgroup, so it takes nine waves,
+// as many as its registers allow (64 x 256, 2,145 waves on 239 workgroups:
+// 109 us a kick point; eight waves are a second round of workgroups, 127;
+// four 130); otherwise several small ones (four waves; nine 163, two 156 on
+// the seven members).
+uint32_t field_batch_default_shape(uint32_t nr, uint32_t nz, uint32_t nmem)
 {
-  const FieldShape f = field_shape(nr, nz, max_lds, 1);
-  hipError_t e = launch_field_shape<false>(f, nullptr, a, 1, nr, nz, s);
-  if (e != hipSuccess || f.g.S == 1) return e;
-  const uint32_t nout = (nz + 1) * (nr + 1);
-  hipLaunchKernelGGL(k_field_combine, dim3((nout + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a,
-                     nout, f.g.S);
-  return hipGetLastError();
+  const uint32_t k = field_shape(nr, nz, 8, 1).g.units * (uint64_t)nmem >= 1024 ? 0 : 1;
+  const uint32_t w = (size_t)nr * nz * sizeof(double) > kCuLds / 2 ? 0 : 1;
+  return 3 * k + w;
 }
 
-namespace {
-
-// Field-sum shapes a batch can use (all partials in one workgroup set): window
-// depth x workgroup size.  Every shape computes the same canonical sums.
-constexpr int kFieldBatchK[] = {8, 4, 2};
-constexpr uint32_t kFieldBatchThreads[] = {1024, 512, 256};
-constexpr uint32_t kFieldBatchShapes = 9;
-
-FieldShape field_batch_shape(uint32_t nr, uint32_t nz, size_t max_lds, uint32_t idx)
+hipError_t launch_field(const FieldArgs& a, uint32_t nr, uint32_t nz, hipStream_t s)
 {
-  return field_shape_k(nr, nz, max_lds, kFieldBatchK[idx / 3], 1, kFieldBatchThreads[idx % 3]);
-}
-
-}  // namespace
-
-uint32_t field_batch_shapes() { return kFieldBatchShapes; }
-
-uint32_t field_batch_default_shape(uint32_t nr, uint32_t nmem)
-{
-  return nmem * (nr + 1) >= 1024 ? 0u : 3u;   // K 8 or 4, 1024 threads
+  return launch_field_shape<false>(
+      field_shape_of(nr, nz, field_batch_default_shape(nr, nz, 1)), nullptr, a, 1, nr, nz, s);
 }
 
 hipError_t launch_field_batch(const FieldArgs* recs, uint32_t nmem, uint32_t nr, uint32_t nz,
-                              size_t max_lds, uint32_t shape, hipStream_t s)
+                              uint32_t shape, hipStream_t s)
 {
   FieldArgs none{};
-  if (shape >= kFieldBatchShapes) shape = field_batch_default_shape(nr, nmem);
-  return launch_field_shape<true>(field_batch_shape(nr, nz, max_lds, shape), recs, none, nmem,
-                                  nr, nz, s);
+  if (shape >= kFieldShapes) shape = field_batch_default_shape(nr, nz, nmem);
+  return launch_field_shape<true>(field_shape_of(nr, nz, shape), recs, none, nmem, nr, nz, s);
 }
 
 hipError_t launch_sums(BeamArrays b, const double* a, const double* bb, int filter, Partials pr,
