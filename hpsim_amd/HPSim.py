@@ -188,12 +188,11 @@ class Beam:
     def get_size(self): return self._n
 
     # -- coordinates ------------------------------------------------------------
-    def _download(self):
-        out = {k: np.empty(self._n) for k in _COORD}
-        out["loss"] = np.empty(self._n, np.uint32)
-        out["lloss"] = np.empty(self._n, np.uint32)
-        check(_lib().hps_beam_download(self._h, *[dptr(out[k]) for k in _COORD],
-                                       uptr(out["loss"]), uptr(out["lloss"])))
+    def _download(self, names=_COORD + ("loss", "lloss")):
+        out = {k: np.empty(self._n, np.float64 if k in _COORD else np.uint32) for k in names}
+        check(_lib().hps_beam_download(
+            self._h, *[dptr(out[k]) if k in out else None for k in _COORD],
+            *[uptr(out.get(k)) for k in ("loss", "lloss")]))
         return out
 
     def arrays(self):
@@ -204,7 +203,7 @@ class Beam:
         if option not in ("good", "lost", "all"):
             raise ValueError(f"invalid option: {option}, pick from (\"good\", \"lost\", \"all\")")
         self.get_loss_num("t")    # UpdateLoss, as the reference getters do
-        a = self._download()
+        a = self._download((name,) if option == "all" else (name, "loss"))
         v = a[name]
         if option == "all":
             return v
@@ -229,7 +228,7 @@ class Beam:
         check(_lib().hps_beam_relative_phi(self._h, 0, dptr(rel)))
         if option == "all":
             return rel
-        loss = self._download()["loss"]
+        loss = self._download(("loss",))["loss"]
         return rel[loss == 0] if option == "good" else rel[loss != 0]
 
     def get_losses(self, option="t"):
@@ -237,8 +236,8 @@ class Beam:
         if option not in ("t", "l"):
             raise ValueError(f"invalid option: {option}, pick from (\"t\", \"l\")")
         self.get_loss_num(option)
-        a = self._download()
-        return a["loss"] if option == "t" else a["lloss"]
+        name = "loss" if option == "t" else "lloss"
+        return self._download((name,))[name]
 
     def get_loss_num(self, option="t"):
         """get_loss_num('t'|'l'|'all'), wrap_beam.cpp:1245-1284."""

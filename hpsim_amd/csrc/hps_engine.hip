@@ -51,6 +51,10 @@ uint32_t next_pow2(uint32_t x)   // utility.cpp:7-16
 
 hipStream_t g_stream[16];
 
+// Largest read-back that goes through a beam's pinned staging block (18,724
+// particles; freed with the beam).
+constexpr size_t kStageBytes = 1 << 20;
+
 }  // namespace
 
 namespace hps {
@@ -87,28 +91,34 @@ struct hps_beam {
   Partials pr{};
   double* snap[2][6] = {{nullptr}};
   uint32_t* snap_l[2][2] = {{nullptr}};
+  Readout* ro = nullptr;            // pinned: the getters' sums and the statistics
+  uint8_t* stage = nullptr;         // pinned: read-back of a small beam (kStageBytes at most)
   bool saved[2] = {false, false};
   double snap_dw[2] = {0, 0}, snap_f[2] = {0, 0}, snap_c[2] = {0, 0};
 };
 
 namespace {
 
-// Canonical-order sums over the beam (k_sums), copied to host.
-struct Sums {
-  double s[5];
-  uint32_t nloss, ngood, nlloss;
+// What a getter reads: the canonical-order sums of up to kReadSlots
+// variable pairs (k_sums), the loss counts, the statistics and the reference
+// particle's energy.  The kernels write them into the beam's pinned block, so
+// a getter waits for the device once; the statistics go back as the argument
+// of a one-wave kernel.  (With every value copied by itself a getter waited
+// three to eight times: twenty getters of a 1,048,576-particle beam 3.3 ms.)
+struct Pair {
+  const double *a, *bb;
+  int filter;              // k_sums: 0 loss == 0, 1 good, 2 all
+  const double* rel_ref;   // a replaced by its relative phase against *rel_ref
 };
 
-int run_sums(hps_beam* b, const double* a, const double* bb, int filter, Sums* out)
+int read_sums(hps_beam* b, const Pair* p, int n, hps_beam_stats* s)
 {
-  HPS_CHECK(launch_sums(b->d, a, bb, filter, b->pr, b->stream));
-  HPS_CHECK(hipMemcpyAsync(out->s, b->pr.out, 5 * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-  uint32_t c[3];
-  HPS_CHECK(hipMemcpyAsync(c, b->pr.out_cnt, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream));
+  for (int k = 0; k < n; ++k) {
+    HPS_CHECK(launch_sums(b->d, p[k].a, p[k].bb, p[k].filter, b->pr, b->stream, p[k].rel_ref,
+                          &b->ro->sums[k], s && k == n - 1 ? b->ro : nullptr, b->st));
+  }
   HPS_CHECK(hipStreamSynchronize(b->stream));
-  out->nloss = c[0];
-  out->ngood = c[1];
-  out->nlloss = c[2];
+  if (s) *s = b->ro->st;
   return 0;
 }
 
@@ -119,73 +129,44 @@ int pull(hps_beam* b, hps_beam_stats* s)
   return 0;
 }
 
-int push(hps_beam* b, const hps_beam_stats* s)
+int push(hps_beam* b, const hps_beam_stats& s)
 {
-  HPS_CHECK(hipMemcpyAsync(b->st, s, sizeof(*s), hipMemcpyHostToDevice, b->stream));
-  HPS_CHECK(hipStreamSynchronize(b->stream));
+  HPS_CHECK(launch_set_stats(b->st, s, b->stream));
   return 0;
 }
 
 double surv(const hps_beam* b, const hps_beam_stats& s) { return (double)(uint32_t)(b->n - s.num_loss); }
 
-// UpdateLossCountKernelCall, beam.cu:493-516
-int update_loss(hps_beam* b, hps_beam_stats& s)
-{
-  Sums r;
-  if (run_sums(b, nullptr, nullptr, 2, &r)) return -1;
-  s.num_loss = r.nloss;
-  return 0;
-}
-
-// UpdateGoodParticleCountKernelCall, beam.cu:1233-1255
-int update_good(hps_beam* b, hps_beam_stats& s)
-{
-  Sums r;
-  if (run_sums(b, nullptr, nullptr, 2, &r)) return -1;
-  s.num_good = r.ngood;
-  return 0;
-}
-
 // UpdateAvgOfOneVariableKernelCall + finalise kernels, beam.cu:411-436,
 // beam_kernel.cu:1396-1410
-int avg_of(hps_beam* b, hps_beam_stats& s, const double* a, bool good, double* out)
+double avg_of(const hps_beam* b, const hps_beam_stats& s, const BeamSums& r, bool good)
 {
-  Sums r;
-  if (run_sums(b, a, nullptr, good ? 1 : 0, &r)) return -1;
-  if (!good) *out = r.s[0] / surv(b, s);
-  else *out = s.num_good > 0 ? r.s[0] / (double)s.num_good : -99999;
-  return 0;
+  if (!good) return r.s[0] / surv(b, s);
+  return s.num_good > 0 ? r.s[0] / (double)s.num_good : -99999;
 }
 
 // UpdateSigmaOfOneVariableKernelCall, beam.cu:651-677
-int sig_of(hps_beam* b, hps_beam_stats& s, const double* a, bool good, double* out)
+double sig_of(const hps_beam* b, const hps_beam_stats& s, const BeamSums& r, bool good)
 {
-  Sums r;
-  if (run_sums(b, a, nullptr, good ? 1 : 0, &r)) return -1;
   const double d = good ? (double)s.num_good : surv(b, s);
   const double avg = r.s[0] / d, avg2 = r.s[1] / d;
-  *out = std::sqrt(avg2 - avg * avg);
-  return 0;
+  return std::sqrt(avg2 - avg * avg);
 }
 
-// UpdateRelativePhiKernelCall, beam.cu:1122-1131 (writes phi_r)
-int relative_phi(hps_beam* b, bool use_good)
+// Beam::UpdateLongitudinalLoss, beam.cpp:776-782; with loss, UpdateLoss before
+// and UpdateGoodParticleCount after it (the counts of the same passes)
+int update_longitudinal_loss(hps_beam* b, hps_beam_stats& s, bool all)
 {
-  const double* ref = use_good ? &b->st->phi_avg_good : b->d.phi;
-  HPS_CHECK(launch_relative_phi(b->d, ref, b->stream));
-  return 0;
-}
-
-// Beam::UpdateLongitudinalLoss, beam.cpp:776-782
-int update_longitudinal_loss(hps_beam* b, hps_beam_stats& s)
-{
-  if (update_good(b, s)) return -1;
-  if (avg_of(b, s, b->d.phi, true, &s.phi_avg_good)) return -1;
-  if (push(b, &s)) return -1;
+  const Pair phi{b->d.phi, nullptr, 1, nullptr}, counts{nullptr, nullptr, 2, nullptr};
+  if (read_sums(b, &phi, 1, &s)) return -1;
+  if (all) s.num_loss = b->ro->sums[0].nloss;
+  s.num_good = b->ro->sums[0].ngood;
+  s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+  if (push(b, s)) return -1;
   HPS_CHECK(launch_lloss_flag(b->d, &b->st->phi_avg_good, b->stream));
-  Sums r;
-  if (run_sums(b, nullptr, nullptr, 2, &r)) return -1;
-  s.num_lloss = r.nlloss;
+  if (read_sums(b, &counts, 1, nullptr)) return -1;
+  s.num_lloss = b->ro->sums[0].nlloss;
+  if (all) s.num_good = b->ro->sums[0].ngood;
   return 0;
 }
 
@@ -193,9 +174,12 @@ int update_longitudinal_loss(hps_beam* b, hps_beam_stats& s)
 int init_phi_avg_good(hps_beam* b)
 {
   hps_beam_stats s;
-  if (pull(b, &s) || update_loss(b, s) || avg_of(b, s, b->d.phi, false, &s.phi_avg)) return -1;
+  const Pair phi{b->d.phi, nullptr, 0, nullptr};
+  if (read_sums(b, &phi, 1, &s)) return -1;
+  s.num_loss = b->ro->sums[0].nloss;
+  s.phi_avg = avg_of(b, s, b->ro->sums[0], false);
   s.phi_avg_good = s.phi_avg;
-  return push(b, &s);
+  return push(b, s);
 }
 
 // Beam::ChangeFrequency, beam.cpp:1654-1668
@@ -206,21 +190,26 @@ int change_frequency(hps_beam* b, double f)
   HPS_CHECK(launch_scale(b->d.phi, b->n, ratio, b->stream));
   b->freq = f;
   hps_beam_stats s;
-  if (pull(b, &s) || avg_of(b, s, b->d.phi, false, &s.phi_avg) || push(b, &s)) return -1;
-  if (relative_phi(b, false)) return -1;
-  if (avg_of(b, s, b->d.phi_r, false, &s.phi_avg_r)) return -1;
-  return push(b, &s);
+  const Pair p[2] = {{b->d.phi, nullptr, 0, nullptr}, {b->d.phi, nullptr, 0, b->d.phi}};
+  if (read_sums(b, p, 2, &s)) return -1;
+  s.phi_avg = avg_of(b, s, b->ro->sums[0], false);
+  s.phi_avg_r = avg_of(b, s, b->ro->sums[1], false);
+  return push(b, s);
 }
 
-int emittance(hps_beam* b, hps_beam_stats& s)   // Beam::UpdateEmittance, beam.cpp:985-994
+// UpdateLoss, then Beam::UpdateEmittance (beam.cpp:985-994)
+int emittance(hps_beam* b, hps_beam_stats& s)
 {
-  if (b->n <= 2) return 0;
-  double w0;
-  HPS_CHECK(hipMemcpyAsync(&w0, b->d.w, sizeof(double), hipMemcpyDeviceToHost, b->stream));
-  HPS_CHECK(hipStreamSynchronize(b->stream));
+  const Pair p[3] = {{b->d.x, b->d.xp, 0, nullptr},
+                     {b->d.y, b->d.yp, 0, nullptr},
+                     {b->d.phi, b->d.w, 0, b->d.phi}};   // relative to particle 0
+  const bool upd = b->n > 2;
+  if (read_sums(b, p, upd ? 3 : 1, &s)) return -1;
+  s.num_loss = b->ro->sums[0].nloss;
+  if (!upd) return 0;
+  const double w0 = b->ro->w0;
   for (int axis = 0; axis < 2; ++axis) {   // beam.cu:1007-1064, beam_kernel.cu:1333-1354
-    Sums r;
-    if (run_sums(b, axis == 0 ? b->d.x : b->d.y, axis == 0 ? b->d.xp : b->d.yp, 0, &r)) return -1;
+    const BeamSums& r = b->ro->sums[axis];
     const double sv = surv(b, s);
     const double x = r.s[0] / sv, x2 = r.s[1] / sv, xp = r.s[2] / sv, xp2 = r.s[3] / sv,
                  xxp = r.s[4] / sv;
@@ -232,9 +221,7 @@ int emittance(hps_beam* b, hps_beam_stats& s)   // Beam::UpdateEmittance, beam.c
     if (axis == 0) { s.x_avg = x; s.x_sig = sig; s.xp_avg = xp; s.xp_sig = sigp; s.x_emit = emit; }
     else { s.y_avg = x; s.y_sig = sig; s.yp_avg = xp; s.yp_sig = sigp; s.y_emit = emit; }
   }
-  if (relative_phi(b, false)) return -1;
-  Sums r;   // beam.cu:1069-1092, beam_kernel.cu:1356-1373
-  if (run_sums(b, b->d.phi_r, b->d.w, 0, &r)) return -1;
+  const BeamSums& r = b->ro->sums[2];   // beam.cu:1069-1092, beam_kernel.cu:1356-1373
   const double sv = surv(b, s);
   const double phi = r.s[0] / sv, phi2 = r.s[1] / sv, w = r.s[2] / sv, w2 = r.s[3] / sv,
                phi_w = r.s[4] / sv;
@@ -249,6 +236,16 @@ int emittance(hps_beam* b, hps_beam_stats& s)   // Beam::UpdateEmittance, beam.c
   return 0;
 }
 
+// All particle arrays src -> dst in one launch (save, restore).
+BeamArrays snapshot(const hps_beam* b, int slot)
+{
+  BeamArrays a = b->d;
+  double* const* v = b->snap[slot];
+  a.x = v[0]; a.xp = v[1]; a.y = v[2]; a.yp = v[3]; a.phi = v[4]; a.w = v[5];
+  a.loss = b->snap_l[slot][0]; a.lloss = b->snap_l[slot][1];
+  return a;
+}
+
 void free_beam(hps_beam* b)
 {
   double* arrs[7] = {b->d.x, b->d.xp, b->d.y, b->d.yp, b->d.phi, b->d.phi_r, b->d.w};
@@ -260,8 +257,8 @@ void free_beam(hps_beam* b)
   (void)hipFree(b->pr.cnt);
   (void)hipFree(b->pr.pmax);
   (void)hipFree(b->pr.rmax2);
-  (void)hipFree(b->pr.out);
-  (void)hipFree(b->pr.out_cnt);
+  (void)hipHostFree(b->ro);
+  (void)hipHostFree(b->stage);
   for (int k = 0; k < 2; ++k) {
     for (int j = 0; j < 6; ++j) (void)hipFree(b->snap[k][j]);
     (void)hipFree(b->snap_l[k][0]);
@@ -361,8 +358,7 @@ int hps_beam_create(hps_beam** out, uint32_t num, double mass, double charge, do
        hipMemset(b->pr.pmax, 0, (size_t)b->pr.mpad * 8) == hipSuccess;
   ok = ok && hipMalloc(&b->pr.rmax2, (size_t)b->pr.mpad * 8) == hipSuccess &&
        hipMemset(b->pr.rmax2, 0, (size_t)b->pr.mpad * 8) == hipSuccess;
-  ok = ok && hipMalloc(&b->pr.out, kMaxQ * sizeof(double)) == hipSuccess;
-  ok = ok && hipMalloc(&b->pr.out_cnt, 4 * sizeof(uint32_t)) == hipSuccess;
+  ok = ok && hipHostMalloc((void**)&b->ro, sizeof(Readout), hipHostMallocDefault) == hipSuccess;
   if (!ok) { free_beam(b); delete b; return fail("device allocation failed for the beam"); }
   b->d.n = num; b->d.mass = mass; b->d.charge = charge;
   *out = b;
@@ -519,23 +515,42 @@ int hps_beam_download(hps_beam* b, double* x, double* xp, double* y, double* yp,
                       double* w, uint32_t* loss, uint32_t* lloss)
 {
   if (!b) return fail("null beam");
-  HPS_CHECK(hipStreamSynchronize(b->stream));
   const size_t nd = (size_t)b->n * sizeof(double), nu = (size_t)b->n * 4;
-  if (x) HPS_CHECK(hipMemcpy(x, b->d.x, nd, hipMemcpyDeviceToHost));
-  if (xp) HPS_CHECK(hipMemcpy(xp, b->d.xp, nd, hipMemcpyDeviceToHost));
-  if (y) HPS_CHECK(hipMemcpy(y, b->d.y, nd, hipMemcpyDeviceToHost));
-  if (yp) HPS_CHECK(hipMemcpy(yp, b->d.yp, nd, hipMemcpyDeviceToHost));
-  if (phi) HPS_CHECK(hipMemcpy(phi, b->d.phi, nd, hipMemcpyDeviceToHost));
-  if (w) HPS_CHECK(hipMemcpy(w, b->d.w, nd, hipMemcpyDeviceToHost));
-  if (loss) HPS_CHECK(hipMemcpy(loss, b->d.loss, nu, hipMemcpyDeviceToHost));
-  if (lloss) HPS_CHECK(hipMemcpy(lloss, b->d.lloss, nu, hipMemcpyDeviceToHost));
+  double* const out[6] = {x, xp, y, yp, phi, w};
+  uint32_t* const out_l[2] = {loss, lloss};
+  const double* src[6] = {b->d.x, b->d.xp, b->d.y, b->d.yp, b->d.phi, b->d.w};
+  const uint32_t* src_l[2] = {b->d.loss, b->d.lloss};
+  if (6 * nd + 2 * nu <= kStageBytes) {
+    // a small beam: one kernel writes the arrays into pinned memory, one wait
+    // (eight copies of 16 KB, each with its own wait: 160 us; so 25)
+    if (!b->stage)
+      HPS_CHECK(hipHostMalloc((void**)&b->stage, 6 * nd + 2 * nu, hipHostMallocDefault));
+    BeamArrays dst = b->d;
+    uint8_t* at = b->stage;
+    double** dd[6] = {&dst.x, &dst.xp, &dst.y, &dst.yp, &dst.phi, &dst.w};
+    for (double** d : dd) { *d = (double*)at; at += nd; }
+    dst.loss = (uint32_t*)at; dst.lloss = (uint32_t*)(at + nu);
+    HPS_CHECK(launch_copy_beam(b->d, dst, b->stream));
+    HPS_CHECK(hipStreamSynchronize(b->stream));
+    for (int k = 0; k < 6; ++k)
+      if (out[k]) std::memcpy(out[k], *dd[k], nd);
+    if (loss) std::memcpy(loss, dst.loss, nu);
+    if (lloss) std::memcpy(lloss, dst.lloss, nu);
+    return 0;
+  }
+  HPS_CHECK(hipStreamSynchronize(b->stream));
+  for (int k = 0; k < 6; ++k)
+    if (out[k]) HPS_CHECK(hipMemcpy(out[k], src[k], nd, hipMemcpyDeviceToHost));
+  for (int k = 0; k < 2; ++k)
+    if (out_l[k]) HPS_CHECK(hipMemcpy(out_l[k], src_l[k], nu, hipMemcpyDeviceToHost));
   return 0;
 }
 
 int hps_beam_relative_phi(hps_beam* b, int use_good, double* out)
 {
   if (!b) return fail("null beam");
-  if (relative_phi(b, use_good != 0)) return -1;
+  // UpdateRelativePhiKernelCall, beam.cu:1122-1131
+  HPS_CHECK(launch_relative_phi(b->d, use_good ? &b->st->phi_avg_good : b->d.phi, b->stream));
   HPS_CHECK(hipStreamSynchronize(b->stream));
   if (out) HPS_CHECK(hipMemcpy(out, b->d.phi_r, (size_t)b->n * 8, hipMemcpyDeviceToHost));
   return 0;
@@ -577,7 +592,10 @@ int hps_beam_get_scalar(hps_beam* b, int which, double* out)
     case 6: v = b->design_w; break;
     case 7: {   // BeamGetCurrent, wrap_beam.cpp:1286-1298
       hps_beam_stats s;
-      if (pull(b, &s) || update_loss(b, s) || push(b, &s)) return -1;
+      const Pair counts{nullptr, nullptr, 2, nullptr};
+      if (read_sums(b, &counts, 1, &s)) return -1;
+      s.num_loss = b->ro->sums[0].nloss;
+      if (push(b, s)) return -1;
       v = b->current * (1.0 - ((double)s.num_loss) / ((double)b->n));
       break;
     }
@@ -591,90 +609,72 @@ int hps_beam_get_loss_num(hps_beam* b, int which, uint32_t* out)   // wrap_beam.
 {
   if (!b || !out) return fail("null argument");
   hps_beam_stats s;
-  if (pull(b, &s)) return -1;
   if (which == 0) {
-    if (update_loss(b, s)) return -1;
+    const Pair counts{nullptr, nullptr, 2, nullptr};
+    if (read_sums(b, &counts, 1, &s)) return -1;
+    s.num_loss = b->ro->sums[0].nloss;
     *out = s.num_loss;
-  } else if (which == 1) {
-    if (update_longitudinal_loss(b, s)) return -1;
-    *out = s.num_lloss;
   } else {
-    if (update_loss(b, s) || update_longitudinal_loss(b, s) || update_good(b, s)) return -1;
-    *out = b->n - s.num_good;
+    if (update_longitudinal_loss(b, s, which != 1)) return -1;
+    *out = which == 1 ? s.num_lloss : b->n - s.num_good;
   }
-  return push(b, &s);
+  return push(b, s);
 }
 
 int hps_beam_get_avg(hps_beam* b, int var, int good, double* out)   // wrap_beam.cpp:914-1049
 {
   if (!b || !out) return fail("null argument");
+  // var 0 x, 1 y, 2 phi, 3 w, else the phase relative to particle 0
+  const double* arr[4] = {b->d.x, b->d.y, b->d.phi, b->d.w};
+  const bool rel = var < 0 || var > 3;
+  const Pair p{rel ? b->d.phi : arr[var], nullptr, good ? 1 : 0, rel ? b->d.phi : nullptr};
   hps_beam_stats s;
-  if (pull(b, &s) || update_loss(b, s)) return -1;
-  double v = 0;
-  int rc = 0;
-  switch (var) {
-    case 0: rc = avg_of(b, s, b->d.x, good != 0, good ? &s.x_avg_good : &s.x_avg); v = good ? s.x_avg_good : s.x_avg; break;
-    case 1: rc = avg_of(b, s, b->d.y, good != 0, good ? &s.y_avg_good : &s.y_avg); v = good ? s.y_avg_good : s.y_avg; break;
-    case 2:
-      if (!good) { rc = avg_of(b, s, b->d.phi, false, &s.phi_avg); v = s.phi_avg; }
-      else { rc = update_good(b, s) || avg_of(b, s, b->d.phi, true, &s.phi_avg_good); v = s.phi_avg_good; }
-      break;
-    case 3: rc = avg_of(b, s, b->d.w, good != 0, good ? &s.w_avg_good : &s.w_avg); v = good ? s.w_avg_good : s.w_avg; break;
-    default:
-      rc = relative_phi(b, false) || avg_of(b, s, b->d.phi_r, good != 0, &s.phi_avg_r);
-      v = s.phi_avg_r;
-      break;
-  }
-  if (rc || push(b, &s)) return -1;
-  *out = v;
-  return 0;
+  if (read_sums(b, &p, 1, &s)) return -1;
+  const BeamSums& r = b->ro->sums[0];
+  s.num_loss = r.nloss;                             // UpdateLoss
+  if (var == 2 && good) s.num_good = r.ngood;       // UpdateGoodParticleCount
+  double* const at[4][2] = {{&s.x_avg, &s.x_avg_good}, {&s.y_avg, &s.y_avg_good},
+                            {&s.phi_avg, &s.phi_avg_good}, {&s.w_avg, &s.w_avg_good}};
+  double* const v = rel ? &s.phi_avg_r : at[var][good ? 1 : 0];
+  *v = avg_of(b, s, r, good != 0);
+  *out = *v;
+  return push(b, s);
 }
 
 int hps_beam_get_sig(hps_beam* b, int var, int good, double* out)   // wrap_beam.cpp:1051-1186
 {
   if (!b || !out) return fail("null argument");
+  const double* arr[4] = {b->d.x, b->d.y, b->d.phi, b->d.w};
+  const bool rel = var < 0 || var > 3;
+  const bool phi_good = var == 2 && good;
+  // the relative phase's spread counts every particle that is not lost
+  const Pair p{rel ? b->d.phi : arr[var], nullptr, good && !rel ? 1 : 0, rel ? b->d.phi : nullptr};
   hps_beam_stats s;
-  if (pull(b, &s) || update_loss(b, s)) return -1;
-  if (b->n < 2) { *out = 0.0; return push(b, &s); }
+  if (read_sums(b, &p, 1, &s)) return -1;
+  s.num_loss = b->ro->sums[0].nloss;
+  if (b->n < 2) { *out = 0.0; return push(b, s); }
   const bool upd = b->n > 2;
-  double v = 0;
-  int rc = 0;
-  switch (var) {
-    case 0:
-      if (upd) rc = sig_of(b, s, b->d.x, good != 0, good ? &s.x_sig_good : &s.x_sig);
-      v = good ? s.x_sig_good : s.x_sig;
-      break;
-    case 1:
-      if (upd) rc = sig_of(b, s, b->d.y, good != 0, good ? &s.y_sig_good : &s.y_sig);
-      v = good ? s.y_sig_good : s.y_sig;
-      break;
-    case 2:
-      if (!good) { if (upd) rc = sig_of(b, s, b->d.phi, false, &s.phi_sig); v = s.phi_sig; break; }
-      rc = update_good(b, s) || avg_of(b, s, b->d.phi, true, &s.phi_avg_good) || push(b, &s) ||
-           relative_phi(b, true);
-      if (!rc && upd) rc = sig_of(b, s, b->d.phi_r, true, &s.phi_sig_good);
-      v = s.phi_sig_good;
-      break;
-    case 3:
-      if (upd) rc = sig_of(b, s, b->d.w, good != 0, good ? &s.w_sig_good : &s.w_sig);
-      v = good ? s.w_sig_good : s.w_sig;
-      break;
-    default:
-      rc = relative_phi(b, false);
-      if (!rc && upd) rc = sig_of(b, s, b->d.phi_r, false, &s.phi_sig_r);
-      v = s.phi_sig_r;
-      break;
+  double* const at[4][2] = {{&s.x_sig, &s.x_sig_good}, {&s.y_sig, &s.y_sig_good},
+                            {&s.phi_sig, &s.phi_sig_good}, {&s.w_sig, &s.w_sig_good}};
+  double* const v = rel ? &s.phi_sig_r : at[var][good ? 1 : 0];
+  if (phi_good) {
+    // about the good particles' mean phase: a second pass against it
+    s.num_good = b->ro->sums[0].ngood;
+    s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+    if (push(b, s)) return -1;
+    const Pair q{b->d.phi, nullptr, 1, &b->st->phi_avg_good};
+    if (upd && read_sums(b, &q, 1, nullptr)) return -1;
   }
-  if (rc || push(b, &s)) return -1;
-  *out = v;
-  return 0;
+  if (upd) *v = sig_of(b, s, b->ro->sums[0], good && !rel);
+  *out = *v;
+  return push(b, s);
 }
 
 int hps_beam_get_emittance(hps_beam* b, int axis, double* out)   // wrap_beam.cpp:1188-1243
 {
   if (!b || !out) return fail("null argument");
   hps_beam_stats s;
-  if (pull(b, &s) || update_loss(b, s) || emittance(b, s) || push(b, &s)) return -1;
+  if (emittance(b, s) || push(b, s)) return -1;
   if (b->n < 2) { *out = 0.0; return 0; }
   *out = axis == 0 ? s.x_emit : (axis == 1 ? s.y_emit : s.z_emit);
   return 0;
@@ -690,16 +690,11 @@ int hps_beam_save(hps_beam* b, int slot)   // beam.cpp:547-595
 {
   if (!b || slot < 0 || slot > 1) return fail("bad save slot");
   const size_t nd = (size_t)b->n * 8, nu = (size_t)b->n * 4;
-  double* src[6] = {b->d.x, b->d.xp, b->d.y, b->d.yp, b->d.phi, b->d.w};
-  for (int j = 0; j < 6; ++j) {
+  for (int j = 0; j < 6; ++j)
     if (!b->snap[slot][j]) HPS_CHECK(hipMalloc(&b->snap[slot][j], nd));
-    HPS_CHECK(hipMemcpyAsync(b->snap[slot][j], src[j], nd, hipMemcpyDeviceToDevice, b->stream));
-  }
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < 2; ++j)
     if (!b->snap_l[slot][j]) HPS_CHECK(hipMalloc(&b->snap_l[slot][j], nu));
-    HPS_CHECK(hipMemcpyAsync(b->snap_l[slot][j], j ? b->d.lloss : b->d.loss, nu,
-                             hipMemcpyDeviceToDevice, b->stream));
-  }
+  HPS_CHECK(launch_copy_beam(b->d, snapshot(b, slot), b->stream));
   HPS_CHECK(hipStreamSynchronize(b->stream));
   b->saved[slot] = true;
   b->snap_dw[slot] = b->design_w; b->snap_f[slot] = b->freq; b->snap_c[slot] = b->current;
@@ -710,18 +705,13 @@ int hps_beam_restore(hps_beam* b, int slot)   // beam.cpp:606-647
 {
   if (!b || slot < 0 || slot > 1) return fail("bad restore slot");
   if (!b->saved[slot]) return fail("Beam can't be restored because no previous beam has been saved.");
-  const size_t nd = (size_t)b->n * 8, nu = (size_t)b->n * 4;
-  double* dst[6] = {b->d.x, b->d.xp, b->d.y, b->d.yp, b->d.phi, b->d.w};
-  for (int j = 0; j < 6; ++j)
-    HPS_CHECK(hipMemcpyAsync(dst[j], b->snap[slot][j], nd, hipMemcpyDeviceToDevice, b->stream));
-  HPS_CHECK(hipMemcpyAsync(b->d.loss, b->snap_l[slot][0], nu, hipMemcpyDeviceToDevice, b->stream));
-  HPS_CHECK(hipMemcpyAsync(b->d.lloss, b->snap_l[slot][1], nu, hipMemcpyDeviceToDevice, b->stream));
+  HPS_CHECK(launch_copy_beam(snapshot(b, slot), b->d, b->stream));
   b->design_w = b->snap_dw[slot]; b->freq = b->snap_f[slot]; b->current = b->snap_c[slot];
   hps_beam_stats s;
-  if (pull(b, &s) || avg_of(b, s, b->d.phi, true, &s.phi_avg_good) || push(b, &s)) return -1;
-  if (relative_phi(b, true)) return -1;
-  HPS_CHECK(hipStreamSynchronize(b->stream));
-  return 0;
+  const Pair phi{b->d.phi, nullptr, 1, nullptr};
+  if (read_sums(b, &phi, 1, &s)) return -1;
+  s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+  return push(b, s);
 }
 
 int hps_beam_translate(hps_beam* b, int axis, double val)   // beam.cpp:1612-1652
@@ -2534,8 +2524,8 @@ constexpr uint32_t kNoAllocChunks = kNoAllocMaxParticles / kChunk;             /
 constexpr size_t kNoAllocSumsOff = 0;
 constexpr size_t kNoAllocCntOff = kNoAllocSumsOff + (size_t)kMaxQ * kNoAllocChunks * 8;
 constexpr size_t kNoAllocOutOff = kNoAllocCntOff + 3 * (size_t)kNoAllocChunks * 4;
-constexpr size_t kNoAllocOutCntOff = kNoAllocOutOff + kMaxQ * 8;
-constexpr size_t kNoAllocBytes = kNoAllocOutCntOff + 256;                       // 311,616 B
+constexpr size_t kNoAllocBytes = kNoAllocOutOff + 320;                         // 311,616 B
+static_assert(sizeof(BeamSums) <= 320, "the final sums");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -2582,8 +2572,7 @@ extern "C" int hps_emittance_noalloc(const double* x, const double* xp, const do
   Partials pr{};
   pr.sums = (double*)(base + kNoAllocSumsOff);
   pr.cnt = (uint32_t*)(base + kNoAllocCntOff);
-  pr.out = (double*)(base + kNoAllocOutOff);
-  pr.out_cnt = (uint32_t*)(base + kNoAllocOutCntOff);
+  BeamSums* const out_sums = (BeamSums*)(base + kNoAllocOutOff);
   pr.nch = (n + kChunk - 1) / kChunk;
   pr.mpad = next_pow2(pr.nch);
   // the trees read the zero padding past the last chunk (left over by an
@@ -2610,12 +2599,12 @@ extern "C" int hps_emittance_noalloc(const double* x, const double* xp, const do
   // the same pass
   auto sums = [&](const double* pa, const double* pb, const double* rel, double* r5,
                   uint32_t* nloss) -> int {
-    HPS_CHECK(launch_sums(a, pa, pb, 0, pr, s, rel));
-    uint32_t c[3];
-    HPS_CHECK(hipMemcpyAsync(r5, pr.out, 5 * sizeof(double), hipMemcpyDeviceToHost, s));
-    HPS_CHECK(hipMemcpyAsync(c, pr.out_cnt, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    HPS_CHECK(launch_sums(a, pa, pb, 0, pr, s, rel, out_sums, nullptr, nullptr));
+    BeamSums r;
+    HPS_CHECK(hipMemcpyAsync(&r, out_sums, sizeof r, hipMemcpyDeviceToHost, s));
     HPS_CHECK(hipStreamSynchronize(s));
-    *nloss = c[0];
+    for (int q = 0; q < 5; ++q) r5[q] = r.s[q];
+    *nloss = r.nloss;
     return 0;
   };
   for (int axis = 0; axis < 2; ++axis) {

@@ -45,8 +45,6 @@ struct Partials {
   uint32_t* cnt;       // [3][mpad]
   double* pmax;        // [mpad]
   double* rmax2;       // [mpad] largest r^2 about (x_avg, y_avg), loss == 0
-  double* out;         // [kMaxQ] final sums for host-side getters
-  uint32_t* out_cnt;   // [1]
   uint32_t mpad;       // NextPow2(nchunks)
   uint32_t nch;        // chunks
 };
@@ -290,11 +288,27 @@ hipError_t launch_capture(const GemmMember* mem, uint32_t nmem, const GemmState*
 
 // Generic canonical sums for the getters: over the filtered particles
 // (filter 0: loss == 0, 1: loss + lloss == 0, 2: all) of a, a*a, b, b*b, a*b,
-// and the count of loss != 0, of (loss+lloss) == 0 and of lloss != 0.
-// Results land in pr.out[0..4] and pr.out_cnt[0..2].  With rel_ref, a is
-// replaced by its relative phase against rel_ref[0] (k_relative_phi's value).
+// and the count of loss != 0, of (loss+lloss) == 0 and of lloss != 0, written
+// to *out (device or pinned memory).  With rel_ref, a is replaced by its
+// relative phase against rel_ref[0] (k_relative_phi's value).  With ro, the
+// statistics st and w[0] are written there too.
+struct BeamSums {
+  double s[5];
+  uint32_t nloss, ngood, nlloss, pad_;
+};
+constexpr int kReadSlots = 3;
+struct Readout {
+  BeamSums sums[kReadSlots];
+  hps_beam_stats st;
+  double w0;
+};
 hipError_t launch_sums(BeamArrays b, const double* a, const double* bb, int filter,
-                       Partials pr, hipStream_t s, const double* rel_ref = nullptr);
+                       Partials pr, hipStream_t s, const double* rel_ref, BeamSums* out,
+                       Readout* ro, const hps_beam_stats* st);
+// *st = s, as a kernel argument
+hipError_t launch_set_stats(hps_beam_stats* st, const hps_beam_stats& s, hipStream_t stream);
+// the six coordinates and two loss arrays src -> dst (n particles)
+hipError_t launch_copy_beam(const BeamArrays& src, const BeamArrays& dst, hipStream_t s);
 hipError_t launch_relative_phi(BeamArrays b, const double* ref, hipStream_t s);
 hipError_t launch_lloss_flag(BeamArrays b, const double* avg, hipStream_t s);
 hipError_t launch_shift(double* a, uint32_t n, double v, hipStream_t s);

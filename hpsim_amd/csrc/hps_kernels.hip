@@ -1848,17 +1848,38 @@ __global__ __launch_bounds__(kBlock) void k_sums(BeamArrays b, const double* pa,
 }
 
 // Cross-chunk trees of k_sums in one workgroup.
-__global__ __launch_bounds__(512) void k_sums_final(Partials pr)
+__global__ __launch_bounds__(576) void k_sums_final(Partials pr, BeamSums* out, Readout* ro,
+                                                    const hps_beam_stats* st, const double* w)
 {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
   if (wave < 5) {
     const double v = wave_tree_sum(pr.sums + (size_t)wave * pr.mpad, pr.mpad, l);
-    if (l == 0) pr.out[wave] = v;
-  } else {
+    if (l == 0) out->s[wave] = v;
+  } else if (wave < 8) {
     const int k = wave - 5;
     const uint32_t n = wave_count(pr.cnt + (size_t)k * pr.mpad, pr.nch, l);
-    if (l == 0) pr.out_cnt[k] = n;
+    if (l == 0) (&out->nloss)[k] = n;
+  } else if (ro) {
+    constexpr int kWords = sizeof(hps_beam_stats) / 4;
+    for (int i = l; i < kWords; i += 64) ((uint32_t*)&ro->st)[i] = ((const uint32_t*)st)[i];
+    if (l == 0) ro->w0 = w[0];
   }
+}
+
+__global__ void k_set_stats(hps_beam_stats* st, hps_beam_stats s)
+{
+  if (threadIdx.x == 0) *st = s;
+}
+
+// A particle per thread, 56 bytes in flight each way.
+__global__ __launch_bounds__(kBlock) void k_copy_beam(BeamArrays src, BeamArrays dst)
+{
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= src.n) return;
+  gst(dst.x, i, gld(src.x, i)); gst(dst.xp, i, gld(src.xp, i));
+  gst(dst.y, i, gld(src.y, i)); gst(dst.yp, i, gld(src.yp, i));
+  gst(dst.phi, i, gld(src.phi, i)); gst(dst.w, i, gld(src.w, i));
+  gst(dst.loss, i, gld(src.loss, i)); gst(dst.lloss, i, gld(src.lloss, i));
 }
 
 __global__ void k_relative_phi(BeamArrays b, const double* ref)
@@ -2182,11 +2203,24 @@ hipError_t launch_field_batch(const FieldArgs* recs, uint32_t nmem, uint32_t nr,
 }
 
 hipError_t launch_sums(BeamArrays b, const double* a, const double* bb, int filter, Partials pr,
-                       hipStream_t s, const double* rel_ref)
+                       hipStream_t s, const double* rel_ref, BeamSums* out, Readout* ro,
+                       const hps_beam_stats* st)
 {
   const uint32_t nch = (b.n + kChunk - 1) / kChunk;
   hipLaunchKernelGGL(k_sums, dim3(nch), dim3(kBlock), 0, s, b, a, bb, filter, pr, rel_ref);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(512), 0, s, pr);
+  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(576), 0, s, pr, out, ro, st, b.w);
+  return hipGetLastError();
+}
+
+hipError_t launch_set_stats(hps_beam_stats* st, const hps_beam_stats& v, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_set_stats, dim3(1), dim3(64), 0, s, st, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_beam(const BeamArrays& src, const BeamArrays& dst, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_copy_beam, dim3(blocks_for(src.n)), dim3(kBlock), 0, s, src, dst);
   return hipGetLastError();
 }
 
