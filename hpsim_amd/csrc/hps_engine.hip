@@ -1678,7 +1678,7 @@ static void free_gemm(hps_batch* bt)
   (void)hipFree(bt->mm.pos_exact); (void)hipFree(bt->mm.pos_nn); (void)hipFree(bt->mm.fallback);
   (void)hipFree(bt->mm.qtot); (void)hipFree(bt->d_xinf); (void)hipFree(bt->d_uinf);
   (void)hipFree(bt->fft.tw); (void)hipFree(bt->fft.shat); (void)hipFree(bt->fft.spec_class);
-  (void)hipFree(bt->fft.list); (void)hipFree(bt->fft.qhat); (void)hipFree(bt->fft.what);
+  (void)hipFree(bt->fft.qhat); (void)hipFree(bt->fft.what);
   bt->fft = FftBufs{};
   bt->mm = MemberMap{};
   bt->d_xinf = nullptr; bt->d_uinf = nullptr;
@@ -1731,8 +1731,7 @@ static int alloc_gemm(hps_batch* bt, uint32_t nr, uint32_t nz, uint32_t B, hipSt
     HPS_CHECK(hipMalloc(&bt->fft.spec_class, kGemmSlots * sizeof(int32_t)));
     HPS_CHECK(hipMemcpy(bt->fft.spec_class, none.data(), kGemmSlots * sizeof(int32_t),
                         hipMemcpyHostToDevice));
-    HPS_CHECK(hipMalloc(&bt->fft.list, (kGemmSlots + 1) * sizeof(uint32_t)));
-    HPS_CHECK(hipMalloc(&bt->fft.qhat, kGemmCols * (size_t)B * F * nr * sizeof(float2)));
+    HPS_CHECK(hipMalloc(&bt->fft.qhat, (size_t)B * F * nr * sizeof(float2)));
     HPS_CHECK(hipMalloc(&bt->fft.what, kGemmCols * (size_t)B * F * R * sizeof(float2)));
   }
   bt->gemm_key[0] = nr; bt->gemm_key[1] = nz; bt->gemm_key[2] = B;
@@ -1751,16 +1750,16 @@ static int tune_gemm(hps_batch* bt, uint32_t nr, uint32_t nz, uint32_t B, hipStr
   for (auto& e : ev) HPS_CHECK(hipEventCreate(&e));
   // untimed first launches: the direct product, and the spectral one, whose
   // first launch also transforms the class tables in use (kept for later)
-  HPS_CHECK(launch_gemm_product(bt->d_gs, bt->d_tables, bt->d_q, bt->d_w, nr, nz, 0, bt->cus,
+  HPS_CHECK(launch_gemm_product(bt->d_mem, B, bt->d_gs, bt->d_perm, bt->mm, bt->d_tables, bt->d_q, bt->d_w, nr, nz, 0, bt->cus,
                                 fb, s));
   for (uint32_t k = 0; k < n; ++k)
     if (gemm_shape(k).spectral && fb)
-      HPS_CHECK(launch_gemm_product(bt->d_gs, bt->d_tables, bt->d_q, bt->d_w, nr, nz, k,
+      HPS_CHECK(launch_gemm_product(bt->d_mem, B, bt->d_gs, bt->d_perm, bt->mm, bt->d_tables, bt->d_q, bt->d_w, nr, nz, k,
                                     bt->cus, fb, s));
   for (uint32_t k = 0; k < n; ++k) {
     HPS_CHECK(hipEventRecord(ev[2 * k], s));
     if (!gemm_shape(k).spectral || fb)
-      HPS_CHECK(launch_gemm_product(bt->d_gs, bt->d_tables, bt->d_q, bt->d_w, nr, nz, k,
+      HPS_CHECK(launch_gemm_product(bt->d_mem, B, bt->d_gs, bt->d_perm, bt->mm, bt->d_tables, bt->d_q, bt->d_w, nr, nz, k,
                                     bt->cus, fb, s));
     HPS_CHECK(hipEventRecord(ev[2 * k + 1], s));
   }
@@ -2261,6 +2260,8 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
           SurCtl* ctl = bt->sur ? bt->d_sur : nullptr;
           HPS_CHECK(launch_gemm_prepare(bt->d_mem, (uint32_t)B, bt->d_gs, bt->d_perm, bt->mm, ctl,
                                         bt->d_tables, bt->d_q, nr, nz, bt->aspect_lnr, bt->cus,
+                                        bt->gemm_shape == UINT32_MAX ||
+                                            !gemm_shape(bt->gemm_shape).spectral,
                                         s));
           if (bt->gemm_shape == UINT32_MAX && tune_gemm(bt, nr, nz, (uint32_t)B, s)) return -1;
           if (gemm_shape(bt->gemm_shape).spectral && !bt->fft.tw)
@@ -2274,7 +2275,7 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
             marks.push_back({6, nev});
             HPS_CHECK(hipEventRecord(bt->evpool[nev], s));
           }
-          HPS_CHECK(launch_gemm_product(bt->d_gs, bt->d_tables, bt->d_q, bt->d_w, nr, nz,
+          HPS_CHECK(launch_gemm_product(bt->d_mem, B, bt->d_gs, bt->d_perm, bt->mm, bt->d_tables, bt->d_q, bt->d_w, nr, nz,
                                         bt->gemm_shape, bt->cus,
                                         bt->fft.tw ? &bt->fft : nullptr, s));
           if (bt->profile) {

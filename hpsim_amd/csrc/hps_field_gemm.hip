@@ -70,15 +70,17 @@ __host__ __device__ __forceinline__ uint32_t ceil_div(uint32_t a, uint32_t b) { 
 
 // ---- schedule --------------------------------------------------------------
 
-// One workgroup.  Thread 0 walks the members in order.  A remeshing member
-// gets the exact product when no surrogate runs, or at an audit kick
-// point, or when its last audit failed: three product columns, for its
-// classes c - 1, c, c + 1 (class table of class k in slot k mod kGemmSlots; a slot
-// holding another class is rebuilt, unless another class already claimed it
-// at this kick point -- then the column uses the slot's class, counted in
-// conflicts).  Columns are grouped by slot (counting sort, member order
-// kept) in perm; with a surrogate, every remeshing member also gets a
-// position in the network's batch.
+// One workgroup.  A remeshing member gets the exact product when no surrogate
+// runs, or at an audit kick point, or when its last audit failed: three
+// product columns, for its classes c - 1, c, c + 1 (class table of class k in
+// slot k mod kGemmSlots; a slot holding another class is rebuilt, unless
+// another class already claimed it at this kick point -- then the column uses
+// the slot's class, counted in conflicts).  Columns are grouped by slot
+// (counting sort, member order kept) in perm; with a surrogate, every
+// remeshing member also gets a position in the network's batch.  Thread 0
+// walks the members in order, on LDS copies: every thread loads members'
+// flags and writes their positions, one slot's state each for the first
+// kGemmSlots.
 __global__ __launch_bounds__(kThreads) void k_gemm_schedule(const GemmMember* __restrict__ mem,
                                                             uint32_t nmem, GemmState* gs,
                                                             uint32_t* perm, MemberMap mm,
@@ -86,21 +88,23 @@ __global__ __launch_bounds__(kThreads) void k_gemm_schedule(const GemmMember* __
 {
   __shared__ uint32_t count[kGemmSlots];
   __shared__ uint32_t claimed[kGemmSlots];
-  static_assert(kGemmSlots <= 127, "slot numbers are kept in int8");
+  __shared__ int32_t cls[kGemmSlots];
+  __shared__ uint8_t build[kGemmSlots];
+  static_assert(kGemmSlots <= 64 && kGemmSlots <= kThreads, "one wave scans the slots");
   __shared__ int8_t mslot[kGemmCols * kGemmMaxMembers];
   __shared__ int32_t mclass[kGemmMaxMembers];   // first class c - 1 of a remeshing member
-  __shared__ uint8_t mrem[kGemmMaxMembers];     // the member remeshes at this kick point
-  __shared__ uint32_t any_rem;
+  __shared__ uint8_t mrem[kGemmMaxMembers];     // 1: the member remeshes, 2: and takes the product
+  __shared__ int16_t mnn[kGemmMaxMembers];      // place in the network's batch
+  __shared__ uint16_t mrank[kGemmCols * kGemmMaxMembers];   // column's place in its slot
+  __shared__ uint32_t any_rem, s_nbuild, s_conflicts, s_nn, s_ncol;
   const int t = threadIdx.x;
-  if (t < (int)kGemmSlots) { count[t] = 0; claimed[t] = 0; }
+  if (t < (int)kGemmSlots) { count[t] = 0; claimed[t] = 0; cls[t] = gs->slot_class[t]; }
   if (t == 0) any_rem = 0;
   __syncthreads();
-  // every member's remesh flag and aspect class, loaded by all threads (one
-  // dependent pair of loads per member); thread 0 then walks them in order
   for (uint32_t m = t; m < nmem; m += kThreads) {
     const ScDev* sc = mem[m].sc;
     const uint32_t rem = sc->remesh;
-    mrem[m] = rem ? 1 : 0;
+    mrem[m] = rem ? ((!ctl || mm.fallback[m]) ? 2 : 1) : 0;
     if (rem) {
       double wl[3];
       mclass[m] = aspect_lagrange(sc->log_aspect, lnr, wl) - 1;
@@ -108,66 +112,79 @@ __global__ __launch_bounds__(kThreads) void k_gemm_schedule(const GemmMember* __
     }
   }
   __syncthreads();
-  if (t != 0) return;
-  bool audit = false;
-  if (ctl) {
-    const uint32_t any = any_rem;
-    if (ctl->audit_every && ctl->kick % ctl->audit_every == 0) ctl->pending = 1;
-    ctl->kick += 1;
-    audit = ctl->pending && any;
-    if (audit) ctl->pending = 0;
-    ctl->audit_now = audit ? 1 : 0;
-  }
-  uint32_t nbuild = 0, conflicts = gs->conflicts, nn = 0, ncol = 0;
-  for (uint32_t m = 0; m < nmem; ++m) {
-    mm.pos_nn[m] = -1;
-    for (uint32_t h = 0; h < kGemmCols; ++h) mslot[kGemmCols * m + h] = -1;
-    if (!mrem[m]) continue;
-    if (ctl) mm.pos_nn[m] = (int32_t)nn++;
-    if (ctl && !audit && !mm.fallback[m]) continue;
-    const int32_t c0 = mclass[m];
-    for (uint32_t h = 0; h < kGemmCols; ++h) {
-      const int32_t c = c0 + (int32_t)h;
-      const int32_t slot = (int32_t)((uint32_t)c & (kGemmSlots - 1));
-      if (gs->slot_class[slot] != c) {
-        if (!claimed[slot]) {
-          gs->slot_class[slot] = c;
-          gs->build[nbuild++] = (uint32_t)slot;
-        } else {
-          ++conflicts;
+  if (t == 0) {
+    bool audit = false;
+    if (ctl) {
+      if (ctl->audit_every && ctl->kick % ctl->audit_every == 0) ctl->pending = 1;
+      ctl->kick += 1;
+      audit = ctl->pending && any_rem;
+      if (audit) ctl->pending = 0;
+      ctl->audit_now = audit ? 1 : 0;
+    }
+    uint32_t nbuild = 0, conflicts = 0, nn = 0, ncol = 0;
+    for (uint32_t m = 0; m < nmem; ++m) {
+      const uint8_t rem = mrem[m];
+      mnn[m] = ctl && rem ? (int16_t)nn++ : (int16_t)-1;
+      const bool product = rem && (audit || rem == 2);
+      for (uint32_t h = 0; h < kGemmCols; ++h) {
+        mslot[kGemmCols * m + h] = -1;
+        if (!product) continue;
+        const int32_t c = mclass[m] + (int32_t)h;
+        const int32_t slot = (int32_t)((uint32_t)c & (kGemmSlots - 1));
+        if (cls[slot] != c) {
+          if (!claimed[slot]) {
+            cls[slot] = c;
+            build[nbuild++] = (uint8_t)slot;
+          } else {
+            ++conflicts;
+          }
         }
+        claimed[slot] = 1;
+        mrank[kGemmCols * m + h] = (uint16_t)count[slot]++;
+        mslot[kGemmCols * m + h] = (int8_t)slot;
+        ++ncol;
       }
-      claimed[slot] = 1;
-      count[slot] += 1;
-      mslot[kGemmCols * m + h] = (int8_t)slot;
-      ++ncol;
+    }
+    s_nbuild = nbuild; s_conflicts = conflicts; s_nn = nn; s_ncol = ncol;
+  }
+  __syncthreads();
+  if (t < (int)kGemmSlots) {
+    uint32_t n = count[t];
+#pragma unroll
+    for (uint32_t o = 1; o < kGemmSlots; o <<= 1) {   // inclusive scan
+      const uint32_t v = __shfl_up(n, o, 64);
+      if ((uint32_t)t >= o) n += v;
+    }
+    const uint32_t start = n - count[t];
+    gs->slot_class[t] = cls[t];
+    gs->slot_start[t] = start;
+    gs->slot_count[t] = count[t];
+    if ((uint32_t)t < s_nbuild) gs->build[t] = build[t];
+    claimed[t] = start;
+  }
+  if (t == 0) {
+    gs->nbuild = s_nbuild;
+    gs->builds_total += s_nbuild;
+    gs->conflicts += s_conflicts;
+    gs->nrem = s_ncol;
+    gs->exact_total += s_ncol;
+    if (ctl) {
+      ctl->nn_n = s_nn;
+      ctl->nn_member_kicks += s_nn;
+      ctl->exact_member_kicks += s_ncol / kGemmCols;
     }
   }
-  gs->nbuild = nbuild;
-  gs->builds_total += nbuild;
-  gs->conflicts = conflicts;
-  uint32_t start = 0;
-  for (uint32_t s = 0; s < kGemmSlots; ++s) {
-    gs->slot_start[s] = start;
-    gs->slot_count[s] = count[s];
-    start += count[s];
-    count[s] = gs->slot_start[s];   // running insertion point
-  }
-  gs->nrem = start;
-  gs->exact_total += start;
-  for (uint32_t e = 0; e < kGemmCols * nmem; ++e) {
+  __syncthreads();
+  for (uint32_t e = t; e < kGemmCols * nmem; e += kThreads) {
     const int32_t slot = mslot[e];
-    mm.pos_exact[e] = -1;
+    int32_t p = -1;
     if (slot >= 0) {
-      mm.pos_exact[e] = (int32_t)count[slot];
-      perm[count[slot]++] = e / kGemmCols;
+      p = (int32_t)(claimed[slot] + mrank[e]);
+      perm[p] = e / kGemmCols;
     }
+    mm.pos_exact[e] = p;
   }
-  if (ctl) {
-    ctl->nn_n = nn;
-    ctl->nn_member_kicks += nn;
-    ctl->exact_member_kicks += ncol / kGemmCols;
-  }
+  for (uint32_t m = t; m < nmem; m += kThreads) mm.pos_nn[m] = mnn[m];
 }
 
 // ---- class tables ------------------------------------------------------------
@@ -609,13 +626,15 @@ GemmShape gemm_shape(uint32_t i)
 
 hipError_t launch_gemm_prepare(const GemmMember* mem, uint32_t nmem, GemmState* gs,
                                uint32_t* perm, MemberMap mm, SurCtl* ctl, float* tables, float* q,
-                               uint32_t nr, uint32_t nz, double lnr, uint32_t cus, hipStream_t s)
+                               uint32_t nr, uint32_t nz, double lnr, uint32_t cus, bool pack,
+                               hipStream_t s)
 {
   hipLaunchKernelGGL(k_gemm_schedule, dim3(1), dim3(kThreads), 0, s, mem, nmem, gs, perm, mm,
                      ctl, lnr);
   hipLaunchKernelGGL(k_gemm_tables, dim3(cus), dim3(kThreads), 0, s, gs, tables, nr, nz, lnr);
-  hipLaunchKernelGGL(k_gemm_pack, dim3(kGemmCols * nmem, ceil_div(nr * nz, kThreads)),
-                     dim3(kThreads), 0, s, mem, gs, perm, q, nr, nz);
+  if (pack)
+    hipLaunchKernelGGL(k_gemm_pack, dim3(kGemmCols * nmem, ceil_div(nr * nz, kThreads)),
+                       dim3(kThreads), 0, s, mem, gs, perm, q, nr, nz);
   return hipGetLastError();
 }
 
@@ -655,14 +674,15 @@ hipError_t launch_capture(const GemmMember* mem, uint32_t nmem, const GemmState*
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_product(const GemmState* gs, const float* tables, const float* q, float* w,
-                               uint32_t nr, uint32_t nz, uint32_t shape, uint32_t cus,
-                               const FftBufs* fb, hipStream_t s)
+hipError_t launch_gemm_product(const GemmMember* mem, uint32_t nmem, const GemmState* gs,
+                               const uint32_t* perm, MemberMap mm, const float* tables,
+                               const float* q, float* w, uint32_t nr, uint32_t nz,
+                               uint32_t shape, uint32_t cus, const FftBufs* fb, hipStream_t s)
 {
   const GemmShape sh = gemm_shape(shape);
   if (sh.spectral) {
     if (!fb) return hipErrorInvalidValue;
-    return launch_fft_product(gs, tables, q, w, *fb, nr, nz, cus, s);
+    return launch_fft_product(mem, nmem, gs, perm, mm.pos_exact, tables, w, *fb, nr, nz, cus, s);
   }
   const dim3 grid(cus * sh.per_cu), block(kThreads);
   if (sh.nt == 64)

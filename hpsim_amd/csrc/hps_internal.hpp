@@ -242,35 +242,37 @@ struct SurCtl {
 };
 constexpr size_t kSurCtlConfigBytes = 32;   // audit_every .. lnr
 static_assert(offsetof(SurCtl, kick) == kSurCtlConfigBytes, "SurCtl configuration block");
-// one kick point: prepare (schedule, class tables to build, charges), the
-// product in launch shape `shape` (all shapes give the same field up to the
+// one kick point: prepare (schedule, class tables to build and, when pack,
+// the direct shapes' charges), the product in launch shape `shape` (all shapes give the same field up to the
 // FP32 summation order of their K splits), store (field tables; y: the
 // network's output for members without an exact product)
 hipError_t launch_gemm_prepare(const GemmMember* mem, uint32_t nmem, GemmState* gs,
                                uint32_t* perm, MemberMap mm, SurCtl* ctl, float* tables, float* q,
-                               uint32_t nr, uint32_t nz, double lnr, uint32_t cus, hipStream_t s);
+                               uint32_t nr, uint32_t nz, double lnr, uint32_t cus, bool pack,
+                               hipStream_t s);
 // Buffers of the spectral product (one K split): twiddles exp(-2 pi i k / L)
-// for k < L / 2 (L = 2 nz), the slots' table spectra [slot][f][row][rs]
+// for k < L / 2 (L = 2 nz), the slots' table spectra [slot][f][rs][row]
 // (f = 0 .. nz, row = 2 rp + comp), the class each slot's spectrum belongs
-// to, a worklist of slots to transform, and per product column the charge
-// spectra [p][f][rs] and field spectra [p][f][row].
+// to, the charge spectra [m][f][rs] per member and the field spectra
+// [p][f][row] per product column.
 struct FftBufs {
   float2* tw;
   float2* shat;
   int32_t* spec_class;
-  uint32_t* list;
   float2* qhat;
   float2* what;
 };
 bool fft_product_supported(uint32_t nr, uint32_t nz);
-hipError_t launch_fft_product(const GemmState* gs, const float* tables, const float* q, float* w,
-                              const FftBufs& fb, uint32_t nr, uint32_t nz, uint32_t cus,
-                              hipStream_t s);
+hipError_t launch_fft_product(const GemmMember* mem, uint32_t nmem, const GemmState* gs,
+                              const uint32_t* perm, const int32_t* pos_exact,
+                              const float* tables, float* w, const FftBufs& fb, uint32_t nr,
+                              uint32_t nz, uint32_t cus, hipStream_t s);
 // fb: null when the spectral shape is not available (then only the direct
 // shapes may be asked for)
-hipError_t launch_gemm_product(const GemmState* gs, const float* tables, const float* q, float* w,
-                               uint32_t nr, uint32_t nz, uint32_t shape, uint32_t cus,
-                               const FftBufs* fb, hipStream_t s);
+hipError_t launch_gemm_product(const GemmMember* mem, uint32_t nmem, const GemmState* gs,
+                               const uint32_t* perm, MemberMap mm, const float* tables,
+                               const float* q, float* w, uint32_t nr, uint32_t nz,
+                               uint32_t shape, uint32_t cus, const FftBufs* fb, hipStream_t s);
 hipError_t launch_gemm_store(const GemmMember* mem, uint32_t nmem, const GemmState* gs,
                              MemberMap mm, const float* w, const float* y, const SurCtl* ctl,
                              uint32_t nr, uint32_t nz, double lnr, uint32_t shape, hipStream_t s);

@@ -310,3 +310,42 @@ def test_gemm_scan_members_within_error_bounds_at_configured_sizes(tmp_path):
     # longitudinally lost ones included (beam.cpp:985-994), whose phases lie
     # far out; it is stated, and bounded in the median over the members
     assert np.median([e["ez"] for _, _, e in rows]) <= 0.01
+
+
+@pytest.mark.parametrize("nr,nz", [(16, 64), (32, 128), (64, 256)])
+def test_spectral_product_forms_give_the_same_bits(nr, nz):
+    """A slot of up to four product columns takes the vector form of the
+    spectral product, of up to sixteen one matrix tile, of more tiles of 32.
+    All are the same chain of fused multiply-adds, so a beam's result does not
+    depend on how many copies of it share its aspect classes (40: a full tile
+    and a partial one)."""
+    from hpsim_amd import HPSim
+    from hpsim_amd import configs as cfg
+    wl = cfg.config(0, num=3000, periods=2)
+    elems = cfg.build_lattice(wl.lattice)
+    dist = cfg.make_distribution(wl.beam)
+    ref = None
+    for n in (1, 4, 5, 16, 17, 40):
+        sims = []
+        for _ in range(n):
+            b = HPSim.Beam(mass=wl.beam.mass, charge=wl.beam.charge, current=wl.beam.current,
+                           num=wl.beam.num)
+            b.set_distribution(*dist)
+            b.set_frequency(wl.beam.freq)
+            b.set_ref_w(wl.beam.w0)
+            sims.append(HPSim.Simulator(b, HPSim.BeamLine(elements=elems),
+                                        HPSim.SpaceCharge(nr=nr, nz=nz, interval=wl.interval)))
+        batch = HPSim.Batch(sims)
+        batch.set_field_mode("gemm")
+        batch.set_gemm_shape(8)
+        batch.simulate()
+        field = sims[0].spch.tables()[1]
+        for m in (sims[0], sims[-1]):
+            a = m.beam.arrays()
+            if ref is None:
+                ref = (a, field)
+            assert np.isfinite(a["x"]).all() and field.any()
+            for k in ref[0]:
+                assert np.array_equal(a[k].view(np.uint32), ref[0][k].view(np.uint32)), (n, k)
+            f = m.spch.tables()[1]
+            assert np.array_equal(f.view(np.uint64), ref[1].view(np.uint64)), n
