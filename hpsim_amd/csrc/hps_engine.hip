@@ -285,6 +285,7 @@ struct hps_spch {
   double* fld2 = nullptr;
   int64_t* bins = nullptr;
   size_t max_lds = 0;        // LDS bytes per workgroup on this device
+  uint32_t cus = 256;        // compute units
 };
 
 struct hps_sim {
@@ -838,6 +839,10 @@ int hps_spch_create(hps_spch** out, uint32_t nr, uint32_t nz, double interval, u
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, s->device) == hipSuccess &&
       lds > 0)
     s->max_lds = (size_t)lds;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) == hipSuccess &&
+      cus > 0)
+    s->cus = (uint32_t)cus;
   if (hipMalloc(&s->dev, sizeof(ScDev)) != hipSuccess ||
       hipMemset(s->dev, 0, sizeof(ScDev)) != hipSuccess) {
     (void)hipFree(s->dev);
@@ -1381,7 +1386,7 @@ extern "C" int hps_sim_simulate(hps_sim* m, int32_t start, int32_t end)
       case L_PHASE_FINAL: return launch_phase_final(l.ph, st);
       case L_BUILD:
         return launch_sc_build(sc->dev, sc->fld1, sc->cfg.nx, sc->cfg.nz, b->d, b->st, sc->bins,
-                               deposit_ok, st);
+                               deposit_ok, sc->cus, st);
       default: {
         FieldArgs f;
         f.sc = sc->dev; f.bins = sc->bins; f.fld1 = sc->fld1; f.fld2 = sc->fld2;
@@ -2122,18 +2127,19 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
   const std::vector<uint32_t> chunk_map = xcd_chunk_map(nchs);
   std::vector<BuildArgs> build(B);
   std::vector<FieldArgs> field(B);
+  bt->cus = m0->sc ? m0->sc->cus : 0;
   if (sc_on) {
-    const uint32_t gb = greens_blocks(nr, nz);
     for (size_t k = 0; k < B; ++k) {
       hps_sim* m = bt->sims[k];
       BuildArgs& a = build[k];
       a.sc = m->sc->dev; a.fld1 = m->sc->fld1; a.b = m->b->d; a.st = m->b->st; a.bins = m->sc->bins;
-      // the grouped field solve has no per-beam Green's table
-      a.greens_blocks = bt->field_mode == 1 ? 0 : gb;
-      // deposit-only rebuilds (grouped solve) take fuller deposit workgroups
-      a.dep_blocks = m->b->blck_size / 4 == 0 ? 0
-                     : bt->field_mode == 1 ? deposit_blocks_batch(m->b->n, nr, nz)
-                                           : deposit_blocks(m->b->n, 4);
+      // the grouped field solve has no per-beam Green's table; its
+      // deposit-only rebuilds take fuller deposit workgroups
+      build_plan(a, bt->field_mode != 1,
+                 m->b->blck_size / 4 == 0 ? 0
+                 : bt->field_mode == 1    ? deposit_blocks_batch(m->b->n, nr, nz)
+                                          : deposit_blocks(m->b->n, 4),
+                 nr, nz, bt->cus);
       const uint32_t nb = sc_build_blocks(a);
       for (uint32_t c = 0; c < nb; ++c)
         build_map.push_back(((uint32_t)k << kBatchLocalBits) | c);
@@ -2144,12 +2150,6 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
   const bool gemm = sc_on && bt->field_mode == 1;
   if (gemm) {
     if (alloc_gemm(bt, nr, nz, (uint32_t)B, s)) { restore(); return -1; }
-    if (!bt->cus) {
-      int dev = 0, n = 0;
-      HPS_CHECK(hipGetDevice(&dev));
-      HPS_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-      bt->cus = (uint32_t)n;
-    }
     std::vector<GemmMember> mem(B);
     for (size_t k = 0; k < B; ++k) {
       hps_sim* m = bt->sims[k];

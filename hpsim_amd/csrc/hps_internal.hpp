@@ -88,19 +88,19 @@ struct BuildArgs {
   BeamArrays b;
   const hps_beam_stats* st;
   int64_t* bins;
-  uint32_t greens_blocks;   // leading workgroups that fill the Green's table
-  uint32_t dep_blocks;      // deposit workgroups: after them, or the first dep_blocks
-                            // when a lone beam has dep_blocks >= greens_blocks
-                            // (0: empty deposit)
+  uint32_t greens_wgs;      // workgroups that fill the Green's table
+  uint32_t dep_blocks;      // deposit workgroups (0: empty deposit)
+  uint32_t side;            // 1: side by side, the deposit's after the table's;
+                            // 0: the first greens_wgs fill the table, then deposit
+  uint32_t pad_;
 };
 
-// Workgroups of one simulation's rebuild grid (k_sc_build): dep_blocks when
-// the deposit covers the Green's table (its first workgroups fill the table),
-// else the table workgroups followed by the deposit workgroups.  The host
-// builds the batched block map from it and the kernel splits the roles by it.
+// Workgroups of one simulation's rebuild grid (k_sc_build).  The host builds
+// the batched block map from it and the kernel splits the roles by it.
 __host__ __device__ __forceinline__ uint32_t sc_build_blocks(const BuildArgs& a)
 {
-  return a.dep_blocks >= a.greens_blocks ? a.dep_blocks : a.greens_blocks + a.dep_blocks;
+  return a.side ? a.greens_wgs + a.dep_blocks
+                : (a.greens_wgs > a.dep_blocks ? a.greens_wgs : a.dep_blocks);
 }
 
 struct FieldArgs {
@@ -136,9 +136,12 @@ uint32_t deposit_blocks_batch(uint32_t n, uint32_t nr, uint32_t nz);
 // deposit launch is empty).
 hipError_t launch_sc_build(ScDev* sc, double* fld1, uint32_t nr, uint32_t nz, BeamArrays b,
                            const hps_beam_stats* st, int64_t* bins, bool deposit,
-                           hipStream_t s);
+                           uint32_t cus, hipStream_t s);
 hipError_t launch_field(const FieldArgs& a, uint32_t nr, uint32_t nz, hipStream_t s);
-uint32_t greens_blocks(uint32_t nr, uint32_t nz);
+// roles of a rebuild's workgroups: greens, with a Green's table of its own
+void build_plan(BuildArgs& a, bool greens, uint32_t dep_blocks, uint32_t nr, uint32_t nz,
+                uint32_t cus);
+constexpr size_t kCuLds = 160 * 1024;
 
 // Batched forms: recs holds one argument record per simulation (the segment
 // and phase kernels also a block map over their chunks).

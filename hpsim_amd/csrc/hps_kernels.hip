@@ -1383,11 +1383,18 @@ __device__ __forceinline__ void greens_entry(const ScDev* sc, double* fld1, uint
                                              uint32_t nz, uint32_t r_num_part, double mass,
                                              uint32_t idx)
 {
-  const uint32_t total = (nr + 1) * nz * nr;
-  if (idx >= total) return;
-  const uint32_t k = idx % nr;            // source ring index rs
-  const uint32_t t = (idx / nr) % nz;     // dz
-  const uint32_t rpi = idx / (nr * nz);
+  uint32_t k, t, rpi;   // source ring rs, dz, field radius rp
+  if (((nr & (nr - 1)) | (nz & (nz - 1))) == 0) {
+    const uint32_t lr = 31u - __builtin_clz(nr), lz = 31u - __builtin_clz(nz);
+    k = idx & (nr - 1);
+    t = (idx >> lr) & (nz - 1);
+    rpi = idx >> (lr + lz);
+  } else {
+    const uint32_t row = idx / nr;
+    k = idx - row * nr;
+    rpi = row / nz;
+    t = row - rpi * nz;
+  }
   const double r_beta = sc->beta, r_freq = sc->freq;
   const double r_current_ov_mc2 = sc->current * sc->frac / mass;
   const double gm = 1.0 / ::sqrt(1.0 - r_beta * r_beta);
@@ -1526,6 +1533,7 @@ __device__ __forceinline__ void deposit_block(const BeamArrays& b, const hps_bea
   const DepConst d = dep_const(st, sc);
   const uint32_t nb = d.nx * d.nz;
   for (uint32_t i = t; i < nb; i += kDepositBlock) hist[i] = 0ull;
+  if (t == 0) ured[0] = 0;
   __syncthreads();
   uint32_t count = 0;
   const uint32_t stride = nblk * kDepositBlock;
@@ -1553,48 +1561,41 @@ __device__ __forceinline__ void deposit_block(const BeamArrays& b, const hps_bea
     const unsigned long long v = hist[i];
     if (v != 0ull) atomicAdd((unsigned long long*)&bins[i], v);
   }
-  ured[t] = count;
+  // on-mesh count: wave sums, one LDS add a wave
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) count += __shfl_down(count, o, 64);
+  if ((t & 63) == 0 && count) atomicAdd(ured, count);
   __syncthreads();
-  for (int o = kDepositBlock / 2; o >= 1; o >>= 1) {
-    if (t < o) ured[t] += ured[t + o];
-    __syncthreads();
-  }
   if (t == 0 && ured[0]) atomicAdd(&sc->st.num_on_mesh, ured[0]);
 }
 
 // The SCHEFF rebuild after a remesh decision, one launch of
-// sc_build_blocks(a) workgroups per simulation.  When the deposit takes at
-// least as many workgroups as the Green's table, there are dep_blocks of
-// them: the first greens_blocks fill a Green's entry per thread and all
-// then deposit (fewer, fuller workgroups than side by side: the
-// 1,048,576-particle step measured 65.1 -> 63.7 ms).  Otherwise workgroups
-// [0, greens_blocks) fill the table and the next dep_blocks deposit
-// (65,536 particles: sc_build 1.55 ms per step side by side, 1.82
-// combined).  Both roles read only the control step's results; all exit
-// when there is no remesh.
+// sc_build_blocks(a) workgroups per simulation: greens_wgs of them fill the
+// Green's table, in turns of a workgroup's threads, dep_blocks deposit; side by
+// side (the first greens_wgs, then the others) or, combined, the first
+// greens_wgs before they deposit (build_plan).  Both roles read only the
+// control step's results; all exit when there is no remesh.
 
 __device__ __forceinline__ void sc_build_body(const BuildArgs& a, uint32_t nr, uint32_t nz,
                                               uint32_t blk, unsigned long long* hist,
                                               uint32_t* ured)
 {
   if (!a.sc->remesh) return;
-  if (a.dep_blocks >= a.greens_blocks) {
-    if (blk < a.greens_blocks)
-      greens_entry(a.sc, a.fld1, nr, nz, a.b.n, a.b.mass, blk * kDepositBlock + threadIdx.x);
-    deposit_block(a.b, a.st, a.sc, a.bins, blk, a.dep_blocks, hist, ured);
-    return;
+  if (blk < a.greens_wgs) {
+    const uint32_t total = (nr + 1) * nz * nr;
+    for (uint32_t i = blk * kDepositBlock + threadIdx.x; i < total;
+         i += a.greens_wgs * kDepositBlock)
+      greens_entry(a.sc, a.fld1, nr, nz, a.b.n, a.b.mass, i);
+    if (a.side) return;
   }
-  if (blk < a.greens_blocks) {
-    greens_entry(a.sc, a.fld1, nr, nz, a.b.n, a.b.mass, blk * kDepositBlock + threadIdx.x);
-    return;
-  }
-  deposit_block(a.b, a.st, a.sc, a.bins, blk - a.greens_blocks, a.dep_blocks, hist, ured);
+  deposit_block(a.b, a.st, a.sc, a.bins, a.side ? blk - a.greens_wgs : blk, a.dep_blocks, hist,
+                ured);
 }
 
 __global__ __launch_bounds__(kDepositBlock) void k_sc_build(BuildArgs a, uint32_t nr, uint32_t nz)
 {
   extern __shared__ unsigned long long hist[];
-  __shared__ uint32_t ured[kDepositBlock];
+  __shared__ uint32_t ured[1];
   sc_build_body(a, nr, nz, blockIdx.x, hist, ured);
 }
 
@@ -1603,7 +1604,7 @@ __global__ __launch_bounds__(kDepositBlock) void k_sc_build_batch(const BuildArg
                                                                   uint32_t nr, uint32_t nz)
 {
   extern __shared__ unsigned long long hist[];
-  __shared__ uint32_t ured[kDepositBlock];
+  __shared__ uint32_t ured[1];
   const uint32_t e = map[blockIdx.x];
   const BuildArgs a = recs[e >> kBatchLocalBits];
   sc_build_body(a, nr, nz, e & kBatchLocalMask, hist, ured);
@@ -1784,7 +1785,6 @@ __device__ __forceinline__ void field_wave_body(const FieldArgs& f, uint32_t nr,
 }
 
 constexpr uint32_t kFieldMaxWaves = 9;
-constexpr size_t kCuLds = 160 * 1024;
 
 template <int K, int kDepth>
 __global__ __launch_bounds__(64 * kFieldMaxWaves) void k_field_wave(FieldArgs f, uint32_t nr,
@@ -2081,27 +2081,55 @@ uint32_t deposit_blocks_batch(uint32_t n, uint32_t nr, uint32_t nz)
   return grid;
 }
 
-uint32_t greens_blocks(uint32_t nr, uint32_t nz)
+#ifndef HPS_FAST_PUSH
+// The workgroups of one simulation's rebuild: greens (with a Green's table of
+// its own) and dep_blocks deposit workgroups.  A deposit of at least as many
+// workgroups as the table has turns is combined with it (1,048,576 particles
+// on 32 x 128, 256 and 132: 63.7 ms per 800-element step against 65.1 side by
+// side); otherwise they run side by side (65,536 particles: 64 and 132,
+// sc_build 1.55 ms per step against 1.82 combined) as long as the device
+// holds them together: two workgroups a CU, one where the histogram takes
+// more than half of its LDS.  Past that they share the room by work, a
+// particle's deposit about two table entries, and the table's workgroups take
+// several turns (300,007 particles on 64 x 256, 256 and 1,040 workgroups of
+// 132 KB LDS in six rounds: 113 us a kick point; all 256 combined 109; 96 and
+// 160: 102, 64 and 192 102, 128 and 128 106, 160 and 96 110).
+void build_plan(BuildArgs& a, bool greens, uint32_t dep_blocks, uint32_t nr, uint32_t nz,
+                uint32_t cus)
 {
-  return ((nr + 1) * nz * nr + kDepositBlock - 1) / kDepositBlock;
+  const size_t lds = (size_t)nr * nz * sizeof(unsigned long long) + kBlockLdsReserve;
+  const uint32_t room = cus * (2 * lds > kCuLds ? 1 : 2);
+  const uint32_t entries = greens ? (nr + 1) * nz * nr : 0;
+  const uint32_t turns = (entries + kDepositBlock - 1) / kDepositBlock;
+  a.dep_blocks = dep_blocks;
+  a.greens_wgs = turns;
+  a.side = dep_blocks < turns ? 1 : 0;
+  if (a.side && dep_blocks + turns > room) {
+    const double work = 2.0 * a.b.n;
+    const uint32_t share = (uint32_t)(room * (work / (work + entries)));
+    if (dep_blocks > share) a.dep_blocks = share > 0 ? share : 1;
+    const uint32_t left = room > a.dep_blocks ? room - a.dep_blocks : 1;
+    a.greens_wgs = turns < left ? turns : left;
+  }
 }
 
 hipError_t launch_sc_build(ScDev* sc, double* fld1, uint32_t nr, uint32_t nz, BeamArrays b,
                            const hps_beam_stats* st, int64_t* bins, bool deposit,
-                           hipStream_t s)
+                           uint32_t cus, hipStream_t s)
 {
   BuildArgs a;
   a.sc = sc; a.fld1 = fld1; a.b = b; a.st = st; a.bins = bins;
-  a.greens_blocks = greens_blocks(nr, nz);
   // a lone beam spreads its deposit over up to one particle per thread (65,536
   // particles: 64 workgroups, 9.9 -> 9.0 ms per 160-element step); from
   // 262,144 particles on the 256-workgroup cap holds
-  a.dep_blocks = deposit ? deposit_blocks(b.n, 1) : 0;
+  build_plan(a, true, deposit ? deposit_blocks(b.n, 1) : 0, nr, nz, cus);
   const size_t lds = (size_t)nr * nz * sizeof(unsigned long long);
   hipLaunchKernelGGL(k_sc_build, dim3(sc_build_blocks(a)), dim3(kDepositBlock), lds, s, a, nr,
                      nz);
   return hipGetLastError();
 }
+
+#endif
 
 hipError_t launch_sc_build_batch(const BuildArgs* recs, const uint32_t* map, uint32_t nblocks,
                                  uint32_t nr, uint32_t nz, hipStream_t s)

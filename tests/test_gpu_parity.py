@@ -293,6 +293,27 @@ def test_space_charge_tables_bit_exact(nr, nz):
     assert err is None, err
 
 
+@pytest.mark.parametrize("num,nr,nz", [
+    (30000, 64, 256),     # histogram over half a CU's LDS: deposit and table share the CUs
+    (12345, 48, 250),     # the same, off powers of two
+    (20000, 7, 33),       # more deposit workgroups than table turns: combined
+    (1025, 50, 100),      # two workgroups a CU, table in one turn
+])
+def test_rebuild_splits_bit_exact(num, nr, nz):
+    """Each way the rebuild's workgroups divide table and deposit."""
+    wl = H.workload(0, num=num, periods=1, sc=True)
+    wl.nr, wl.nz = nr, nz
+    ob, osc, _ = H.run_oracle(wl)
+    gb, gsc, _ = H.run_gpu(wl)
+    for name, g, o in zip(("greens", "field", "bins"), gsc.tables(), osc.tables()):
+        assert np.array_equal(g.view(np.uint64), o.view(np.uint64)), name
+    gs, os_ = gsc.state(), osc.state()
+    for k in ("remesh_count", "kick_count", "num_on_mesh"):
+        assert gs[k] == os_[k], (k, gs[k], os_[k])
+    err = H.compare_arrays(gb.arrays(), ob.arrays())
+    assert err is None, err
+
+
 @pytest.mark.parametrize("num,adj,adj_w", [(4096, 2, 0.0), (6000, 3, 1.6), (2, 2, 0.0), (5, 1, 0.0)])
 def test_adjacent_bunch_space_charge_bit_exact(num, adj, adj_w):
     """adj_bunch > 0: image rings in the Green's table, image point charges
