@@ -361,7 +361,7 @@ int hps_beam_create(hps_beam** out, uint32_t num, double mass, double charge, do
        hipMemset(b->pr.rmax2, 0, (size_t)b->pr.mpad * 8) == hipSuccess;
   ok = ok && hipHostMalloc((void**)&b->ro, sizeof(Readout), hipHostMallocDefault) == hipSuccess;
   if (!ok) { free_beam(b); delete b; return fail("device allocation failed for the beam"); }
-  b->d.n = num; b->d.mass = mass; b->d.charge = charge;
+  b->d.n = num; b->d.mass = mass; b->d.rmass = 1.0 / mass; b->d.charge = charge;
   *out = b;
   return 0;
 }
@@ -2593,6 +2593,7 @@ extern "C" int hps_emittance_noalloc(const double* x, const double* xp, const do
   a.loss = const_cast<uint32_t*>(loss); a.lloss = const_cast<uint32_t*>(lloss);
   a.n = n;
   a.mass = mass;
+  a.rmass = 1.0 / mass;
   double w0 = 0;
   HPS_CHECK(hipMemcpyAsync(&w0, w, sizeof(double), hipMemcpyDeviceToHost, s));
   // the same sums and expressions as hps_beam_get_emittance (UpdateLoss, then

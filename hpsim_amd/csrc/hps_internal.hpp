@@ -17,6 +17,7 @@ struct BeamArrays {
   uint32_t *loss, *lloss;
   uint32_t n;
   double mass, charge;
+  double rmass;            // rounded 1 / mass (div_by)
 };
 
 // Device-resident SCHEFF state: the SpaceCharge members the reference keeps
@@ -31,6 +32,7 @@ struct ScDev {
   // kick constants of ApplySpchKickKernel (space_charge_kernel.cu:578-640)
   // that the control step fixes, computed once per kick point
   double k_xbar, k_ybar, k_epsq, k_gmg, k_dr, k_dzg, k_hl, k_c1, k_c2, k_bgmg;
+  double k_repsq, k_rdr, k_rdzg, k_rbgmg;   // 1 / epsq, 1 / dr, 1 / dzg, 1 / bgmg
   double k_xfac, k_yfac, k_er_ratio, k_ez_ratio;
   double k_pl;          // bunch spacing beta*gamma*lambda (adjacent-bunch images)
   uint32_t adj_eff;     // adjacent bunches each side at this kick point

@@ -212,6 +212,7 @@ __device__ __forceinline__ bool is_good(uint32_t loss, uint32_t lloss)
 struct KickConst {
   double phimc, xbar, ybar, epsq, gmg, dr, dzg, hl, c2, c3, xfac, yfac;
   double er_ratio, ez_ratio, cbgcoef, r_beta, phi_ref, pl;
+  double repsq, rdr, rdzg;   // rounded reciprocals of epsq, dr, dzg
   uint32_t nx, nz, adj;
 };
 
@@ -240,7 +241,10 @@ __device__ __forceinline__ KickConst kick_const(const ScDev* scg, const hps_beam
   k.nz = sc->st.nz;
   k.hl = sc->k_hl;
   k.c2 = sc->k_c2;
-  k.c3 = r_length / sc->k_bgmg;
+  k.c3 = div_by(r_length, sc->k_bgmg, sc->k_rbgmg);
+  k.repsq = sc->k_repsq;
+  k.rdr = sc->k_rdr;
+  k.rdzg = sc->k_rdzg;
   k.xfac = sc->k_xfac;
   k.yfac = sc->k_yfac;
   k.er_ratio = sc->k_er_ratio;
@@ -276,6 +280,10 @@ __device__ __forceinline__ void kick_prepare(ScDev* sc, double r_beta, double r_
   sc->k_c2 = r_beta * gmg * wave_len / TWOPI;
   sc->k_pl = r_beta * gmg * wave_len;
   sc->k_bgmg = r_beta * gmg;
+  sc->k_repsq = 1.0 / epsq;
+  sc->k_rdr = 1.0 / (dr * ratio_r);
+  sc->k_rdzg = 1.0 / dzg;
+  sc->k_rbgmg = 1.0 / (r_beta * gmg);
   sc->k_xfac = xfac;
   sc->k_yfac = epsq * xfac;
   sc->k_er_ratio = ratio_q / (ratio_r * ratio_z * ratio_g * ratio_g);
@@ -283,20 +291,21 @@ __device__ __forceinline__ void kick_prepare(ScDev* sc, double r_beta, double r_
 }
 
 __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const double* tbl,
-                                     double r_mass)
+                                     double r_mass, double rmass)
 {
   const double phi = relative_phi(p.phi, k.phi_ref);   // phi_r of UpdateRelativePhi(true)
-  const double gm = p.w / r_mass + 1.0;
+  const double gm = div_by(p.w, r_mass, rmass) + 1.0;
   const double bgz = psqrt((gm - 1.0) * (gm + 1.0));
   double bgx = bgz * p.xp;
   double bgy = bgz * p.yp;
   double bgzstar = k.gmg * (bgz - k.r_beta * gm);
   const double xxbar = p.x - k.xbar;
   const double yybar = p.y - k.ybar;
-  double r = psqrt(xxbar * xxbar / k.epsq + yybar * yybar * k.epsq);
+  double r = psqrt(div_by(xxbar * xxbar, k.epsq, k.repsq) + yybar * yybar * k.epsq);
   if (r == 0.0) r = 1.0e-8;
-  const double xovr = xxbar * k.xfac / r;
-  const double yovr = yybar * k.yfac / r;
+  const double rr = recip(r);
+  const double xovr = div_by(xxbar * k.xfac, r, rr);
+  const double yovr = div_by(yybar * k.yfac, r, rr);
   double ddz = phi - k.phimc;
   for (int guard = 0; (ddz > PI || ddz < -PI) && guard < 4096; ++guard) {
     if (ddz > 0.0) ddz -= TWOPI;
@@ -307,7 +316,7 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
   if (r > k.nx * k.dr || __builtin_fabs(z) > k.hl) {
     z = -k.c2 * (phi - k.phimc);
     const double d = psqrt(z * z + r * r);
-    const double invd3 = 1.0 / (d * d * d);
+    const double invd3 = pdiv(1.0, d * d * d);
     double rod3 = r * invd3;
     double zod3 = z * invd3;
     // point charges of the neighbouring bunches (space_charge_kernel.cu:650-662)
@@ -316,7 +325,7 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
       for (int lr = 0; lr < 2; ++lr) {
         const double sz = z + xi * k.pl;
         const double dd = psqrt(sz * sz + r * r);
-        const double iv = 1.0 / (dd * dd * dd);
+        const double iv = pdiv(1.0, dd * dd * dd);
         rod3 += r * iv;
         zod3 += sz * iv;
         xi = -xi;
@@ -325,11 +334,12 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
     cbgr = k.cbgcoef * rod3;
     cbgzs = k.cbgcoef * zod3;
   } else {
-    const uint32_t i = (uint32_t)(1 + to_int(r / k.dr));
-    const double a = r / k.dr - (i - 1.0);
+    const double ri = div_by(r, k.dr, k.rdr), zj = div_by(z + k.hl, k.dzg, k.rdzg);
+    const uint32_t i = (uint32_t)(1 + to_int(ri));
+    const double a = ri - (i - 1.0);
     const double b = 1.0 - a;
-    const uint32_t j = (uint32_t)(1 + to_int((z + k.hl) / k.dzg));
-    const double c = (z + k.hl) / k.dzg - (j - 1.0);
+    const uint32_t j = (uint32_t)(1 + to_int(zj));
+    const double c = zj - (j - 1.0);
     const double d = 1.0 - c;
     const uint32_t tbl_sz = (k.nx + 1) * (k.nz + 1);
     uint32_t l = (j - 1) * (k.nx + 1) + i;
@@ -351,9 +361,10 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
   if (bgzf <= 0.0) {
     p.loss = 9999;
   } else {
-    p.xp = bgx / bgzf;
-    p.yp = bgy / bgzf;
-    p.w *= 1.0 + (gm + 1.0) * (bgzf - bgz) / (gm * bgz);
+    const double rbg = recip(bgzf);
+    p.xp = div_by(bgx, bgzf, rbg);
+    p.yp = div_by(bgy, bgzf, rbg);
+    p.w *= 1.0 + pdiv((gm + 1.0) * (bgzf - bgz), gm * bgz);
   }
 }
 
@@ -533,7 +544,7 @@ __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSm
       for (int g = 0; g < kGroup; ++g) {
         const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
         if (alive_in[g] && p[g].lloss == 0 && (i & a.kick_mask) != 0)
-          kick(p[g], k, a.fld2, b.mass);
+          kick(p[g], k, a.fld2, b.mass, b.rmass);
       }
     }
     for (int o = a.op_begin; o < a.op_end; ++o) {
@@ -541,7 +552,7 @@ __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSm
 #pragma unroll
       for (int g = 0; g < kGroup; ++g) {
         const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
-        if (p[g].loss == 0) apply_op<kClass>(op, p[g], i, b.mass, b.charge, xa, ya);
+        if (p[g].loss == 0) apply_op<kClass>(op, p[g], i, b.mass, b.rmass, b.charge, xa, ya);
       }
     }
 #pragma unroll
@@ -688,11 +699,11 @@ __device__ __forceinline__ void segment_body_live(const SegArgs& a, uint32_t c, 
       const hps_beam_stats* stp = a.st;
       asm volatile("" : "+s"(scp), "+s"(stp));
       const KickConst k = kick_const(scp, stp, a.kick_len);
-      if (p.lloss == 0 && (i & a.kick_mask) != 0) kick(p, k, a.fld2, b.mass);
+      if (p.lloss == 0 && (i & a.kick_mask) != 0) kick(p, k, a.fld2, b.mass, b.rmass);
     }
     for (int o = a.op_begin; o < a.op_end; ++o) {
       const OpConst& op = ((const OpConst*)a.ops)[o];
-      if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.charge, xa, ya);
+      if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
     }
     store_particle(b, i, p);
     if (a.stats == STAT_SC) {
@@ -816,12 +827,12 @@ __device__ __forceinline__ void segment_body_wide(const SegArgs& a, uint32_t c, 
   const bool alive_in = i < b.n && p.loss == 0;
   if (a.kick && alive_in && p.lloss == 0 && (i & a.kick_mask) != 0) {
     const KickConst k = kick_const(a.sc, a.st, a.kick_len);
-    kick(p, k, a.fld2, b.mass);
+    kick(p, k, a.fld2, b.mass, b.rmass);
   }
   const double xa = a.st->x_avg, ya = a.st->y_avg;
   for (int o = a.op_begin; o < a.op_end; ++o) {
     const OpConst& op = ((const OpConst*)a.ops)[o];
-    if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.charge, xa, ya);
+    if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
   }
   const bool in = i < b.n;
   if (alive_in) store_particle(b, i, p);
@@ -1438,6 +1449,7 @@ __device__ __forceinline__ void greens_entry(const ScDev* sc, double* fld1, uint
 struct DepConst {
   uint32_t nx, nz;
   double phimc, xbar, ybar, epsq, ref, dr, dzg, hl, c2, drdr;
+  double repsq, rdr, rdzg, rdrdr;   // reciprocals for div_by
 };
 
 __device__ __forceinline__ DepConst dep_const(const hps_beam_stats* st, const ScDev* sc)
@@ -1458,6 +1470,10 @@ __device__ __forceinline__ DepConst dep_const(const hps_beam_stats* st, const Sc
   d.hl = d.nz * 0.5 * d.dzg;
   d.c2 = r_beta * gm * wave_len / TWOPI;
   d.drdr = d.dr * d.dr;
+  d.repsq = recip(d.epsq);
+  d.rdr = recip(d.dr);
+  d.rdzg = recip(d.dzg);
+  d.rdrdr = recip(d.drdr);
   return d;
 }
 
@@ -1471,8 +1487,8 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
   const uint32_t nx = d.nx, nz = d.nz;
   const double dr = d.dr, dzg = d.dzg, drdr = d.drdr, hl = d.hl;
   double z = relative_phi(phi, d.ref);
-  const double rsq_sh = (x - d.xbar) * (x - d.xbar) / d.epsq + (y - d.ybar) * (y - d.ybar) * d.epsq;
-  const int i = to_int(psqrt(rsq_sh) / dr + 1);
+  const double rsq_sh = div_by((x - d.xbar) * (x - d.xbar), d.epsq, d.repsq) + (y - d.ybar) * (y - d.ybar) * d.epsq;
+  const int i = to_int(div_by(psqrt(rsq_sh), dr, d.rdr) + 1);
   if (i < 1 || i > (int)nx) return false;
   double ddz = z - d.phimc;
   for (int guard = 0; (ddz > PI || ddz < -PI) && guard < 4096; ++guard) {
@@ -1482,7 +1498,7 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
   z = -d.c2 * ddz;
   if (!(__builtin_fabs(z) < hl)) return false;
   const double zz = z + hl;
-  const int jm1 = to_int(zz / dzg + 1);
+  const int jm1 = to_int(div_by(zz, dzg, d.rdzg) + 1);
   int i1 = i + 1;
   if (rsq_sh < 0.5 * drdr * (double)(i * i + (i - 1) * (i - 1))) i1 = i - 1;
   if (i1 < 1) i1 = 1;
@@ -1495,14 +1511,14 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
   if (i1 == i) {
     a = 1.0;
   } else {
-    const double sqrtmp = psqrt(4.0 * rsq_sh / drdr - 1.0);
+    const double sqrtmp = psqrt(div_by(4.0 * rsq_sh, drdr, d.rdrdr) - 1.0);
     const double rminsq = 0.25 * drdr * (sqrtmp - 1.0) * (sqrtmp - 1.0);
     const double rmaxsq = rminsq + sqrtmp * drdr;
-    if (i1 < i) a = (rmaxsq - (i - 1) * (i - 1) * drdr) / (rmaxsq - rminsq);
-    else a = ((i1 - 1) * (i1 - 1) * drdr - rminsq) / (rmaxsq - rminsq);
+    if (i1 < i) a = pdiv(rmaxsq - (i - 1) * (i - 1) * drdr, rmaxsq - rminsq);
+    else a = pdiv((i1 - 1) * (i1 - 1) * drdr - rminsq, rmaxsq - rminsq);
   }
   double cc = 1.0;
-  if (j1 != jm1) cc = (zz - (j1 - 1 + 0.5) * dzg) / ((jm1 - j1) * dzg);
+  if (j1 != jm1) cc = pdiv(zz - (j1 - 1 + 0.5) * dzg, (jm1 - j1) * dzg);
   const double bb = 1.0 - a;
   const double dd = 1.0 - cc;
   if (jm1 < 1 || jm1 > (int)nz) return false;
@@ -1943,6 +1959,8 @@ __global__ void k_probe(int fn, const double* x, const double* y, double* out, u
     case 14: psincos(v, &s, &c); r = c; break;
     case 15: psinhcosh(v, &s, &c); r = s; break;
     case 16: psinhcosh(v, &s, &c); r = c; break;
+    case 17: r = pdiv(v, y[i]); break;
+    case 18: r = div_by(v, y[i], 1.0 / y[i]); break;
     default: break;
   }
   out[i] = r;

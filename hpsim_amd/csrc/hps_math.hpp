@@ -42,6 +42,60 @@ HPS_HD uint64_t bits_of(double v) { return __builtin_bit_cast(uint64_t, v); }
 HPS_HD double double_of(uint64_t u) { return __builtin_bit_cast(double, u); }
 HPS_HD double pow2i(int k) { return double_of((uint64_t)(k + 1023) << 52); }
 
+// Quotients and square roots of the per-particle maps, the kick, the deposit
+// and the Green's table.  The tracking kernels are bound by vector
+// instructions (k_segment 88 % of its waves' time), and the compiler spends
+// eleven on a quotient and twenty-one on a root, several of which only scale
+// operands near the ends of the exponent range.  These are its sequences
+// without the scaling: the reciprocal of v_rcp_f64 with two Newton steps,
+// one corrected quotient (the residual is exact), v_div_fixup for zeros,
+// infinities and NaN; the root of v_rsq_f64 with one Goldschmidt step and
+// two corrections.  Where neither operand nor result comes within 2^54 of
+// the ends of the normal range (numerators from 2^-968, denominators between
+// 2^-1000 and 2^1000, roots of 2^-960 and up) every step rounds the same, so
+// the result is the correctly rounded one.  Quotients by one denominator
+// share its reciprocal: four instructions for each further one.
+// 1,048,576 particles on 32 x 128, 800 elements: k_segment 36.7 -> 33.3 us a
+// kick point, k_sc_build 15.2 -> 14.3; 500,009 particles without space charge,
+// 400 elements: 3.13 -> 2.70 ms (with the coefficients of uconst).
+// The build of hps_push_fast.hip and host code divide as they are compiled.
+static HPS_HD double recip(double d)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HPS_FAST_PUSH)
+  double y = __builtin_amdgcn_rcp(d);
+  y = ::fma(y, ::fma(-d, y, 1.0), y);
+  return ::fma(y, ::fma(-d, y, 1.0), y);
+#else
+  return 1.0 / d;
+#endif
+}
+
+// n / d with y = recip(d), or the rounded 1 / d
+static HPS_HD double div_by(double n, double d, double y)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HPS_FAST_PUSH)
+  const double q = n * y;
+  return __builtin_amdgcn_div_fixup(::fma(::fma(-d, q, n), y, q), d, n);
+#else
+  (void)y;
+  return n / d;
+#endif
+}
+
+static HPS_HD double pdiv(double n, double d) { return div_by(n, d, recip(d)); }
+
+// A polynomial coefficient in scalar registers.  The compiler turns a Horner
+// step fma(p, z, c) into the two-operand v_fmac, whose addend must first be
+// moved into a vector register pair: two vector instructions more per step
+// (37 steps in a half quad, 15 in each sine and cosine of a gap).
+static HPS_HD double uconst(double c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(c));
+#endif
+  return c;
+}
+
 HPS_HD double exp(double x)
 {
   if (x != x) return x;
@@ -52,19 +106,19 @@ HPS_HD double exp(double x)
   r = ::fma(-kd, kLn2Lo, r);
   // Taylor coefficients 1/13! ... 1/2!, then 1, 1.
   double p = 1.6059043836821613e-10;
-  p = ::fma(p, r, 2.08767569878681e-09);
-  p = ::fma(p, r, 2.505210838544172e-08);
-  p = ::fma(p, r, 2.755731922398589e-07);
-  p = ::fma(p, r, 2.7557319223985893e-06);
-  p = ::fma(p, r, 2.48015873015873e-05);
-  p = ::fma(p, r, 0.0001984126984126984);
-  p = ::fma(p, r, 0.001388888888888889);
-  p = ::fma(p, r, 0.008333333333333333);
-  p = ::fma(p, r, 0.041666666666666664);
-  p = ::fma(p, r, 0.16666666666666666);
-  p = ::fma(p, r, 0.5);
-  p = ::fma(p, r, 1.0);
-  p = ::fma(p, r, 1.0);
+  p = ::fma(p, r, uconst(2.08767569878681e-09));
+  p = ::fma(p, r, uconst(2.505210838544172e-08));
+  p = ::fma(p, r, uconst(2.755731922398589e-07));
+  p = ::fma(p, r, uconst(2.7557319223985893e-06));
+  p = ::fma(p, r, uconst(2.48015873015873e-05));
+  p = ::fma(p, r, uconst(0.0001984126984126984));
+  p = ::fma(p, r, uconst(0.001388888888888889));
+  p = ::fma(p, r, uconst(0.008333333333333333));
+  p = ::fma(p, r, uconst(0.041666666666666664));
+  p = ::fma(p, r, uconst(0.16666666666666666));
+  p = ::fma(p, r, uconst(0.5));
+  p = ::fma(p, r, uconst(1.0));
+  p = ::fma(p, r, uconst(1.0));
   const int k = (int)kd;
   const int k1 = k / 2;
   return (p * pow2i(k1)) * pow2i(k - k1);
@@ -86,24 +140,36 @@ HPS_HD double log(double x)
   e -= 1023;
   double m = double_of((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
   if (m > kSqrt2) { m = m * 0.5; e += 1; }
-  const double s = (m - 1.0) / (m + 1.0);
+  const double s = pdiv(m - 1.0, m + 1.0);
   const double z = s * s;
   // 1/23, 1/21, ..., 1/3
   double p = 0.043478260869565216;
-  p = ::fma(p, z, 0.047619047619047616);
-  p = ::fma(p, z, 0.05263157894736842);
-  p = ::fma(p, z, 0.058823529411764705);
-  p = ::fma(p, z, 0.06666666666666667);
-  p = ::fma(p, z, 0.07692307692307693);
-  p = ::fma(p, z, 0.09090909090909091);
-  p = ::fma(p, z, 0.1111111111111111);
-  p = ::fma(p, z, 0.14285714285714285);
-  p = ::fma(p, z, 0.2);
-  p = ::fma(p, z, 0.3333333333333333);
+  p = ::fma(p, z, uconst(0.047619047619047616));
+  p = ::fma(p, z, uconst(0.05263157894736842));
+  p = ::fma(p, z, uconst(0.058823529411764705));
+  p = ::fma(p, z, uconst(0.06666666666666667));
+  p = ::fma(p, z, uconst(0.07692307692307693));
+  p = ::fma(p, z, uconst(0.09090909090909091));
+  p = ::fma(p, z, uconst(0.1111111111111111));
+  p = ::fma(p, z, uconst(0.14285714285714285));
+  p = ::fma(p, z, uconst(0.2));
+  p = ::fma(p, z, uconst(0.3333333333333333));
   const double s2 = 2.0 * s;
   const double lm = ::fma(s2 * z, p, s2);
   const double ed = (double)e;
   return ::fma(ed, kLn2Hi, ::fma(ed, kLn2Lo, lm));
+}
+
+// kd mod 4 of a whole kd: four instructions where a conversion to 64-bit
+// integers takes nine
+HPS_HD int quadrant(double kd) { return (int)::fma(-4.0, ::floor(kd * 0.25), kd); }
+
+// sine and cosine turned by q quarter turns
+HPS_HD void turn(int q, double s, double c, double* sp, double* cp)
+{
+  const uint64_t ns = (uint64_t)(q & 2) << 62, nc = (uint64_t)((q + 1) & 2) << 62;
+  *sp = double_of(bits_of(q & 1 ? c : s) ^ ns);
+  *cp = double_of(bits_of(q & 1 ? s : c) ^ nc);
 }
 
 HPS_HD void sincos(double x, double* sp, double* cp)
@@ -113,33 +179,30 @@ HPS_HD void sincos(double x, double* sp, double* cp)
   double r = ::fma(-kd, kPio2A, x);
   r = ::fma(-kd, kPio2B, r);
   r = ::fma(-kd, kPio2C, r);
-  const int q = (int)(((int64_t)kd) & 3);
+  const int q = quadrant(kd);
   const double z = r * r;
   // sin: 1/17!, -1/15!, ..., -1/3!
   double ps = 2.8114572543455206e-15;
-  ps = ::fma(ps, z, -7.647163731819816e-13);
-  ps = ::fma(ps, z, 1.6059043836821613e-10);
-  ps = ::fma(ps, z, -2.505210838544172e-08);
-  ps = ::fma(ps, z, 2.7557319223985893e-06);
-  ps = ::fma(ps, z, -0.0001984126984126984);
-  ps = ::fma(ps, z, 0.008333333333333333);
-  ps = ::fma(ps, z, -0.16666666666666666);
+  ps = ::fma(ps, z, uconst(-7.647163731819816e-13));
+  ps = ::fma(ps, z, uconst(1.6059043836821613e-10));
+  ps = ::fma(ps, z, uconst(-2.505210838544172e-08));
+  ps = ::fma(ps, z, uconst(2.7557319223985893e-06));
+  ps = ::fma(ps, z, uconst(-0.0001984126984126984));
+  ps = ::fma(ps, z, uconst(0.008333333333333333));
+  ps = ::fma(ps, z, uconst(-0.16666666666666666));
   const double s = ::fma(r * z, ps, r);
   // cos: -1/18!, 1/16!, ..., -1/2!
   double pc = -1.5619206968586225e-16;
-  pc = ::fma(pc, z, 4.779477332387385e-14);
-  pc = ::fma(pc, z, -1.1470745597729725e-11);
-  pc = ::fma(pc, z, 2.08767569878681e-09);
-  pc = ::fma(pc, z, -2.755731922398589e-07);
-  pc = ::fma(pc, z, 2.48015873015873e-05);
-  pc = ::fma(pc, z, -0.001388888888888889);
-  pc = ::fma(pc, z, 0.041666666666666664);
-  pc = ::fma(pc, z, -0.5);
+  pc = ::fma(pc, z, uconst(4.779477332387385e-14));
+  pc = ::fma(pc, z, uconst(-1.1470745597729725e-11));
+  pc = ::fma(pc, z, uconst(2.08767569878681e-09));
+  pc = ::fma(pc, z, uconst(-2.755731922398589e-07));
+  pc = ::fma(pc, z, uconst(2.48015873015873e-05));
+  pc = ::fma(pc, z, uconst(-0.001388888888888889));
+  pc = ::fma(pc, z, uconst(0.041666666666666664));
+  pc = ::fma(pc, z, uconst(-0.5));
   const double c = ::fma(z, pc, 1.0);
-  if (q == 0) { *sp = s; *cp = c; }
-  else if (q == 1) { *sp = c; *cp = -s; }
-  else if (q == 2) { *sp = -s; *cp = -c; }
-  else { *sp = -c; *cp = s; }
+  turn(q, s, c, sp, cp);
 }
 
 HPS_HD double sinh(double x)
@@ -148,15 +211,15 @@ HPS_HD double sinh(double x)
   if (ax < 1.0) {
     const double z = x * x;
     double p = 1.9572941063391263e-20;   // 1/21!
-    p = ::fma(p, z, 8.22063524662433e-18);
-    p = ::fma(p, z, 2.8114572543455206e-15);
-    p = ::fma(p, z, 7.647163731819816e-13);
-    p = ::fma(p, z, 1.6059043836821613e-10);
-    p = ::fma(p, z, 2.505210838544172e-08);
-    p = ::fma(p, z, 2.7557319223985893e-06);
-    p = ::fma(p, z, 0.0001984126984126984);
-    p = ::fma(p, z, 0.008333333333333333);
-    p = ::fma(p, z, 0.16666666666666666);
+    p = ::fma(p, z, uconst(8.22063524662433e-18));
+    p = ::fma(p, z, uconst(2.8114572543455206e-15));
+    p = ::fma(p, z, uconst(7.647163731819816e-13));
+    p = ::fma(p, z, uconst(1.6059043836821613e-10));
+    p = ::fma(p, z, uconst(2.505210838544172e-08));
+    p = ::fma(p, z, uconst(2.7557319223985893e-06));
+    p = ::fma(p, z, uconst(0.0001984126984126984));
+    p = ::fma(p, z, uconst(0.008333333333333333));
+    p = ::fma(p, z, uconst(0.16666666666666666));
     return ::fma(x * z, p, x);
   }
   const double e = hps::exp(ax);
@@ -170,15 +233,15 @@ HPS_HD double cosh(double x)
   if (ax < 1.0) {
     const double z = x * x;
     double p = 4.110317623312165e-19;    // 1/20!
-    p = ::fma(p, z, 1.5619206968586225e-16);
-    p = ::fma(p, z, 4.779477332387385e-14);
-    p = ::fma(p, z, 1.1470745597729725e-11);
-    p = ::fma(p, z, 2.08767569878681e-09);
-    p = ::fma(p, z, 2.755731922398589e-07);
-    p = ::fma(p, z, 2.48015873015873e-05);
-    p = ::fma(p, z, 0.001388888888888889);
-    p = ::fma(p, z, 0.041666666666666664);
-    p = ::fma(p, z, 0.5);
+    p = ::fma(p, z, uconst(1.5619206968586225e-16));
+    p = ::fma(p, z, uconst(4.779477332387385e-14));
+    p = ::fma(p, z, uconst(1.1470745597729725e-11));
+    p = ::fma(p, z, uconst(2.08767569878681e-09));
+    p = ::fma(p, z, uconst(2.755731922398589e-07));
+    p = ::fma(p, z, uconst(2.48015873015873e-05));
+    p = ::fma(p, z, uconst(0.001388888888888889));
+    p = ::fma(p, z, uconst(0.041666666666666664));
+    p = ::fma(p, z, uconst(0.5));
     return ::fma(z, p, 1.0);
   }
   const double e = hps::exp(ax);
@@ -238,29 +301,26 @@ __device__ __forceinline__ void sincos_short(double x, double* sp, double* cp)
   double r = ::fma(-kd, kPio2A, x);
   r = ::fma(-kd, kPio2B, r);
   r = ::fma(-kd, kPio2C, r);
-  const int q = (int)(((int64_t)kd) & 3);
+  const int q = quadrant(kd);
   const double z = r * r;
   // sin: 1/13!, -1/11!, ..., -1/3!
   double ps = 1.6059043836821613e-10;
-  ps = ::fma(ps, z, -2.505210838544172e-08);
-  ps = ::fma(ps, z, 2.7557319223985893e-06);
-  ps = ::fma(ps, z, -0.0001984126984126984);
-  ps = ::fma(ps, z, 0.008333333333333333);
-  ps = ::fma(ps, z, -0.16666666666666666);
+  ps = ::fma(ps, z, uconst(-2.505210838544172e-08));
+  ps = ::fma(ps, z, uconst(2.7557319223985893e-06));
+  ps = ::fma(ps, z, uconst(-0.0001984126984126984));
+  ps = ::fma(ps, z, uconst(0.008333333333333333));
+  ps = ::fma(ps, z, uconst(-0.16666666666666666));
   const double s = ::fma(r * z, ps, r);
   // cos: 1/14!, -1/12!, ..., -1/2!
   double pc = -1.1470745597729725e-11;
-  pc = ::fma(pc, z, 2.08767569878681e-09);
-  pc = ::fma(pc, z, -2.755731922398589e-07);
-  pc = ::fma(pc, z, 2.48015873015873e-05);
-  pc = ::fma(pc, z, -0.001388888888888889);
-  pc = ::fma(pc, z, 0.041666666666666664);
-  pc = ::fma(pc, z, -0.5);
+  pc = ::fma(pc, z, uconst(2.08767569878681e-09));
+  pc = ::fma(pc, z, uconst(-2.755731922398589e-07));
+  pc = ::fma(pc, z, uconst(2.48015873015873e-05));
+  pc = ::fma(pc, z, uconst(-0.001388888888888889));
+  pc = ::fma(pc, z, uconst(0.041666666666666664));
+  pc = ::fma(pc, z, uconst(-0.5));
   const double c = ::fma(z, pc, 1.0);
-  if (q == 0) { *sp = s; *cp = c; }
-  else if (q == 1) { *sp = c; *cp = -s; }
-  else if (q == 2) { *sp = -s; *cp = -c; }
-  else { *sp = -c; *cp = s; }
+  turn(q, s, c, sp, cp);
 }
 
 // sinhcosh with the Taylor series for |x| < 1 cut at x^15 (sinh) and x^16
@@ -272,21 +332,21 @@ __device__ __forceinline__ void sinhcosh_short(double x, double* shp, double* ch
   if (ax < 1.0) {
     const double z = x * x;
     double p = 7.647163731819816e-13;    // 1/15!
-    p = ::fma(p, z, 1.6059043836821613e-10);
-    p = ::fma(p, z, 2.505210838544172e-08);
-    p = ::fma(p, z, 2.7557319223985893e-06);
-    p = ::fma(p, z, 0.0001984126984126984);
-    p = ::fma(p, z, 0.008333333333333333);
-    p = ::fma(p, z, 0.16666666666666666);
+    p = ::fma(p, z, uconst(1.6059043836821613e-10));
+    p = ::fma(p, z, uconst(2.505210838544172e-08));
+    p = ::fma(p, z, uconst(2.7557319223985893e-06));
+    p = ::fma(p, z, uconst(0.0001984126984126984));
+    p = ::fma(p, z, uconst(0.008333333333333333));
+    p = ::fma(p, z, uconst(0.16666666666666666));
     *shp = ::fma(x * z, p, x);
     double c = 4.779477332387385e-14;     // 1/16!
-    c = ::fma(c, z, 1.1470745597729725e-11);
-    c = ::fma(c, z, 2.08767569878681e-09);
-    c = ::fma(c, z, 2.755731922398589e-07);
-    c = ::fma(c, z, 2.48015873015873e-05);
-    c = ::fma(c, z, 0.001388888888888889);
-    c = ::fma(c, z, 0.041666666666666664);
-    c = ::fma(c, z, 0.5);
+    c = ::fma(c, z, uconst(1.1470745597729725e-11));
+    c = ::fma(c, z, uconst(2.08767569878681e-09));
+    c = ::fma(c, z, uconst(2.755731922398589e-07));
+    c = ::fma(c, z, uconst(2.48015873015873e-05));
+    c = ::fma(c, z, uconst(0.001388888888888889));
+    c = ::fma(c, z, uconst(0.041666666666666664));
+    c = ::fma(c, z, uconst(0.5));
     *chp = ::fma(z, c, 1.0);
     return;
   }
@@ -313,8 +373,8 @@ static __device__ __forceinline__ void psinhcosh(double x, double* shp, double* 
 #endif
 }
 
-// The square root of the per-particle maps, the kick and the deposit: the
-// correctly rounded ::sqrt, or sqrt_rsq in the build of hps_push_fast.hip,
+// The square root of the per-particle maps, the kick and the deposit (see
+// recip above), or sqrt_rsq in the build of hps_push_fast.hip,
 // which serves batches whose results are held to error bounds, not to the
 // oracle's bits.  Internal to each translation unit, so the two builds keep
 // their own.
@@ -323,7 +383,14 @@ static __device__ __forceinline__ double psqrt(double x)
 #ifdef HPS_FAST_PUSH
   return sqrt_rsq(x);
 #else
-  return ::sqrt(x);
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = ::fma(-h, g, 0.5);
+  g = ::fma(g, r, g);
+  h = ::fma(h, r, h);
+  g = ::fma(::fma(-g, g, x), h, g);
+  g = ::fma(::fma(-g, g, x), h, g);
+  return (x == 0.0 || x == kInf) ? x : g;
 #endif
 }
 

@@ -47,6 +47,28 @@ def test_device_division_is_ieee():
     assert np.array_equal(g.view(np.uint64), (x / y).view(np.uint64))
 
 
+@pytest.mark.parametrize("fn,span", [("pdiv", 20), ("div_by", 20), ("pdiv", 140), ("div_by", 140),
+                                     ("psqrt", 280)])
+def test_unscaled_quotients_and_roots_are_ieee(fn, span):
+    """The maps' quotients and roots without exponent scaling: correctly
+    rounded over 10^-span .. 10^span, and the IEEE results for zeros of
+    either sign, infinities and NaN."""
+    from hpsim_amd import HPSim
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal(400000) * 10.0 ** rng.uniform(-span, span, 400000)
+    y = rng.standard_normal(400000) * 10.0 ** rng.uniform(-span, span, 400000)
+    sp = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1.0, -1.0, 3.0, 938.272])
+    x = np.concatenate([x, np.repeat(sp, sp.size)])
+    y = np.concatenate([y, np.tile(sp, sp.size)])
+    if fn == "psqrt":
+        x = np.concatenate([np.abs(x), sp])
+    with np.errstate(all="ignore"):
+        ref = np.sqrt(x) if fn == "psqrt" else x / y
+    g = HPSim.probe_math(fn, x, None if fn == "psqrt" else y)
+    same = (g.view(np.uint64) == ref.view(np.uint64)) | (np.isnan(g) & np.isnan(ref))
+    assert same.all(), (fn, x[~same][:4], g[~same][:4], ref[~same][:4])
+
+
 @pytest.mark.parametrize("num,periods", [(1000, 3), (4096, 4)])
 def test_tracking_no_space_charge_bit_exact(num, periods):
     wl = H.workload(0, num=num, periods=periods, sc=False)
