@@ -87,11 +87,13 @@ static HPS_HD double pdiv(double n, double d) { return div_by(n, d, recip(d)); }
 // A polynomial coefficient in scalar registers.  The compiler turns a Horner
 // step fma(p, z, c) into the two-operand v_fmac, whose addend must first be
 // moved into a vector register pair: two vector instructions more per step
-// (37 steps in a half quad, 15 in each sine and cosine of a gap).
+// (37 steps in a half quad, 15 in each sine and cosine of a gap).  The empty
+// asm is not volatile: a volatile one keeps the compiler from merging blocks,
+// and the build of hps_push_fast.hip then shares other reciprocals.
 static HPS_HD double uconst(double c)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+s"(c));
+  asm("" : "+s"(c));
 #endif
   return c;
 }
