@@ -2128,6 +2128,8 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
   std::vector<BuildArgs> build(B);
   std::vector<FieldArgs> field(B);
   bt->cus = m0->sc ? m0->sc->cus : 0;
+  uint64_t total = 0;
+  for (size_t k = 0; k < B; ++k) total += bt->sims[k]->b->n;
   if (sc_on) {
     for (size_t k = 0; k < B; ++k) {
       hps_sim* m = bt->sims[k];
@@ -2137,7 +2139,7 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
       // deposit-only rebuilds take fuller deposit workgroups
       build_plan(a, bt->field_mode != 1,
                  m->b->blck_size / 4 == 0 ? 0
-                 : bt->field_mode == 1    ? deposit_blocks_batch(m->b->n, nr, nz)
+                 : bt->field_mode == 1    ? deposit_blocks_batch(m->b->n, total, nr, nz, bt->cus)
                                           : deposit_blocks(m->b->n, 4),
                  nr, nz, bt->cus);
       const uint32_t nb = sc_build_blocks(a);

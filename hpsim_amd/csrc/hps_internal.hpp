@@ -133,7 +133,8 @@ constexpr size_t kBlockLdsReserve = 4 * kDepositBlock;
 // deposit workgroups for n particles, per_thread particles per thread (at most
 // kDepositMaxBlocks workgroups)
 uint32_t deposit_blocks(uint32_t n, uint32_t per_thread);
-uint32_t deposit_blocks_batch(uint32_t n, uint32_t nr, uint32_t nz);
+// the same for one of a batch's members; total: particles of all of them
+uint32_t deposit_blocks_batch(uint32_t n, uint64_t total, uint32_t nr, uint32_t nz, uint32_t cus);
 // Green's table + charge deposit (deposit = false for beams whose reference
 // deposit launch is empty).
 hipError_t launch_sc_build(ScDev* sc, double* fld1, uint32_t nr, uint32_t nz, BeamArrays b,

@@ -2087,12 +2087,17 @@ uint32_t deposit_blocks(uint32_t n, uint32_t per_thread)
 // histogram over more particles: 64 members of 4,194,304 particles on the
 // 64 x 256 mesh, deposit per 160-element step 360 / 294 / 261 / 241 / 233 /
 // 227 ms at 1,024 / 512 / 256 / 128 / 64 / 32 workgroups per member; the
-// 256-beam scan on 32 x 128 takes 84 ms at 128 and 91 ms at 32.
-uint32_t deposit_blocks_batch(uint32_t n, uint32_t nr, uint32_t nz)
+// 256-beam scan on 32 x 128 takes 84 ms at 128 and 91 ms at 32.  A batch of
+// few members fills the device instead, each with its share, by particles, of
+// the workgroups that run at once (four members of 2,097,152 particles on
+// 64 x 256: 32 workgroups each, half of the CUs, 120 us a rebuild; 64 each
+// 77 us.  Seven members of 16,384 to 1,048,576 on 32 x 128: 24.1 -> 20.8).
+uint32_t deposit_blocks_batch(uint32_t n, uint64_t total, uint32_t nr, uint32_t nz, uint32_t cus)
 {
-  const uint32_t cap = (size_t)nr * nz * sizeof(unsigned long long) > 65536
-                           ? kDepositMaxBlocksBig
-                           : kDepositMaxBlocksBatch;
+  const bool big = (size_t)nr * nz * sizeof(unsigned long long) > 65536;
+  const uint32_t share = (uint32_t)((uint64_t)cus * (big ? 1 : 2) * n / total);
+  uint32_t cap = big ? kDepositMaxBlocksBig : kDepositMaxBlocksBatch;
+  if (cap < share) cap = share;
   uint32_t grid = (n + 4 * kDepositBlock - 1) / (4 * kDepositBlock);
   if (grid < 1) grid = 1;
   if (grid > cap) grid = cap;

@@ -349,3 +349,37 @@ def test_spectral_product_forms_give_the_same_bits(nr, nz):
                 assert np.array_equal(a[k].view(np.uint32), ref[0][k].view(np.uint32)), (n, k)
             f = m.spch.tables()[1]
             assert np.array_equal(f.view(np.uint64), ref[1].view(np.uint64)), n
+
+
+@pytest.mark.parametrize("nr,nz,num", [(64, 256, 140001), (32, 128, 600000)])
+def test_deposit_shares_give_the_same_bits(nr, nz, num):
+    """A member's deposit workgroups follow its share of the batch's particles
+    (35 in a batch of two and 32 in one of nine on 64 x 256; 147 and 128 on
+    32 x 128): its charges, counts and coordinates do not depend on it."""
+    from hpsim_amd import HPSim
+    wl = cfg.config(0, num=num, periods=1)
+    elems = cfg.build_lattice(wl.lattice)
+    dist = cfg.make_distribution(wl.beam)
+    ref = None
+    for n in (2, 9):
+        sims = []
+        for _ in range(n):
+            b = HPSim.Beam(mass=wl.beam.mass, charge=wl.beam.charge, current=wl.beam.current,
+                           num=wl.beam.num)
+            b.set_distribution(*dist)
+            b.set_frequency(wl.beam.freq)
+            b.set_ref_w(wl.beam.w0)
+            sims.append(HPSim.Simulator(b, HPSim.BeamLine(elements=elems),
+                                        HPSim.SpaceCharge(nr=nr, nz=nz, interval=wl.interval)))
+        batch = HPSim.Batch(sims)
+        batch.set_field_mode("gemm")
+        batch.set_gemm_shape(8)
+        batch.simulate()
+        a, bins = sims[-1].beam.arrays(), sims[-1].spch.tables()[2]
+        on = sims[-1].spch.state()["num_on_mesh"]
+        if ref is None:
+            ref = (a, bins, on)
+        assert on == ref[2] > 0
+        assert np.array_equal(bins, ref[1])
+        for k in ref[0]:
+            assert np.array_equal(a[k].view(np.uint32), ref[0][k].view(np.uint32)), (n, k)
