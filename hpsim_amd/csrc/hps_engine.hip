@@ -51,8 +51,8 @@ uint32_t next_pow2(uint32_t x)   // utility.cpp:7-16
 
 hipStream_t g_stream[16];
 
-// Largest read-back that goes through a beam's pinned staging block (18,724
-// particles; freed with the beam).
+// Largest read-back that goes through a pinned staging block (18,724
+// particles).
 constexpr size_t kStageBytes = 1 << 20;
 
 }  // namespace
@@ -91,17 +91,72 @@ struct hps_beam {
   Partials pr{};
   double* snap[2][6] = {{nullptr}};
   uint32_t* snap_l[2][2] = {{nullptr}};
-  Readout* ro = nullptr;            // pinned: the getters' sums and the statistics
-  uint8_t* stage = nullptr;         // pinned: read-back of a small beam (kStageBytes at most)
+  Readout ro{};                     // the getters' sums and the statistics, last read
   bool saved[2] = {false, false};
   double snap_dw[2] = {0, 0}, snap_f[2] = {0, 0}, snap_c[2] = {0, 0};
 };
 
 namespace {
 
+// A pinned block for one call that reads back: the getters' sums and a small
+// beam's arrays.  Blocks are shared by all beams, devices and threads; a call
+// holds one until it has waited for its stream, and kPinnedKeep are kept free
+// for the next (4 MB; more are given back at once).  One of its own per beam
+// cost 50 us to make and 500 us to free with the beam.
+struct Pinned {
+  Readout ro;
+  uint8_t stage[kStageBytes];
+};
+constexpr size_t kPinnedKeep = 4;
+std::mutex g_pinned_mu;
+std::vector<Pinned*> g_pinned_free;
+
+class PinnedLease {
+ public:
+  PinnedLease()
+  {
+    {
+      std::lock_guard<std::mutex> lock(g_pinned_mu);
+      if (!g_pinned_free.empty()) {
+        p_ = g_pinned_free.back();
+        g_pinned_free.pop_back();
+        return;
+      }
+    }
+    if (hipHostMalloc((void**)&p_, sizeof(Pinned), hipHostMallocPortable) != hipSuccess)
+      p_ = nullptr;
+  }
+  PinnedLease(const PinnedLease&) = delete;
+  PinnedLease& operator=(const PinnedLease&) = delete;
+  // a call that failed before it waited may have left kernels writing here:
+  // freeing waits for them
+  ~PinnedLease()
+  {
+    if (p_ && waited_) {
+      std::lock_guard<std::mutex> lock(g_pinned_mu);
+      if (g_pinned_free.size() < kPinnedKeep) {
+        g_pinned_free.push_back(p_);
+        return;
+      }
+    }
+    if (p_) (void)hipHostFree(p_);
+  }
+  Pinned* get() const { return p_; }
+  hipError_t wait(hipStream_t s)
+  {
+    const hipError_t e = hipStreamSynchronize(s);
+    waited_ = e == hipSuccess;
+    return e;
+  }
+
+ private:
+  Pinned* p_ = nullptr;
+  bool waited_ = false;
+};
+
 // What a getter reads: the canonical-order sums of up to kReadSlots
 // variable pairs (k_sums), the loss counts, the statistics and the reference
-// particle's energy.  The kernels write them into the beam's pinned block, so
+// particle's energy.  The kernels write them into a pinned block, so
 // a getter waits for the device once; the statistics go back as the argument
 // of a one-wave kernel.  (With every value copied by itself a getter waited
 // three to eight times: twenty getters of a 1,048,576-particle beam 3.3 ms.)
@@ -113,12 +168,16 @@ struct Pair {
 
 int read_sums(hps_beam* b, const Pair* p, int n, hps_beam_stats* s)
 {
+  PinnedLease pin;
+  if (!pin.get()) return fail("pinned host allocation failed");
+  Readout* const ro = &pin.get()->ro;
   for (int k = 0; k < n; ++k) {
     HPS_CHECK(launch_sums(b->d, p[k].a, p[k].bb, p[k].filter, b->pr, b->stream, p[k].rel_ref,
-                          &b->ro->sums[k], s && k == n - 1 ? b->ro : nullptr, b->st));
+                          &ro->sums[k], s && k == n - 1 ? ro : nullptr, b->st));
   }
-  HPS_CHECK(hipStreamSynchronize(b->stream));
-  if (s) *s = b->ro->st;
+  HPS_CHECK(pin.wait(b->stream));
+  b->ro = *ro;
+  if (s) *s = ro->st;
   return 0;
 }
 
@@ -159,14 +218,14 @@ int update_longitudinal_loss(hps_beam* b, hps_beam_stats& s, bool all)
 {
   const Pair phi{b->d.phi, nullptr, 1, nullptr}, counts{nullptr, nullptr, 2, nullptr};
   if (read_sums(b, &phi, 1, &s)) return -1;
-  if (all) s.num_loss = b->ro->sums[0].nloss;
-  s.num_good = b->ro->sums[0].ngood;
-  s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+  if (all) s.num_loss = b->ro.sums[0].nloss;
+  s.num_good = b->ro.sums[0].ngood;
+  s.phi_avg_good = avg_of(b, s, b->ro.sums[0], true);
   if (push(b, s)) return -1;
   HPS_CHECK(launch_lloss_flag(b->d, &b->st->phi_avg_good, b->stream));
   if (read_sums(b, &counts, 1, nullptr)) return -1;
-  s.num_lloss = b->ro->sums[0].nlloss;
-  if (all) s.num_good = b->ro->sums[0].ngood;
+  s.num_lloss = b->ro.sums[0].nlloss;
+  if (all) s.num_good = b->ro.sums[0].ngood;
   return 0;
 }
 
@@ -176,8 +235,8 @@ int init_phi_avg_good(hps_beam* b)
   hps_beam_stats s;
   const Pair phi{b->d.phi, nullptr, 0, nullptr};
   if (read_sums(b, &phi, 1, &s)) return -1;
-  s.num_loss = b->ro->sums[0].nloss;
-  s.phi_avg = avg_of(b, s, b->ro->sums[0], false);
+  s.num_loss = b->ro.sums[0].nloss;
+  s.phi_avg = avg_of(b, s, b->ro.sums[0], false);
   s.phi_avg_good = s.phi_avg;
   return push(b, s);
 }
@@ -192,8 +251,8 @@ int change_frequency(hps_beam* b, double f)
   hps_beam_stats s;
   const Pair p[2] = {{b->d.phi, nullptr, 0, nullptr}, {b->d.phi, nullptr, 0, b->d.phi}};
   if (read_sums(b, p, 2, &s)) return -1;
-  s.phi_avg = avg_of(b, s, b->ro->sums[0], false);
-  s.phi_avg_r = avg_of(b, s, b->ro->sums[1], false);
+  s.phi_avg = avg_of(b, s, b->ro.sums[0], false);
+  s.phi_avg_r = avg_of(b, s, b->ro.sums[1], false);
   return push(b, s);
 }
 
@@ -205,11 +264,11 @@ int emittance(hps_beam* b, hps_beam_stats& s)
                      {b->d.phi, b->d.w, 0, b->d.phi}};   // relative to particle 0
   const bool upd = b->n > 2;
   if (read_sums(b, p, upd ? 3 : 1, &s)) return -1;
-  s.num_loss = b->ro->sums[0].nloss;
+  s.num_loss = b->ro.sums[0].nloss;
   if (!upd) return 0;
-  const double w0 = b->ro->w0;
+  const double w0 = b->ro.w0;
   for (int axis = 0; axis < 2; ++axis) {   // beam.cu:1007-1064, beam_kernel.cu:1333-1354
-    const BeamSums& r = b->ro->sums[axis];
+    const BeamSums& r = b->ro.sums[axis];
     const double sv = surv(b, s);
     const double x = r.s[0] / sv, x2 = r.s[1] / sv, xp = r.s[2] / sv, xp2 = r.s[3] / sv,
                  xxp = r.s[4] / sv;
@@ -221,7 +280,7 @@ int emittance(hps_beam* b, hps_beam_stats& s)
     if (axis == 0) { s.x_avg = x; s.x_sig = sig; s.xp_avg = xp; s.xp_sig = sigp; s.x_emit = emit; }
     else { s.y_avg = x; s.y_sig = sig; s.yp_avg = xp; s.yp_sig = sigp; s.y_emit = emit; }
   }
-  const BeamSums& r = b->ro->sums[2];   // beam.cu:1069-1092, beam_kernel.cu:1356-1373
+  const BeamSums& r = b->ro.sums[2];   // beam.cu:1069-1092, beam_kernel.cu:1356-1373
   const double sv = surv(b, s);
   const double phi = r.s[0] / sv, phi2 = r.s[1] / sv, w = r.s[2] / sv, w2 = r.s[3] / sv,
                phi_w = r.s[4] / sv;
@@ -257,8 +316,6 @@ void free_beam(hps_beam* b)
   (void)hipFree(b->pr.cnt);
   (void)hipFree(b->pr.pmax);
   (void)hipFree(b->pr.rmax2);
-  (void)hipHostFree(b->ro);
-  (void)hipHostFree(b->stage);
   for (int k = 0; k < 2; ++k) {
     for (int j = 0; j < 6; ++j) (void)hipFree(b->snap[k][j]);
     (void)hipFree(b->snap_l[k][0]);
@@ -359,7 +416,6 @@ int hps_beam_create(hps_beam** out, uint32_t num, double mass, double charge, do
        hipMemset(b->pr.pmax, 0, (size_t)b->pr.mpad * 8) == hipSuccess;
   ok = ok && hipMalloc(&b->pr.rmax2, (size_t)b->pr.mpad * 8) == hipSuccess &&
        hipMemset(b->pr.rmax2, 0, (size_t)b->pr.mpad * 8) == hipSuccess;
-  ok = ok && hipHostMalloc((void**)&b->ro, sizeof(Readout), hipHostMallocDefault) == hipSuccess;
   if (!ok) { free_beam(b); delete b; return fail("device allocation failed for the beam"); }
   b->d.n = num; b->d.mass = mass; b->d.rmass = 1.0 / mass; b->d.charge = charge;
   *out = b;
@@ -524,15 +580,15 @@ int hps_beam_download(hps_beam* b, double* x, double* xp, double* y, double* yp,
   if (6 * nd + 2 * nu <= kStageBytes) {
     // a small beam: one kernel writes the arrays into pinned memory, one wait
     // (eight copies of 16 KB, each with its own wait: 160 us; so 25)
-    if (!b->stage)
-      HPS_CHECK(hipHostMalloc((void**)&b->stage, 6 * nd + 2 * nu, hipHostMallocDefault));
+    PinnedLease pin;
+    if (!pin.get()) return fail("pinned host allocation failed");
     BeamArrays dst = b->d;
-    uint8_t* at = b->stage;
+    uint8_t* at = pin.get()->stage;
     double** dd[6] = {&dst.x, &dst.xp, &dst.y, &dst.yp, &dst.phi, &dst.w};
     for (double** d : dd) { *d = (double*)at; at += nd; }
     dst.loss = (uint32_t*)at; dst.lloss = (uint32_t*)(at + nu);
     HPS_CHECK(launch_copy_beam(b->d, dst, b->stream));
-    HPS_CHECK(hipStreamSynchronize(b->stream));
+    HPS_CHECK(pin.wait(b->stream));
     for (int k = 0; k < 6; ++k)
       if (out[k]) std::memcpy(out[k], *dd[k], nd);
     if (loss) std::memcpy(loss, dst.loss, nu);
@@ -595,7 +651,7 @@ int hps_beam_get_scalar(hps_beam* b, int which, double* out)
       hps_beam_stats s;
       const Pair counts{nullptr, nullptr, 2, nullptr};
       if (read_sums(b, &counts, 1, &s)) return -1;
-      s.num_loss = b->ro->sums[0].nloss;
+      s.num_loss = b->ro.sums[0].nloss;
       if (push(b, s)) return -1;
       v = b->current * (1.0 - ((double)s.num_loss) / ((double)b->n));
       break;
@@ -613,7 +669,7 @@ int hps_beam_get_loss_num(hps_beam* b, int which, uint32_t* out)   // wrap_beam.
   if (which == 0) {
     const Pair counts{nullptr, nullptr, 2, nullptr};
     if (read_sums(b, &counts, 1, &s)) return -1;
-    s.num_loss = b->ro->sums[0].nloss;
+    s.num_loss = b->ro.sums[0].nloss;
     *out = s.num_loss;
   } else {
     if (update_longitudinal_loss(b, s, which != 1)) return -1;
@@ -631,7 +687,7 @@ int hps_beam_get_avg(hps_beam* b, int var, int good, double* out)   // wrap_beam
   const Pair p{rel ? b->d.phi : arr[var], nullptr, good ? 1 : 0, rel ? b->d.phi : nullptr};
   hps_beam_stats s;
   if (read_sums(b, &p, 1, &s)) return -1;
-  const BeamSums& r = b->ro->sums[0];
+  const BeamSums& r = b->ro.sums[0];
   s.num_loss = r.nloss;                             // UpdateLoss
   if (var == 2 && good) s.num_good = r.ngood;       // UpdateGoodParticleCount
   double* const at[4][2] = {{&s.x_avg, &s.x_avg_good}, {&s.y_avg, &s.y_avg_good},
@@ -652,7 +708,7 @@ int hps_beam_get_sig(hps_beam* b, int var, int good, double* out)   // wrap_beam
   const Pair p{rel ? b->d.phi : arr[var], nullptr, good && !rel ? 1 : 0, rel ? b->d.phi : nullptr};
   hps_beam_stats s;
   if (read_sums(b, &p, 1, &s)) return -1;
-  s.num_loss = b->ro->sums[0].nloss;
+  s.num_loss = b->ro.sums[0].nloss;
   if (b->n < 2) { *out = 0.0; return push(b, s); }
   const bool upd = b->n > 2;
   double* const at[4][2] = {{&s.x_sig, &s.x_sig_good}, {&s.y_sig, &s.y_sig_good},
@@ -660,13 +716,13 @@ int hps_beam_get_sig(hps_beam* b, int var, int good, double* out)   // wrap_beam
   double* const v = rel ? &s.phi_sig_r : at[var][good ? 1 : 0];
   if (phi_good) {
     // about the good particles' mean phase: a second pass against it
-    s.num_good = b->ro->sums[0].ngood;
-    s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+    s.num_good = b->ro.sums[0].ngood;
+    s.phi_avg_good = avg_of(b, s, b->ro.sums[0], true);
     if (push(b, s)) return -1;
     const Pair q{b->d.phi, nullptr, 1, &b->st->phi_avg_good};
     if (upd && read_sums(b, &q, 1, nullptr)) return -1;
   }
-  if (upd) *v = sig_of(b, s, b->ro->sums[0], good && !rel);
+  if (upd) *v = sig_of(b, s, b->ro.sums[0], good && !rel);
   *out = *v;
   return push(b, s);
 }
@@ -711,7 +767,7 @@ int hps_beam_restore(hps_beam* b, int slot)   // beam.cpp:606-647
   hps_beam_stats s;
   const Pair phi{b->d.phi, nullptr, 1, nullptr};
   if (read_sums(b, &phi, 1, &s)) return -1;
-  s.phi_avg_good = avg_of(b, s, b->ro->sums[0], true);
+  s.phi_avg_good = avg_of(b, s, b->ro.sums[0], true);
   return push(b, s);
 }
 
