@@ -220,7 +220,7 @@ __global__ __launch_bounds__(64 * kMaxFrag) void k_conv(ConvArgs a)
 }
 
 // dw[co][t][ci] += sum over positions of dpre[p][co] * in[src(p, t)][ci]:
-// one wave per (tap, 16 co, 16 ci, chunk of 256 positions); FP32 atomics.
+// one workgroup per (tap, 16 co, 16 ci, chunk of 256 positions); FP32 atomics.
 __global__ __launch_bounds__(64 * kWaves) void k_wgrad(WgradArgs a)
 {
   const int lane = threadIdx.x & 63;
@@ -228,10 +228,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_wgrad(WgradArgs a)
   const int P = a.B * a.Zout;
   const int nco = a.Cout / 16, nci = a.Cin / 16;
   const int nchunk = cdiv(P, kWgradChunk);
-  const int task = blockIdx.x * kWaves + wave;
-  if (task >= a.taps * nco * nci * nchunk) return;
-  const int chunk = task % nchunk;
-  int r = task / nchunk;
+  const int chunk = blockIdx.x % nchunk;
+  int r = blockIdx.x / nchunk;
   const int cit = r % nci; r /= nci;
   const int cot = r % nco;
   const int t = r / nco;
@@ -239,11 +237,15 @@ __global__ __launch_bounds__(64 * kWaves) void k_wgrad(WgradArgs a)
   const int kq = 4 * (lane >> 4);
   const int co = cot * 16 + (lane & 15), ci = cit * 16 + (lane & 15);
   const int pend = min(P, (chunk + 1) * kWgradChunk);
-  // kAhead steps of 16 positions are loaded before the first is used: with
-  // one at a time a task was 16 dependent memory round trips (23 us a layer
-  // at 64 samples)
+  // A task is one workgroup: its waves take 64 positions each, whose loads
+  // are all issued before the first is used, and meet in LDS, so a weight gets
+  // one atomic add per task.  (A wave per task left most SIMDs with one wave
+  // or none, whose memory round trips nothing hid: 19.3 us a layer at 64
+  // samples, so 9.2.)
   constexpr int kAhead = 4;
-  for (int q0 = chunk * kWgradChunk; q0 < pend; q0 += 16 * kAhead) {
+  static_assert(16 * kAhead * kWaves == kWgradChunk, "one step per wave");
+  const int q0 = chunk * kWgradChunk + wave * 16 * kAhead;
+  if (q0 < pend) {
     float dv[kAhead][4], xv[kAhead][4];
 #pragma unroll
     for (int h = 0; h < kAhead; ++h) {
@@ -278,12 +280,18 @@ __global__ __launch_bounds__(64 * kWaves) void k_wgrad(WgradArgs a)
       acc = mfma(da, xl, acc);
     }
   }
-  // D[m = co][n = ci]: this lane holds ci = cit*16 + lane%16, co rows 4(lane/16)+i
+  // D[m = co][n = ci]: a lane holds ci = cit*16 + lane%16, co rows 4(lane/16)+i;
+  // thread 64 i + lane adds element i of its lane over the waves
+  __shared__ float part[kWaves][4][64];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int cor = cot * 16 + 4 * (lane >> 4) + i;
-    atomicAdd(&a.dw[((size_t)cor * a.taps + t) * a.Cin + ci], acc[i]);
-  }
+  for (int i = 0; i < 4; ++i) part[wave][i][lane] = acc[i];
+  __syncthreads();
+  static_assert(kWaves == 4, "a wave per element of the accumulator");
+  float v = part[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) v += part[w][wave][lane];
+  const int cor = cot * 16 + 4 * (lane >> 4) + wave;
+  atomicAdd(&a.dw[((size_t)cor * a.taps + t) * a.Cin + ci], v);
 }
 
 // Bounded conditioning v = 2 tanh(u / 2) (the FiLM polynomial stays within
@@ -469,7 +477,7 @@ hipError_t conv(const ConvArgs& a, hipStream_t s)
 hipError_t wgrad(const WgradArgs& a, hipStream_t s)
 {
   const int tasks = a.taps * (a.Cout / 16) * (a.Cin / 16) * cdiv(a.B * a.Zout, kWgradChunk);
-  hipLaunchKernelGGL(k_wgrad, dim3(cdiv(tasks, kWaves)), dim3(64 * kWaves), 0, s, a);
+  hipLaunchKernelGGL(k_wgrad, dim3(tasks), dim3(64 * kWaves), 0, s, a);
   return hipGetLastError();
 }
 
