@@ -78,7 +78,7 @@ struct NetImpl {
   // training / evaluation buffers for max_b samples
   int max_b = 0;
   std::vector<float*> pre, out, dy;
-  float *scale = nullptr, *dpre = nullptr, *xb = nullptr, *tb = nullptr, *ub = nullptr;
+  float *scale = nullptr, *dpre = nullptr, *fpart = nullptr, *xb = nullptr, *tb = nullptr, *ub = nullptr;
   float *lossb = nullptr, *hist = nullptr;
   uint32_t* idx = nullptr;
   size_t idx_cap = 0;
@@ -136,7 +136,7 @@ void free_bufs(std::vector<float*>& v)
 
 void free_net(NetImpl* n)
 {
-  for (float* p : {n->w, n->g, n->m, n->v, n->scale, n->dpre, n->xb, n->tb, n->ub, n->lossb,
+  for (float* p : {n->w, n->g, n->m, n->v, n->scale, n->dpre, n->fpart, n->xb, n->tb, n->ub, n->lossb,
                    n->hist, n->iscale, n->data.x, n->data.y, n->data.u})
     (void)hipFree(p);
   (void)hipFree(n->wt); (void)hipFree(n->wb); (void)hipFree(n->idx); (void)hipFree(n->d_film);
@@ -188,12 +188,15 @@ int upload_film(NetImpl* n, int B, unet::FilmLayer* dst, int* held)
 {
   if (*held == B) return 0;
   std::vector<unet::FilmLayer> fl(n->layers.size());
-  size_t soff = 0;
+  size_t soff = 0, poff = 0;
   for (size_t k = 0; k < n->layers.size(); ++k) {
     fl[k].cout = n->layers[k].cout;
     fl[k].a_off = n->layers[k].a_off;
     fl[k].s_off = soff * B;
+    fl[k].slabs = unet::film_slabs(n->layers[k].zout);
+    fl[k].p_off = poff;
     soff += n->layers[k].cout;
+    poff += (size_t)B * fl[k].slabs * n->layers[k].cout;
   }
   NN_CHECK(hipMemcpyAsync(dst, fl.data(), fl.size() * sizeof(unet::FilmLayer),
                           hipMemcpyHostToDevice, n->s));
@@ -206,10 +209,11 @@ int alloc_train(NetImpl* n, int B)
 {
   if (B <= n->max_b) return 0;
   free_bufs(n->pre); free_bufs(n->out); free_bufs(n->dy);
-  for (float* p : {n->scale, n->dpre, n->xb, n->tb, n->ub, n->lossb}) (void)hipFree(p);
+  for (float* p : {n->scale, n->dpre, n->fpart, n->xb, n->tb, n->ub, n->lossb}) (void)hipFree(p);
   n->max_b = B;
-  size_t big = 0;
+  size_t big = 0, film = 0;
   for (const Layer& l : n->layers) {
+    film += (size_t)B * unet::film_slabs(l.zout) * l.cout;
     float *a = nullptr, *b = nullptr, *c = nullptr;
     NN_CHECK(hipMalloc(&a, act_size(l, B) * 4));
     NN_CHECK(hipMalloc(&b, act_size(l, B) * 4));
@@ -219,6 +223,7 @@ int alloc_train(NetImpl* n, int B)
   }
   NN_CHECK(hipMalloc(&n->scale, n->scale_per_sample * B * 4));
   NN_CHECK(hipMalloc(&n->dpre, big * 4));
+  NN_CHECK(hipMalloc(&n->fpart, film * 4));
   NN_CHECK(hipMalloc(&n->xb, (size_t)B * n->Z0 * n->cin * 4));
   NN_CHECK(hipMemset(n->xb, 0, (size_t)B * n->Z0 * n->cin * 4));
   NN_CHECK(hipMalloc(&n->tb, (size_t)B * n->zn * n->cout * 4));
@@ -245,12 +250,14 @@ int loss_grad(NetImpl* n, int B, bool grad)
   std::vector<int> skip_to(L, -1);
   for (size_t k = 0; k < L; ++k)
     if (n->layers[k].skip >= 0) skip_to[n->layers[k].skip] = (int)k;
-  size_t soff = n->scale_per_sample;
+  size_t soff = n->scale_per_sample, poff = 0;
+  for (const Layer& l : n->layers) poff += (size_t)B * unet::film_slabs(l.zout) * l.cout;
   for (size_t kk = L; kk-- > 0;) {
     const Layer& l = n->layers[kk];
     soff -= l.cout;
-    NN_CHECK(unet::film_bwd(n->dy[kk], n->pre[kk], n->scale + soff * B, n->ub, n->dpre,
-                            n->g + l.a_off, B, l.zout, l.cout, s));
+    poff -= (size_t)B * unet::film_slabs(l.zout) * l.cout;
+    NN_CHECK(unet::film_bwd(n->dy[kk], n->pre[kk], n->scale + soff * B, n->dpre, n->fpart + poff,
+                            B, l.zout, l.cout, s));
     const float* in = kk == 0 ? n->xb : n->out[kk - 1];
     unet::WgradArgs wa{n->dpre, in, n->g + l.w_off, B, l.zin, l.zout, l.cin, l.cout, l.taps,
                        l.dil, l.mode};
@@ -271,6 +278,7 @@ int loss_grad(NetImpl* n, int B, bool grad)
                                                                                    : unet::kPoint));
     NN_CHECK(unet::conv(a, s));
   }
+  NN_CHECK(unet::film_sum(n->d_film, (int)L, n->fpart, n->ub, n->g, B, s));
   return 0;
 }
 

@@ -315,18 +315,18 @@ __global__ void k_film(const float* __restrict__ params, const FilmLayer* __rest
   }
 }
 
-// dpre = dy * scale; g[b][co] = sum_z dy * pre -> dA[co][j] += g v_b^j.
+// dpre = dy * scale; part[b][slab][co] = sum over the slab's z of dy * pre.
 // Workgroup (b, slab of z): C / 4 threads take four channels each, the others
 // further rows of the slab; the rows' sums meet in LDS.  (One thread per
-// (b, co) over all z left the chip idle: 25 us a layer at 64 samples.)
-constexpr int kFilmSlab = 34;   // rows of a slab
-
+// (b, co) over all z left the chip idle: 25 us a layer at 64 samples.)  The
+// slabs' sums are stored and added up by one k_film_sum for all layers: added
+// atomically, three values a channel, they met in the few cache lines of a
+// layer's coefficients (12.5 us a layer at 64 samples, so 3.6).
 __global__ __launch_bounds__(256) void k_film_bwd(const float* __restrict__ dy,
                                                   const float* __restrict__ pre,
                                                   const float* __restrict__ scale,
-                                                  const float* __restrict__ u,
                                                   float* __restrict__ dpre,
-                                                  float* __restrict__ dA, int Z, int C)
+                                                  float* __restrict__ part, int Z, int C)
 {
   __shared__ float4 red[256];
   const int b = blockIdx.x, C4 = C / 4, ng = 256 / C4;
@@ -350,11 +350,42 @@ __global__ __launch_bounds__(256) void k_film_bwd(const float* __restrict__ dy,
     float t = 0.f;
     for (int k = 0; k < ng; ++k)
       t += reinterpret_cast<const float*>(red)[4 * k * C4 + threadIdx.x];
-    const float x = film_v(u[b]);
-    float* a = dA + (size_t)threadIdx.x * 3;
-    atomicAdd(a, t * x);
-    atomicAdd(a + 1, t * x * x);
-    atomicAdd(a + 2, t * x * x * x);
+    part[((size_t)b * gridDim.y + blockIdx.y) * C + threadIdx.x] = t;
+  }
+}
+
+// dA[co][j] += sum over samples and slabs of part[b][slab][co] v_b^j, every
+// layer: workgroup (16 channels, layer), a thread a channel of every sixteenth
+// sample, the sixteen sums of a channel met in LDS.
+__global__ __launch_bounds__(256) void k_film_sum(const FilmLayer* __restrict__ layers,
+                                                  const float* __restrict__ part,
+                                                  const float* __restrict__ u, float* __restrict__ g,
+                                                  int B)
+{
+  __shared__ float red[3][256];
+  const FilmLayer L = layers[blockIdx.y];
+  const int co = blockIdx.x * 16 + (threadIdx.x & 15);
+  float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+  if (co < L.cout) {
+    const float* p = part + L.p_off + co;
+    for (int b = threadIdx.x >> 4; b < B; b += 16) {
+      float t = 0.f;
+      for (int k = 0; k < L.slabs; ++k) t += p[((size_t)b * L.slabs + k) * L.cout];
+      const float x = film_v(u[b]);
+      a0 += t * x;
+      a1 += t * x * x;
+      a2 += t * x * x * x;
+    }
+  }
+  red[0][threadIdx.x] = a0;
+  red[1][threadIdx.x] = a1;
+  red[2][threadIdx.x] = a2;
+  __syncthreads();
+  const int j = threadIdx.x >> 4;
+  if (j < 3 && co < L.cout) {
+    float v = 0.f;
+    for (int k = 0; k < 16; ++k) v += red[j][16 * k + (threadIdx.x & 15)];
+    g[L.a_off + (size_t)co * 3 + j] += v;
   }
 }
 
@@ -489,11 +520,19 @@ hipError_t film(const float* params, const FilmLayer* layers, int nlayers, const
   return hipGetLastError();
 }
 
-hipError_t film_bwd(const float* dy, const float* pre, const float* scale, const float* u,
-                    float* dpre, float* dA, int B, int Z, int C, hipStream_t s)
+hipError_t film_bwd(const float* dy, const float* pre, const float* scale, float* dpre,
+                    float* part, int B, int Z, int C, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_film_bwd, dim3(B, cdiv(Z, kFilmSlab)), dim3(256), 0, s, dy, pre, scale, u,
-                     dpre, dA, Z, C);
+  hipLaunchKernelGGL(k_film_bwd, dim3(B, film_slabs(Z)), dim3(256), 0, s, dy, pre, scale, dpre,
+                     part, Z, C);
+  return hipGetLastError();
+}
+
+hipError_t film_sum(const FilmLayer* layers, int nlayers, const float* part, const float* u,
+                    float* g, int B, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_film_sum, dim3(cdiv(kMaxCout, 16), nlayers), dim3(256), 0, s, layers, part,
+                     u, g, B);
   return hipGetLastError();
 }
 

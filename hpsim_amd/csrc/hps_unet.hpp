@@ -38,11 +38,16 @@ struct WgradArgs {
   int B, Zin, Zout, Cin, Cout, taps, dil, mode;
 };
 
+// rows of z in one slab of the FiLM gradient, and the slabs of Z rows
+constexpr int kFilmSlab = 34;
+inline int film_slabs(int Z) { return (Z + kFilmSlab - 1) / kFilmSlab; }
+
 struct FilmLayer {
   int cout;
-  int pad_;
+  int slabs;                // film_slabs of its rows
   size_t a_off;             // FiLM coefficients A[cout][3] in the parameters
   size_t s_off;             // this layer's scales [max_b][cout] in the scale buffer
+  size_t p_off;             // and its FiLM gradient sums [max_b][slabs][cout]
 };
 
 // one layer's weights in the flat parameter vector
@@ -64,8 +69,13 @@ hipError_t conv(const ConvArgs& a, hipStream_t s);
 hipError_t wgrad(const WgradArgs& a, hipStream_t s);
 hipError_t film(const float* params, const FilmLayer* layers, int nlayers, const float* u,
                 const uint32_t* dyn_b, int B, float* scale, hipStream_t s);
-hipError_t film_bwd(const float* dy, const float* pre, const float* scale, const float* u,
-                    float* dpre, float* dA, int B, int Z, int C, hipStream_t s);
+// part: [B][film_slabs(Z)][C], for film_sum
+hipError_t film_bwd(const float* dy, const float* pre, const float* scale, float* dpre,
+                    float* part, int B, int Z, int C, hipStream_t s);
+// the FiLM coefficients' gradients of all layers into g (the parameters'
+// gradient) from the layers' part arrays at part + p_off
+hipError_t film_sum(const FilmLayer* layers, int nlayers, const float* part, const float* u,
+                    float* g, int B, hipStream_t s);
 // per-sample relative squared error of y against tgt * inv_scale; dy the
 // gradient of its mean (optional)
 hipError_t loss(const float* y, const float* tgt, float* dy, float* l, int Z0, int Cpad, int zn,
