@@ -241,7 +241,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_wgrad(WgradArgs a)
   // are all issued before the first is used, and meet in LDS, so a weight gets
   // one atomic add per task.  (A wave per task left most SIMDs with one wave
   // or none, whose memory round trips nothing hid: 19.3 us a layer at 64
-  // samples, so 9.2.)
+  // samples, so 9.2; with eight waves and 512 positions 9.9.)
   constexpr int kAhead = 4;
   static_assert(16 * kAhead * kWaves == kWgradChunk, "one step per wave");
   const int q0 = chunk * kWgradChunk + wave * 16 * kAhead;
@@ -391,15 +391,19 @@ __global__ __launch_bounds__(256) void k_film_sum(const FilmLayer* __restrict__ 
 
 // loss_b = |y - t / out_scale|^2 / |t / out_scale|^2 over z < zn, c < cout
 // (y [B][Z0][Cpad], t [B][zn][cout]); dy (optional) = d loss_mean / d y
-__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const float* __restrict__ tgt,
-                                              float* __restrict__ dy, float* __restrict__ loss,
-                                              int Z0, int Cpad, int zn, int cout, float inv_scale,
-                                              int B)
+// A workgroup per sample, as wide as it goes: the passes over its rows are
+// dependent loads and divisions (64 samples of 129 x 66: 256 threads 25 us,
+// 1,024 threads 11).
+constexpr int kLossBlock = 1024;
+
+__global__ __launch_bounds__(kLossBlock) void k_loss(
+    const float* __restrict__ y, const float* __restrict__ tgt, float* __restrict__ dy,
+    float* __restrict__ loss, int Z0, int Cpad, int zn, int cout, float inv_scale, int B)
 {
-  __shared__ float red[2][256];
+  __shared__ float red[2][kLossBlock];
   const int b = blockIdx.x, t = threadIdx.x;
   float nt = 0.f, nd = 0.f;
-  for (int e = t; e < zn * cout; e += 256) {
+  for (int e = t; e < zn * cout; e += kLossBlock) {
     const int z = e / cout, c = e % cout;
     const float tv = tgt[((size_t)b * zn + z) * cout + c] * inv_scale;
     const float d = y[((size_t)b * Z0 + z) * Cpad + c] - tv;
@@ -409,7 +413,7 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const
   red[0][t] = nt;
   red[1][t] = nd;
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
+  for (int o = kLossBlock / 2; o > 0; o >>= 1) {
     if (t < o) { red[0][t] += red[0][t + o]; red[1][t] += red[1][t + o]; }
     __syncthreads();
   }
@@ -417,7 +421,7 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const
   if (t == 0) loss[b] = red[1][0] / ntot;
   if (!dy) return;
   const float k = 2.f / (ntot * (float)B);
-  for (int e = t; e < Z0 * Cpad; e += 256) {
+  for (int e = t; e < Z0 * Cpad; e += kLossBlock) {
     const int z = e / Cpad, c = e % Cpad;
     float v = 0.f;
     if (z < zn && c < cout)
@@ -539,7 +543,7 @@ hipError_t film_sum(const FilmLayer* layers, int nlayers, const float* part, con
 hipError_t loss(const float* y, const float* tgt, float* dy, float* l, int Z0, int Cpad, int zn,
                 int cout, float inv_scale, int B, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_loss, dim3(B), dim3(256), 0, s, y, tgt, dy, l, Z0, Cpad, zn, cout,
+  hipLaunchKernelGGL(k_loss, dim3(B), dim3(kLossBlock), 0, s, y, tgt, dy, l, Z0, Cpad, zn, cout,
                      inv_scale, B);
   return hipGetLastError();
 }
