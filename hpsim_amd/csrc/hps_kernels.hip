@@ -51,6 +51,15 @@ __device__ __forceinline__ void gst(T* p, size_t i, T v)
   ((__attribute__((address_space(1))) T*)p)[i] = v;
 }
 
+// A barrier for what the workgroup exchanges through LDS: __syncthreads also
+// waits for the wave's outstanding global stores.
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // --- canonical reductions -------------------------------------------------
 
 // Canonical halving tree over the 256 lane values of Q sums (levels 128 and
@@ -1240,7 +1249,10 @@ __global__ __launch_bounds__(kBlock) void k_phase_wave_batch(const PhaseArgs* re
 // control logic of space_charge.cpp:84-138 (mesh_size_cutoff_w = 0) on the
 // device, and the cleared charge histogram
 // when it decides to remesh.  Thread 0 reads every input into registers
-// before it writes any output.
+// before it writes any output.  What bounds it is one chain of memory round
+// trips and divisions: the decision goes to the other waves through LDS alone,
+// so they clear the histogram while thread 0 works on, and wait for none of its
+// stores (1,048,576 particles on 32 x 128: 6.2 -> 5.6 us).
 constexpr uint32_t kPhaseFinalBlock = 512;
 
 __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
@@ -1295,34 +1307,51 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
       r2max = r2max < r2 ? r2 : r2max;
     }
   }
+  // thread 0 decides; then the other waves clear the histogram while it works
+  // out and stores the rest
+  double avg_r = 0.0, gamma = 0.0, beta = 0.0, sigz = 0.0, sigr = 0.0;
+  int rm = 0;
   if (t == 0) {
     if (a.do_sums) {
       const double gd = (double)good_cnt;
       const double avg = s[1] / gd, avg2 = s[2] / gd;
       phi_sig_good = ::sqrt(avg2 - avg * avg);
-      st->phi_avg_r = s[0] / (double)(uint32_t)(b.n - num_loss);
-      st->phi_sig_good = phi_sig_good;
+      avg_r = s[0] / (double)(uint32_t)(b.n - num_loss);
     }
     const double sigphi = b.n < 2 ? 0.0 : phi_sig_good;
     const double sigx = b.n < 2 ? 0.0 : x_sig_good;
     const double sigy = b.n < 2 ? 0.0 : y_sig_good;
-    const double gamma = (double)ke / b.mass + 1.0;
-    const double beta = ::sqrt(1.0 - 1.0 / (gamma * gamma));
+    gamma = (double)ke / b.mass + 1.0;
+    beta = ::sqrt(1.0 - 1.0 / (gamma * gamma));
     const double lmbd = 299.792458 / a.freq;
-    const double sigz = sigphi * 0.5 / 3.14159265 * beta * lmbd;
-    const double sigr = ::sqrt(sigx * sigx + sigy * sigy);
+    sigz = sigphi * 0.5 / 3.14159265 * beta * lmbd;
+    sigr = ::sqrt(sigx * sigx + sigy * sigy);
     const double cratior = sigr * sigz;
     const double cratioz = sigz * sigz * gamma * gamma;
     const double cratior_old = ss.sigr_old * ss.sigz_old;
     const double cratioz_old = ss.sigz_old * ss.sigz_old * ss.gm_old * ss.gm_old;
+    rm = cratior_old == 0.0 || cratioz_old == 0.0 ||
+         __builtin_fabs(cratior - cratior_old) / cratior_old > ss.remesh_val ||
+         __builtin_fabs(cratioz - cratioz_old) / cratioz_old > ss.remesh_val;
+    remesh = rm;
+    nbins = ss.nx * ss.nz;
+  }
+  lds_barrier();
+  if (wave != 0) {
+    if (remesh)
+      for (uint32_t i = t - 64; i < nbins; i += kPhaseFinalBlock - 64) gst(a.bins, i, (int64_t)0);
+    return;
+  }
+  if (t == 0) {
+    if (a.do_sums) {
+      st->phi_avg_r = avg_r;
+      st->phi_sig_good = phi_sig_good;
+    }
     // adjacent bunches below the cutoff energy only (space_charge.cpp:102-105)
     const uint32_t adj = (ss.adj_bunch_w == 0.0 || ke < ss.adj_bunch_w) ? ss.adj_bunch : 0u;
     double ratio_r = 1.0, ratio_z = 1.0, ratio_q = 1.0, ratio_g = 1.0;
-    int rm = 0;
     ss.kick_count += 1;
-    if (cratior_old == 0.0 || cratioz_old == 0.0 ||
-        __builtin_fabs(cratior - cratior_old) / cratior_old > ss.remesh_val ||
-        __builtin_fabs(cratioz - cratioz_old) / cratioz_old > ss.remesh_val) {
+    if (rm) {
       ss.sigr_old = sigr;
       ss.sigz_old = sigz;
       ss.gm_old = gamma;
@@ -1345,7 +1374,6 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
       // shared Green's tables in (gm as the Green's table computes it)
       sc->log_aspect = log_aspect(ss.dr, ss.dz, 1.0 / ::sqrt(1.0 - beta * beta));
       ss.num_on_mesh = 0;
-      rm = 1;
     } else {
       ratio_r = sigr / ss.sigr_old;
       ratio_z = sigz / ss.sigz_old;
@@ -1368,12 +1396,7 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
     kick_prepare(sc, beta, a.freq, a.current * a.frac, x_avg_good, y_avg_good, x_sig_good,
                  y_sig_good, ss.dr, ss.dz, ss.nz, ratio_r, ratio_z, ratio_q, ratio_g, b.n,
                  b.mass);
-    remesh = rm;
-    nbins = ss.nx * ss.nz;
   }
-  __syncthreads();
-  if (remesh)
-    for (uint32_t i = t; i < nbins; i += kPhaseFinalBlock) gst(a.bins, i, (int64_t)0);
 }
 
 __global__ __launch_bounds__(kPhaseFinalBlock) void k_phase_final(PhaseArgs a) { phase_final_body(a); }
