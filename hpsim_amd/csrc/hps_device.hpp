@@ -27,6 +27,7 @@ constexpr int kDepositShift = 36;                // fixed-point deposit: 2^-36
 struct Particle {
   double x, xp, y, yp, phi, w;
   uint32_t loss, lloss;
+  uint32_t mark;   // the maps' marks of its values (Quick, hps_math.hpp)
 };
 
 enum OpKind : int32_t {
@@ -182,6 +183,39 @@ struct Op {
   GapUniform gu;          // GAP1 / GAP2 element constants (gap_uniform)
 };
 
+// Whether the constants of a map are in Quick's range.
+inline bool op_usual(const Op& o, double charge)
+{
+  const auto numerators = [](const double* v, size_t n) {
+    for (size_t k = 0; k < n; ++k)
+      if (!zero_or_in_range(v[k])) return false;
+    return true;
+  };
+  switch (o.kind) {
+    case OP_DRIFT: return numerators(o.a, 1) && in_range(o.a[2]);
+    case OP_QUAD: return numerators(o.a, 1) && numerators(o.a + 2, 1) &&
+                         in_range(o.a[3]) && in_range(charge);
+    case OP_STEER: return numerators(o.a, 2) && in_range(charge);
+    case OP_GAP1:
+    case OP_GAP2: {
+      const GapUniform& u = o.gu;
+      const hps_gap_param& g = o.g;
+      const double fit[] = {g.fit_t0, g.fit_t1, g.fit_t2, g.fit_t3, g.fit_t4, g.fit_t5,
+                            g.fit_s1, g.fit_s2, g.fit_s3, g.fit_s4, g.fit_s5, g.fit_beta_min};
+      const double first[] = {u.twopi_dd1, u.twopi_half_q1, u.pi_dcl1, u.betag1};
+      const double second[] = {u.twopi_dd2, u.betag_ccl, u.concomm, u.concomm1, u.con2nex,
+                               u.inv_fkis, u.fkr, u.bgw, u.twopi_dg, u.q_efl, u.efl_inv_mass,
+                               u.twopi_half_q2, u.pi_dcl2, u.two_con1, u.inv_gmgcl};
+      if (!in_range(u.wave_len) || !numerators(fit, sizeof fit / 8)) return false;
+      if (o.kind == OP_GAP1) return in_range(u.beta_in1) && numerators(first, sizeof first / 8);
+      return in_range(u.beta_in2) && in_range(u.beta_out) && in_range(u.gmg) &&
+             in_range(u.inv_mass) && in_range(g.fit_beta_center) && in_range(o.a[5]) &&
+             numerators(second, sizeof second / 8);
+    }
+    default: return true;
+  }
+}
+
 // An op read through the constant address space: the op table does not
 // change while a kernel runs, so its fields (uniform across the workgroup)
 // load with scalar loads into SGPRs instead of vector loads into VGPRs,
@@ -196,13 +230,13 @@ __device__ __forceinline__ double bessi0c(double r_x)
   double ans, y;
   const double ax = __builtin_fabs(r_x);
   if (ax < 3.75) {
-    y = pdiv(r_x, 3.75);
+    y = r_x / 3.75;
     y = y * y;
     ans = 1.0 + y * (3.5156229 + y * (3.0899424 + y * (1.2067492 + y * (0.2659732 +
           y * (0.360768e-1 + y * 0.45813e-2)))));
   } else {
-    y = pdiv(3.75, ax);
-    ans = (hps::exp(ax) * pdiv(1.0, psqrt(ax))) * (0.39894228 + y * (0.1328592e-1 +
+    y = 3.75 / ax;
+    ans = (hps::exp(ax) * (1.0 / psqrt(ax))) * (0.39894228 + y * (0.1328592e-1 +
           y * (0.225319e-2 + y * (-0.157565e-2 + y * (0.916281e-2 + y * (-0.2057706e-1 +
           y * (0.2635537e-1 + y * (-0.1647633e-1 + y * 0.392377e-2))))))));
   }
@@ -215,16 +249,16 @@ __device__ __forceinline__ double bessi1c(double r_x)
   double y, ans;
   const double ax = __builtin_fabs(r_x);
   if (ax < 3.75) {
-    y = pdiv(r_x, 3.75);
+    y = r_x / 3.75;
     y = y * y;
     ans = ax * (0.5 + y * (0.87890594 + y * (0.51498869 + y * (0.15084934 + y * (0.2658733e-1 +
           y * (0.301532e-2 + y * 0.32411e-3))))));
   } else {
-    y = pdiv(3.75, ax);
+    y = 3.75 / ax;
     ans = 0.2282967e-1 + y * (-0.2895312e-1 + y * (0.1787654e-1 - y * 0.420059e-2));
     ans = 0.39894228 + y * (-0.3988024e-1 + y * (-0.362018e-2 + y * (0.163801e-2 + y *
           (-0.1031555e-1 + y * ans))));
-    ans = ans * (hps::exp(ax) * pdiv(1.0, psqrt(ax)));
+    ans = ans * (hps::exp(ax) * (1.0 / psqrt(ax)));
   }
   return r_x < 0.0 ? -ans : ans;
 }
@@ -232,25 +266,26 @@ __device__ __forceinline__ double bessi1c(double r_x)
 // Bessi1p, simulation_kernel.cu:66-73
 __device__ __forceinline__ double bessi1p(double r_x)
 {
-  if (r_x != 0.0) return bessi0c(r_x) - pdiv(bessi1c(r_x), r_x);
+  if (r_x != 0.0) return bessi0c(r_x) - bessi1c(r_x) / r_x;
   return 0.5;
 }
 
 // bessi0c(x), bessi1c(x) and bessi1p(x) of one argument, sharing the
 // common factors (identical results to the three separate calls).
+template <class A>
 __device__ __forceinline__ void bessel_all(double r_x, double& b0, double& b1, double& b1p)
 {
   const double ax = __builtin_fabs(r_x);
   if (ax < 3.75) {
-    double y = pdiv(r_x, 3.75);
+    double y = A::div(r_x, 3.75);
     y = y * y;
     b0 = 1.0 + y * (3.5156229 + y * (3.0899424 + y * (1.2067492 + y * (0.2659732 +
          y * (0.360768e-1 + y * 0.45813e-2)))));
     b1 = ax * (0.5 + y * (0.87890594 + y * (0.51498869 + y * (0.15084934 + y * (0.2658733e-1 +
          y * (0.301532e-2 + y * 0.32411e-3))))));
   } else {
-    const double y = pdiv(3.75, ax);
-    const double f = hps::exp(ax) * pdiv(1.0, psqrt(ax));
+    const double y = A::div(3.75, ax);
+    const double f = hps::exp(ax) * A::div(1.0, A::sqrt(ax));
     b0 = f * (0.39894228 + y * (0.1328592e-1 + y * (0.225319e-2 + y * (-0.157565e-2 +
          y * (0.916281e-2 + y * (-0.2057706e-1 + y * (0.2635537e-1 + y * (-0.1647633e-1 +
          y * 0.392377e-2))))))));
@@ -260,11 +295,11 @@ __device__ __forceinline__ void bessel_all(double r_x, double& b0, double& b1, d
     b1 = a1 * f;
   }
   if (r_x < 0.0) b1 = -b1;
-  b1p = r_x != 0.0 ? b0 - pdiv(b1, r_x) : 0.5;
+  b1p = r_x != 0.0 ? b0 - A::div(b1, r_x) : 0.5;
 }
 
 // GetTransitTimeFactors, simulation_kernel.cu:290-308
-template <class G>
+template <class A, class G>
 __device__ __forceinline__ void ttf(double r_beta, const G& g, double& t, double& tp, double& sp)
 {
   double beta = r_beta;
@@ -272,7 +307,7 @@ __device__ __forceinline__ void ttf(double r_beta, const G& g, double& t, double
   else if (r_beta < g.fit_beta_min) beta = g.fit_beta_min;
   t = g.fit_t0 + beta * (g.fit_t1 + beta * (g.fit_t2 + beta * (g.fit_t3 + beta *
       (g.fit_t4 + beta * g.fit_t5))));
-  const double coef = pdiv(beta * beta, TWOPI * g.fit_beta_center);
+  const double coef = A::div(beta * beta, TWOPI * g.fit_beta_center);
   tp = coef * (g.fit_t1 + beta * (2 * g.fit_t2 + beta * (3 * g.fit_t3 + beta *
        (4 * g.fit_t4 + 5 * beta * g.fit_t5))));
   sp = -coef * (g.fit_s1 + beta * (2 * g.fit_s2 + beta * (3 * g.fit_s3 + beta *
@@ -280,6 +315,7 @@ __device__ __forceinline__ void ttf(double r_beta, const G& g, double& t, double
 }
 
 // SimulatePartialDriftKernel body, simulation_kernel.cu:95-115
+template <class A>
 __device__ __forceinline__ void drift(Particle& p, double h, double aper, double wavelen,
                                       uint32_t elem, double mass, double rmass)
 {
@@ -291,15 +327,17 @@ __device__ __forceinline__ void drift(Particle& p, double h, double aper, double
   if (aper2 != 0.0 && x * x + y * y > aper2) {
     p.loss = elem;
   } else {
+    const double gm1 = A::div_by(p.w, mass, rmass);
+    p.mark |= A::mark(gm1);
     p.x = x;
     p.y = y;
-    const double gm1 = div_by(p.w, mass, rmass);
-    const double bt = pdiv(psqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
-    p.phi += pdiv(TWOPI * h, wavelen * bt);
+    const double bt = A::div(A::sqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
+    p.phi += A::div(TWOPI * h, wavelen * bt);
   }
 }
 
 // SimulateHalfQuadKernel body, simulation_kernel.cu:147-214
+template <class A>
 __device__ __forceinline__ void half_quad(Particle& p, double length, double aper,
                                           double gradient, double wavelen, uint32_t elem,
                                           double mass, double rmass, double charge)
@@ -309,16 +347,18 @@ __device__ __forceinline__ void half_quad(Particle& p, double length, double ape
   const double qg = gradient * charge;
   double x = p.x, y = p.y, xp = p.xp, yp = p.yp;
   const double w = p.w;
+  const double gm1 = A::div_by(w, mass, rmass);
+  p.mark |= A::mark(gm1);
   if (qg == 0) {
     // the loss test below uses the coordinates before this half-drift
     p.x = x + xp * length * 0.5;
     p.y = y + yp * length * 0.5;
   } else {
-    const double gamma1 = div_by(w, mass, rmass);
-    const double bg = psqrt(gamma1 * (gamma1 + 2.0) * (1.0 + xp * xp + yp * yp));
+    const double bg = A::sqrt(gm1 * (gm1 + 2.0) * (1.0 + xp * xp + yp * yp));
+    p.mark |= A::mark(bg);
     const double absqg = qg > 0.0 ? qg : -qg;
-    const double k = psqrt(pdiv(absqg, bg * mass) * CLIGHT);
-    const double inv_k = pdiv(1.0, k);
+    const double k = A::sqrt(A::div(absqg, bg * mass) * CLIGHT);
+    const double inv_k = A::div(1.0, k);
     const double kds = length * 0.25 * k;
     double s, c;
     double sh, ch;
@@ -341,42 +381,41 @@ __device__ __forceinline__ void half_quad(Particle& p, double length, double ape
   if (aper2 != 0 && x * x + y * y > aper2) {
     p.loss = elem;
   } else {
-    const double gm1 = div_by(w, mass, rmass);
-    const double bt = pdiv(psqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
-    p.phi += pdiv(TWOPI * length * 0.5, wavelen * bt);
+    const double bt = A::div(A::sqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
+    p.phi += A::div(TWOPI * length * 0.5, wavelen * bt);
   }
 }
 
 // SimulateRFGapFirstHalfKernel body, simulation_kernel.cu:239-285
-template <class G, class U>
+template <class A, class G, class U>
 __device__ __forceinline__ void gap_first_half(Particle& p, const G& gap, const U& u, bool ccl,
                                                double mass, double rmass)
 {
   const double x = p.x, y = p.y, xp = p.xp, yp = p.yp, phi = p.phi, w = p.w;
+  const double gam = A::div_by(w, mass, rmass);
+  p.mark |= A::mark(gam);
   p.x = x + u.dd1 * xp;
   p.y = y + u.dd1 * yp;
   if (gap.amplitude == 0.0) {
-    const double gm1 = div_by(w, mass, rmass);
-    const double bt = pdiv(psqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
-    p.phi += pdiv(u.twopi_dd1, u.wave_len * bt);
+    const double bt = A::div(A::sqrt(gam * (gam + 2.0)), gam + 1.0);
+    p.phi += A::div(u.twopi_dd1, u.wave_len * bt);
   } else {
     const double beta_in = u.beta_in1;
-    const double gam = div_by(w, mass, rmass);
-    const double beta = pdiv(psqrt((gam + 2.0) * gam), gam + 1.0);
+    const double beta = A::div(A::sqrt((gam + 2.0) * gam), gam + 1.0);
     if (!ccl) {
-      const double bl = beta * u.wave_len, rbl = recip(bl);
-      const double dphi_qlen1 = div_by(u.twopi_half_q1, bl, rbl);
+      const double bl = beta * u.wave_len, rbl = A::recip(bl);
+      const double dphi_qlen1 = A::div_by(u.twopi_half_q1, bl, rbl);
       double dphi_clen = 0.0;
-      if (u.dcl1_nonzero) dphi_clen = div_by(u.pi_dcl1, bl, rbl);
-      p.phi = phi + (1.0 - pdiv(beta - beta_in, beta)) * u.pclbl_dps1 + dphi_clen - dphi_qlen1;
+      if (u.dcl1_nonzero) dphi_clen = A::div_by(u.pi_dcl1, bl, rbl);
+      p.phi = phi + (1.0 - A::div(beta - beta_in, beta)) * u.pclbl_dps1 + dphi_clen - dphi_qlen1;
     } else {
-      p.phi = phi + (1.0 - pdiv((beta - beta_in) * u.betag1, beta * beta_in)) * u.pclbl_dps1;
+      p.phi = phi + (1.0 - A::div((beta - beta_in) * u.betag1, beta * beta_in)) * u.pclbl_dps1;
     }
   }
 }
 
 // SimulateRFGapSecondHalfKernel body, simulation_kernel.cu:326-493
-template <class G, class U>
+template <class A, class G, class U>
 __device__ __forceinline__ void gap_second_half(Particle& p, const G& gap, const U& u,
                                                 double wavelen, bool ccl,
                                                 double mass, double rmass)
@@ -387,16 +426,17 @@ __device__ __forceinline__ void gap_second_half(Particle& p, const G& gap, const
   double w = p.w;
   const double beta_in = u.beta_in2;
   double gam = w * inv_mass;
-  const double bg1 = psqrt(gam * (gam + 2.0));
-  double beta = pdiv(bg1, gam + 1.0);
+  p.mark |= A::mark(gam);
+  const double bg1 = A::sqrt(gam * (gam + 2.0));
+  double beta = A::div(bg1, gam + 1.0);
   double t_fac, tp_fac, sp_fac;
-  ttf(beta, gap, t_fac, tp_fac, sp_fac);
+  ttf<A>(beta, gap, t_fac, tp_fac, sp_fac);
   if (gap.amplitude == 0.0 || (ccl && beta < gap.fit_beta_min)) {
     p.x = x + u.dd2 * xp;
     p.y = y + u.dd2 * yp;
-    const double gm1 = div_by(p.w, mass, rmass);
-    const double bt = pdiv(psqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
-    p.phi += pdiv(u.twopi_dd2, wavelen * bt);
+    const double gm1 = A::div_by(p.w, mass, rmass);
+    const double bt = A::div(A::sqrt(gm1 * (gm1 + 2.0)), gm1 + 1.0);
+    p.phi += A::div(u.twopi_dd2, wavelen * bt);
     return;
   }
   const double wave_len = u.wave_len;
@@ -404,7 +444,7 @@ __device__ __forceinline__ void gap_second_half(Particle& p, const G& gap, const
   double con5nex, tw;
   if (ccl) {
     con5nex = u.concomm * (t_fac * u.inv_fkis - u.bgw * tp_fac * inv_gmg2);
-    tw = t_fac - pdiv(TWOPI * tp_fac * (pdiv(beta_in, beta) - 1.0) * u.betag_ccl, beta_in);
+    tw = t_fac - A::div(TWOPI * tp_fac * (A::div(beta_in, beta) - 1.0) * u.betag_ccl, beta_in);
   } else {
     con5nex = u.concomm * (t_fac * u.inv_fkis - u.bgw * tp_fac * inv_gmg2);
     tw = t_fac;
@@ -415,7 +455,7 @@ __device__ __forceinline__ void gap_second_half(Particle& p, const G& gap, const
   const double sinps = u.sinps, cosps = u.cosps;
   double phi1, sinp1, cosp1;
   if (ccl)
-    phi1 = phi + gap.phase_shift - pdiv(u.twopi_dg, beta * wave_len) + u.cell_pi;
+    phi1 = phi + gap.phase_shift - A::div(u.twopi_dg, beta * wave_len) + u.cell_pi;
   else
     phi1 = phi + gap.phase_shift;
   psincos(phi1, &sinp1, &cosp1);
@@ -424,40 +464,42 @@ __device__ __forceinline__ void gap_second_half(Particle& p, const G& gap, const
   const double rs_p = x * x + y * y;
   const double rrp = x * xp + y * yp;
   double rpris = 0.0, bes1covr;
-  const double ris = psqrt(rs_p);
+  const double ris = A::sqrt0(rs_p);
   const double fkrris = fkr * ris;
   double b0c, b1c, b1p;
-  bessel_all(fkrris, b0c, b1c, b1p);
-  const double rris = recip(ris), rgmg = recip(gmg);
-  if (ris != 0.0) bes1covr = div_by(b1c, ris, rris);
+  bessel_all<A>(fkrris, b0c, b1c, b1p);
+  const double rris = A::recip(ris), rgmg = A::recip(gmg);
+  if (ris != 0.0) bes1covr = A::div_by(b1c, ris, rris);
   else bes1covr = fkr * 0.5;
-  const double delte = u.q_efl * (tw * b0c * cosp1 + (div_by(tw - TWOPI * tp_fac, gmg, rgmg) * bes1covr +
-                       div_by(tw, gmg, rgmg) * fkr * b1p - tw * gmg * bes1covr) * rrp * sinp1);
+  const double delte = u.q_efl * (tw * b0c * cosp1 +
+                       (A::div_by(tw - TWOPI * tp_fac, gmg, rgmg) * bes1covr +
+                        A::div_by(tw, gmg, rgmg) * fkr * b1p - tw * gmg * bes1covr) * rrp * sinp1);
   w += delte;
   gam = w * inv_mass;
-  const double bg = psqrt(gam * (gam + 2.0));
-  beta = pdiv(bg, gam + 1.0);
-  const double bgr = pdiv(bg1, bg);
+  const double bg = A::sqrt(gam * (gam + 2.0));
+  beta = A::div(bg, gam + 1.0);
+  const double bgr = A::div(bg1, bg);
   const double onema = 1.0 - (con5nex * bes1covr + con5nex1 * b1p + con5nex2 * bes1covr) * cosp1;
+  p.mark |= A::mark0(rs_p) | A::mark0(rrp) | A::mark(gam) | A::mark(onema);
   const double dovbl = u.con2nex * bes1covr * tw * sinp1;
-  const double bgrovonema = pdiv(bgr, onema);
+  const double bgrovonema = A::div(bgr, onema);
   xp = -dovbl * x + bgrovonema * xp;
   x = x * onema + u.dd2 * xp;
   yp = -dovbl * y + bgrovonema * yp;
   y = y * onema + u.dd2 * yp;
-  if (rs_p > 0.0) rpris = div_by(rrp, ris, rris);
+  if (rs_p > 0.0) rpris = A::div_by(rrp, ris, rris);
   const double prome = u.two_con1 * (-tp_fac * b0c + ris * tw * b1c * u.inv_gmgcl) *
                        (sinp1 - sinps) - u.efl_inv_mass * tw * b1c * rpris * (cosp1 - cosps);
   double phi_new;
   if (ccl) {
-    phi_new = phi + (1.0 - pdiv((beta - u.beta_out) * u.betag_ccl, beta * u.beta_out)) *
+    phi_new = phi + (1.0 - A::div((beta - u.beta_out) * u.betag_ccl, beta * u.beta_out)) *
               u.pclbl_dps2 + prome;
   } else {
-    const double bl = beta * wave_len, rbl = recip(bl);
-    const double dphi_qlen2 = div_by(u.twopi_half_q2, bl, rbl);
+    const double bl = beta * wave_len, rbl = A::recip(bl);
+    const double dphi_qlen2 = A::div_by(u.twopi_half_q2, bl, rbl);
     double dphi_clen = 0.0;
-    if (u.dcl2_nonzero) dphi_clen = div_by(u.pi_dcl2, bl, rbl);
-    phi_new = phi + (1.0 - pdiv(beta - u.beta_out, beta)) * u.pclbl_dps2 + prome + dphi_clen -
+    if (u.dcl2_nonzero) dphi_clen = A::div_by(u.pi_dcl2, bl, rbl);
+    phi_new = phi + (1.0 - A::div(beta - u.beta_out, beta)) * u.pclbl_dps2 + prome + dphi_clen -
               dphi_qlen2;
   }
   if (w <= 0.0 || x != x || y != y || xp != xp || yp != yp || w != w || phi_new != phi_new) {
@@ -480,14 +522,16 @@ __device__ __forceinline__ void rotation(Particle& p, double angle)
 }
 
 // SimulateSteererKernel body, simulation_kernel.cu:128-137
+template <class A>
 __device__ __forceinline__ void steerer(Particle& p, double blh, double blv, double mass,
                                         double rmass, double charge)
 {
-  const double gm1 = div_by(p.w, mass, rmass);
-  const double btgm = psqrt(gm1 * (gm1 + 2.0));
-  const double pm = pdiv(btgm * mass, CLIGHT);
-  if (blh > 1e-10) p.xp += pdiv(blh * charge, pm);
-  if (blv > 1e-10) p.yp += pdiv(blv * charge, pm);
+  const double gm1 = A::div_by(p.w, mass, rmass);
+  p.mark |= A::mark(gm1);
+  const double btgm = A::sqrt(gm1 * (gm1 + 2.0));
+  const double pm = A::div(btgm * mass, CLIGHT);
+  if (blh > 1e-10) p.xp += A::div(blh * charge, pm);
+  if (blv > 1e-10) p.yp += A::div(blv * charge, pm);
 }
 
 // SimulateBuncherKernel body, simulation_kernel.cu:807-874 (rsqrt as 1/sqrt).
@@ -632,22 +676,23 @@ __device__ __forceinline__ void dipole_second_half(Particle& p, D* a, double mas
 
 // Apply one map step to an alive particle.  rmass: the rounded 1 / mass
 // (div_by).
-template <int kClass, class OpT>
+template <class A, int kClass, class OpT>
 __device__ __forceinline__ void apply_op(const OpT& op, Particle& p, uint32_t index, double mass,
                                          double rmass, double charge, double x_avg, double y_avg)
 {
   switch (op.kind) {
-    case OP_DRIFT: drift(p, op.a[0], op.a[1], op.a[2], op.elem, mass, rmass); break;
+    case OP_DRIFT: drift<A>(p, op.a[0], op.a[1], op.a[2], op.elem, mass, rmass); break;
     case OP_QUAD:
       if constexpr (kClass >= OPC_QUAD)
-        half_quad(p, op.a[0], op.a[1], op.a[2], op.a[3], op.elem, mass, rmass, charge);
+        half_quad<A>(p, op.a[0], op.a[1], op.a[2], op.a[3], op.elem, mass, rmass, charge);
       break;
     case OP_GAP1:
-      if constexpr (kClass >= OPC_GAP) gap_first_half(p, op.g, op.gu, op.ccl != 0, mass, rmass);
+      if constexpr (kClass >= OPC_GAP)
+        gap_first_half<A>(p, op.g, op.gu, op.ccl != 0, mass, rmass);
       break;
     case OP_GAP2:
       if constexpr (kClass >= OPC_GAP)
-        gap_second_half(p, op.g, op.gu, op.a[5], op.ccl != 0, mass, rmass);
+        gap_second_half<A>(p, op.g, op.gu, op.a[5], op.ccl != 0, mass, rmass);
       break;
     case OP_BUNCH:
       if constexpr (kClass >= OPC_GAP) buncher(p, op.a, op.elem, mass, charge);
@@ -659,7 +704,7 @@ __device__ __forceinline__ void apply_op(const OpT& op, Particle& p, uint32_t in
       if constexpr (kClass >= OPC_GAP) dipole_second_half(p, op.a, mass);
       break;
     case OP_ROT: rotation(p, op.a[0]); break;
-    case OP_STEER: steerer(p, op.a[0], op.a[1], mass, rmass, charge); break;
+    case OP_STEER: steerer<A>(p, op.a[0], op.a[1], mass, rmass, charge); break;
     case OP_APER_C: {   // simulation_kernel.cu:548-555 (particle 0 exempt)
       if (index == 0) break;
       const double aper2 = op.a[0] * op.a[0];
@@ -682,13 +727,14 @@ __device__ __forceinline__ void apply_op(const OpT& op, Particle& p, uint32_t in
 // of radius rs, before the c1 charge factor: the complete-elliptic-integral
 // fit of UpdateFldTbl1Kernel (space_charge_kernel.cu:52-71, repeated for the
 // image rings at :74-94); er is 0 on the axis.
+template <class A>
 HPS_HD void ring_green(double rs, double rp, double d, double& er, double& ez)
 {
   const double d2 = d * d;
   const double c = (rp - rs) * (rp - rs);
   const double b = (rp + rs) * (rp + rs);
   const double rsrp = rs * rp;
-  double a = pdiv(4.0 * rsrp, b + d2);
+  double a = A::div(4.0 * rsrp, b + d2);
   const double g = 1.0 - a;
   const double h = hps::log(g);
   const double ee = 1.0 + g * (0.4630106 - 0.2452740 * h + g * (0.1077857 - 0.04125321 * h));
@@ -697,8 +743,8 @@ HPS_HD void ring_green(double rs, double rp, double d, double& er, double& ez)
   a = ::sqrt(b + d2);
   const double rs2mrp2 = (rs * rs - rp * rp);
   er = 0.0;
-  if (rp != 0.0) er = pdiv(ek - pdiv((rs2mrp2 + d2) * ee, c + d2), 2.0 * rp * a);
-  ez = pdiv(d * ee, a * (c + d2));
+  if (rp != 0.0) er = A::div(ek - A::div((rs2mrp2 + d2) * ee, c + d2), 2.0 * rp * a);
+  ez = A::div(d * ee, a * (c + d2));
 }
 
 // log of the bunch-frame cell aspect dz*gm/dr of a SCHEFF mesh (0 for

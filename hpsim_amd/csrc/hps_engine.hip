@@ -1406,8 +1406,12 @@ extern "C" int hps_sim_simulate(hps_sim* m, int32_t start, int32_t end)
       a.stats = st.stats;
       a.rmax = (st.stats == STAT_SC && m->sc && m->sc->cfg.adj_bunch != 0) ? 1 : 0;
       a.op_class = OPC_LIGHT;
-      for (int32_t o = st.op_begin; o < st.op_end; ++o)
+      bool usual = in_range(b->mass) && zero_or_in_range(st.kick_len);
+      for (int32_t o = st.op_begin; o < st.op_end; ++o) {
         a.op_class = std::max(a.op_class, op_class_of(c.ops[o].kind));
+        usual = usual && op_usual(c.ops[o], b->charge);
+      }
+      a.mark = usual ? 0u : Quick::kOff;
       launches.push_back(l);
       if (a.stats != STAT_NONE) {
         l.kind = L_SEG_FINAL;
@@ -2438,8 +2442,12 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
         a.stats = st.stats;
         a.rmax = (st.stats == STAT_SC && m->sc && m->sc->cfg.adj_bunch != 0) ? 1 : 0;
         a.op_class = OPC_LIGHT;
-        for (int32_t o = st.op_begin; o < st.op_end; ++o)
+        bool usual = in_range(b->mass) && zero_or_in_range(st.kick_len);
+        for (int32_t o = st.op_begin; o < st.op_end; ++o) {
           a.op_class = std::max(a.op_class, op_class_of(cs[k].ops[o].kind));
+          usual = usual && op_usual(cs[k].ops[o], b->charge);
+        }
+        a.mark = usual ? 0u : Quick::kOff;
       }
       launches.push_back({L_SEG, cursor, recs[0].op_class});
       if (st0.stats != STAT_NONE) launches.push_back({L_SEG_FINAL, cursor, 0});

@@ -211,7 +211,8 @@ __global__ __launch_bounds__(kThreads) void k_gemm_tables(const GemmState* __res
     const double rs = ::sqrt(0.5 * (rs_i * rs_i + (rs_i + 1) * (rs_i + 1)));
     const double d = (dzi + 1) * dzg - 0.5 * dzg;
     double er, ez;
-    ring_green(rs, (double)rp_i, d, er, ez);
+    if (in_range(dzg)) ring_green<Quick>(rs, (double)rp_i, d, er, ez);
+    else ring_green<Any>(rs, (double)rp_i, d, er, ez);
     float* row = tables + slot * slot_sz + ((size_t)rp_i * nr + rs_i) * 4 * nz;
     // delta = -dz (zs >= zp, E_z negated) and delta = dz + 1 (zs < zp)
     row[nz - 1 - dzi] = (float)er;

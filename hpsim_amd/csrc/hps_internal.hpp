@@ -23,9 +23,10 @@ struct BeamArrays {
 // Device-resident SCHEFF state: the SpaceCharge members the reference keeps
 // on the host (space_charge.h:83-124) plus the values of the last control
 // step (Scheff::Start, space_charge.cpp:82-139).
+constexpr int32_t kRemesh = 1, kRemeshQuick = 2;   // Quick: with k_mark 0
 struct ScDev {
   hps_spch_state st;
-  int32_t remesh;       // last control step rebuilt the tables
+  int32_t remesh;       // last control step rebuilds the tables: 0, kRemesh or kRemeshQuick
   int32_t valid;        // tables hold a field
   double beta, freq, frac, current;
   double ratio_r, ratio_z, ratio_q, ratio_g;
@@ -36,6 +37,8 @@ struct ScDev {
   double k_xfac, k_yfac, k_er_ratio, k_ez_ratio;
   double k_pl;          // bunch spacing beta*gamma*lambda (adjacent-bunch images)
   uint32_t adj_eff;     // adjacent bunches each side at this kick point
+  uint32_t fld_off;     // the field tables' charge factor was not below 2^64
+  uint32_t k_mark;      // 0 where the kick constants are in Quick's range, else Quick::kOff
   uint32_t pad_;
   double log_aspect;    // log(dz * gamma / dr) of the last remesh (grouped field solve)
 };
@@ -68,6 +71,8 @@ struct SegArgs {
   int32_t stats;           // StatKind computed after the maps
   int32_t op_class;        // OpClass: heaviest map in [op_begin, op_end)
   int32_t rmax;            // STAT_SC also keeps the per-chunk largest r^2
+  uint32_t mark;           // 0 where the mass, the kick length and the maps' constants are in
+                           // Quick's range (hps_math.hpp), else Quick::kOff
 };
 
 struct PhaseArgs {

@@ -223,12 +223,14 @@ struct KickConst {
   double er_ratio, ez_ratio, cbgcoef, r_beta, phi_ref, pl;
   double repsq, rdr, rdzg;   // rounded reciprocals of epsq, dr, dzg
   uint32_t nx, nz, adj;
+  uint32_t mark;   // 0 where these are in Quick's range, else Quick::kOff
 };
 
 // The kick constants of ApplySpchKickKernel (space_charge_kernel.cu:578-640):
 // the parts fixed by the control step come from ScDev (kick_prepare in
 // k_phase_final); the element length, the on-mesh count (k_deposit) and the
 // phase references (which a host frequency step may change) are read here.
+template <class A>
 __device__ __forceinline__ KickConst kick_const(const ScDev* scg, const hps_beam_stats* stg,
                                                 double r_length)
 {
@@ -250,7 +252,7 @@ __device__ __forceinline__ KickConst kick_const(const ScDev* scg, const hps_beam
   k.nz = sc->st.nz;
   k.hl = sc->k_hl;
   k.c2 = sc->k_c2;
-  k.c3 = div_by(r_length, sc->k_bgmg, sc->k_rbgmg);
+  k.c3 = A::div_by(r_length, sc->k_bgmg, sc->k_rbgmg);
   k.repsq = sc->k_repsq;
   k.rdr = sc->k_rdr;
   k.rdzg = sc->k_rdzg;
@@ -263,15 +265,18 @@ __device__ __forceinline__ KickConst kick_const(const ScDev* scg, const hps_beam
   k.phi_ref = st->phi_avg_good;
   k.pl = sc->k_pl;
   k.adj = sc->adj_eff;
+  k.mark = sc->k_mark;
   return k;
 }
 
 // The control-step part of the kick constants, in the expressions of
 // ApplySpchKickKernel; r_num_part, r_mass: the beam's size and mass.
-__device__ __forceinline__ void kick_prepare(ScDev* sc, double r_beta, double r_freq,
+// fld_off: of the last remesh.  Returns whether Quick covers them.
+__device__ __forceinline__ bool kick_prepare(ScDev* sc, double r_beta, double r_freq,
     double r_current, double x_avg_good, double y_avg_good, double x_sig_good,
     double y_sig_good, double dr, double dz, uint32_t nz, double ratio_r, double ratio_z,
-    double ratio_q, double ratio_g, uint32_t r_num_part, double r_mass)
+    double ratio_q, double ratio_g, uint32_t r_num_part, double r_mass, bool remesh,
+    uint32_t fld_off)
 {
   const double epsq = x_sig_good / y_sig_good;
   const double gmg = 1.0 / ::sqrt(1.0 - r_beta * r_beta);
@@ -297,24 +302,40 @@ __device__ __forceinline__ void kick_prepare(ScDev* sc, double r_beta, double r_
   sc->k_yfac = epsq * xfac;
   sc->k_er_ratio = ratio_q / (ratio_r * ratio_z * ratio_g * ratio_g);
   sc->k_ez_ratio = ratio_q / (ratio_z * ratio_z);
+  if constexpr (!kBounded) return false;
+  // The others follow: gmg is 1 at least, c2 and pl are products of two of
+  // these, xfac and yfac at most 2.  With c1 and the ratios below 2^64 (they
+  // may be 0) the field tables, kept until the next remesh, and the field
+  // outside the mesh stay below 2^500.
+  const uint32_t m = Quick::mark(epsq) | Quick::mark(sc->k_dr) | Quick::mark(dzg) |
+                     Quick::mark(wave_len) | Quick::mark(sc->k_bgmg);
+  const uint32_t c1_off = !below_range_end(sc->k_c1), table_off = remesh ? c1_off : fld_off;
+  const uint32_t off = (uint32_t)Quick::off(m) | c1_off | table_off |
+                       !below_range_end(sc->k_er_ratio) | !below_range_end(sc->k_ez_ratio);
+  sc->fld_off = table_off;
+  sc->k_mark = off ? Quick::kOff : 0u;
+  return off == 0;
 }
 
+template <class A>
 __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const double* tbl,
                                      double r_mass, double rmass)
 {
   const double phi = relative_phi(p.phi, k.phi_ref);   // phi_r of UpdateRelativePhi(true)
-  const double gm = div_by(p.w, r_mass, rmass) + 1.0;
-  const double bgz = psqrt((gm - 1.0) * (gm + 1.0));
+  const double gm1 = A::div_by(p.w, r_mass, rmass);
+  const double gm = gm1 + 1.0;
+  const double bgz = A::sqrt((gm - 1.0) * (gm + 1.0));
   double bgx = bgz * p.xp;
   double bgy = bgz * p.yp;
   double bgzstar = k.gmg * (bgz - k.r_beta * gm);
   const double xxbar = p.x - k.xbar;
   const double yybar = p.y - k.ybar;
-  double r = psqrt(div_by(xxbar * xxbar, k.epsq, k.repsq) + yybar * yybar * k.epsq);
+  const double r2 = A::div_by(xxbar * xxbar, k.epsq, k.repsq) + yybar * yybar * k.epsq;
+  double r = A::sqrt(r2);
   if (r == 0.0) r = 1.0e-8;
-  const double rr = recip(r);
-  const double xovr = div_by(xxbar * k.xfac, r, rr);
-  const double yovr = div_by(yybar * k.yfac, r, rr);
+  const double rr = A::recip(r);
+  const double xovr = A::div_by(xxbar * k.xfac, r, rr);
+  const double yovr = A::div_by(yybar * k.yfac, r, rr);
   double ddz = phi - k.phimc;
   for (int guard = 0; (ddz > PI || ddz < -PI) && guard < 4096; ++guard) {
     if (ddz > 0.0) ddz -= TWOPI;
@@ -324,8 +345,9 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
   double cbgr, cbgzs;
   if (r > k.nx * k.dr || __builtin_fabs(z) > k.hl) {
     z = -k.c2 * (phi - k.phimc);
-    const double d = psqrt(z * z + r * r);
-    const double invd3 = pdiv(1.0, d * d * d);
+    const double d = A::sqrt(z * z + r * r);
+    p.mark |= A::mark(d);
+    const double invd3 = A::div(1.0, d * d * d);
     double rod3 = r * invd3;
     double zod3 = z * invd3;
     // point charges of the neighbouring bunches (space_charge_kernel.cu:650-662)
@@ -333,8 +355,8 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
       int xi = (int)nb;
       for (int lr = 0; lr < 2; ++lr) {
         const double sz = z + xi * k.pl;
-        const double dd = psqrt(sz * sz + r * r);
-        const double iv = pdiv(1.0, dd * dd * dd);
+        const double dd = A::sqrt(sz * sz + r * r);
+        const double iv = A::div(1.0, dd * dd * dd);
         rod3 += r * iv;
         zod3 += sz * iv;
         xi = -xi;
@@ -343,7 +365,7 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
     cbgr = k.cbgcoef * rod3;
     cbgzs = k.cbgcoef * zod3;
   } else {
-    const double ri = div_by(r, k.dr, k.rdr), zj = div_by(z + k.hl, k.dzg, k.rdzg);
+    const double ri = A::div_by(r, k.dr, k.rdr), zj = A::div_by(z + k.hl, k.dzg, k.rdzg);
     const uint32_t i = (uint32_t)(1 + to_int(ri));
     const double a = ri - (i - 1.0);
     const double b = 1.0 - a;
@@ -355,6 +377,10 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
     uint32_t m = l + (k.nx + 1);
     if (m >= tbl_sz) m = tbl_sz - 1;
     if (l >= tbl_sz) l = tbl_sz - 1;
+    if constexpr (std::is_same<A, Quick>::value) {   // out of its range i and j are anything
+      if (m < 1) m = 1;
+      if (l < 1) l = 1;
+    }
     const double tl0 = gld(tbl, 2 * l), tl1 = gld(tbl, 2 * l + 1);
     const double tk0 = gld(tbl, 2 * (l - 1)), tk1 = gld(tbl, 2 * (l - 1) + 1);
     const double tm0 = gld(tbl, 2 * m), tm1 = gld(tbl, 2 * m + 1);
@@ -367,13 +393,16 @@ __device__ __forceinline__ void kick(Particle& p, const KickConst& k, const doub
   bgzstar += cbgzs;
   const double gstar = 1.0 + 0.5 * bgzstar * bgzstar;
   const double bgzf = k.gmg * (bgzstar + k.r_beta * gstar);
+  // Terms that lie below their quotient's range are lost in bgx and bgy, by
+  // less than half an ulp, wherever these are in range themselves.
+  p.mark |= A::mark(gm1) | A::mark(r2) | A::mark(bgx) | A::mark(bgy) | A::mark(bgzf) | k.mark;
   if (bgzf <= 0.0) {
     p.loss = 9999;
   } else {
-    const double rbg = recip(bgzf);
-    p.xp = div_by(bgx, bgzf, rbg);
-    p.yp = div_by(bgy, bgzf, rbg);
-    p.w *= 1.0 + pdiv((gm + 1.0) * (bgzf - bgz), gm * bgz);
+    const double rbg = A::recip(bgzf);
+    p.xp = A::div_by(bgx, bgzf, rbg);
+    p.yp = A::div_by(bgy, bgzf, rbg);
+    p.w *= 1.0 + A::div((gm + 1.0) * (bgzf - bgz), gm * bgz);
   }
 }
 
@@ -482,11 +511,13 @@ constexpr int kSegGroupQuad = HPS_SEG_GROUP_QUAD;
 constexpr int kSegGroupLight = HPS_SEG_GROUP_LIGHT;
 
 // Particle i of the beam, or an excluded placeholder (loss = 1) past the end.
-__device__ __forceinline__ Particle load_particle(const BeamArrays& b, uint32_t i)
+__device__ __forceinline__ Particle load_particle(const BeamArrays& b, uint32_t i,
+                                                  uint32_t mark = 0)
 {
   Particle p;
   p.loss = 1; p.lloss = 0;
   p.x = p.xp = p.y = p.yp = p.phi = p.w = 0.0;
+  p.mark = mark;
   if (i < b.n) {
     p.loss = gld(b.loss, i);
     p.lloss = gld(b.lloss, i);
@@ -505,6 +536,70 @@ __device__ __forceinline__ void store_particle(const BeamArrays& b, uint32_t i, 
   if (q.loss != 0) gst(b.loss, i, q.loss);
 }
 
+// The arguments of k_segment_batch, in their order.
+struct SegBatchArgs {
+  const SegArgs* recs;
+  const uint32_t* map;
+  const uint64_t* roff;
+};
+
+// This workgroup's SegArgs in memory: the one argument of k_segment and
+// k_segment_wide, or its record of k_segment_batch.  The empty asm hides where
+// the pointer comes from, so nothing read before is kept for what reads here.
+typedef const __attribute__((address_space(4))) SegArgs SegArgsConst;
+
+template <bool kBatch>
+__device__ __forceinline__ SegArgsConst* own_args()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef const __attribute__((address_space(4))) SegBatchArgs CArgs;
+  typedef const __attribute__((address_space(4))) uint32_t CMap;
+  typedef const __attribute__((address_space(4))) uint64_t COff;
+  uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm("" : "+s"(at));
+  if constexpr (kBatch) {
+    const CArgs& k = *(CArgs*)at;
+    const uint32_t e = ((CMap*)(uint64_t)k.map)[blockIdx.x];
+    at = (uint64_t)k.recs + ((COff*)(uint64_t)k.roff)[0] + (e >> kBatchLocalBits) * sizeof(SegArgs);
+  }
+  return (SegArgsConst*)at;
+#else
+  return nullptr;
+#endif
+}
+
+// The kick and the maps of particle i once more, from memory and through Any,
+// where Quick does not cover it.  Nothing is stored between, and the two share
+// no value.  (With either form tried at each map k_segment took 82 to 90
+// VGPRs, five waves per SIMD instead of seven; with the arguments shared, 40
+// more scalar registers were spilled.)
+template <int kClass, bool kBatch>
+__device__ __forceinline__ void redo(uint32_t i, Particle& p)
+{
+  if constexpr (kBounded) {
+    if (__builtin_expect(!Quick::off(p.mark), 1)) return;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+v"(i));
+#endif
+    SegArgsConst& a = *own_args<kBatch>();
+    BeamArrays b;
+    b.x = a.b.x; b.xp = a.b.xp; b.y = a.b.y; b.yp = a.b.yp; b.phi = a.b.phi; b.w = a.b.w;
+    b.loss = a.b.loss; b.lloss = a.b.lloss;
+    b.n = a.b.n;
+    const double mass = a.b.mass, charge = a.b.charge;
+    p = load_particle(b, i);
+    if (p.loss != 0) return;
+    if (a.kick && p.lloss == 0 && (i & a.kick_mask) != 0)
+      kick<Any>(p, kick_const<Any>(a.sc, a.st, a.kick_len), a.fld2, mass, 0.0);
+    const hps_beam_stats* st = a.st;
+    const double xa = st->x_avg, ya = st->y_avg;
+    for (int o = a.op_begin; o < a.op_end; ++o) {
+      const OpConst& op = ((const OpConst*)a.ops)[o];
+      if (p.loss == 0) apply_op<Any, kClass>(op, p, i, mass, 0.0, charge, xa, ya);
+    }
+  }
+}
+
 // One workgroup per 1024-particle chunk; each lane carries its four
 // particles (i = chunk*1024 + j*256 + lane) through the kick, the maps and
 // the store in groups of kGroup, and accumulates the chunk statistics in the
@@ -516,7 +611,7 @@ __device__ __forceinline__ void store_particle(const BeamArrays& b, uint32_t i, 
 //                  (UpdateLoss + UpdateAvgXY, simulation_engine.cu:311-312).
 // The group size trades registers (waves per SIMD) against independent
 // chains per wave.
-template <int kClass, int kGroup>
+template <int kClass, int kGroup, bool kBatch>
 __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSmem& sm)
 {
   static_assert(kPerLane % kGroup == 0, "group must divide the particles per lane");
@@ -539,7 +634,7 @@ __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSm
 #pragma unroll
     for (int g = 0; g < kGroup; ++g) {
       const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
-      p[g] = load_particle(b, i);
+      p[g] = load_particle(b, i, a.mark);
       alive_in[g] = i < b.n && p[g].loss == 0;
     }
     if (a.kick) {
@@ -548,12 +643,12 @@ __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSm
       const ScDev* scp = a.sc;
       const hps_beam_stats* stp = a.st;
       asm volatile("" : "+s"(scp), "+s"(stp));
-      const KickConst k = kick_const(scp, stp, a.kick_len);
+      const KickConst k = kick_const<Usual>(scp, stp, a.kick_len);
 #pragma unroll
       for (int g = 0; g < kGroup; ++g) {
         const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
         if (alive_in[g] && p[g].lloss == 0 && (i & a.kick_mask) != 0)
-          kick(p[g], k, a.fld2, b.mass, b.rmass);
+          kick<Usual>(p[g], k, a.fld2, b.mass, b.rmass);
       }
     }
     for (int o = a.op_begin; o < a.op_end; ++o) {
@@ -561,9 +656,13 @@ __device__ __forceinline__ void segment_body(const SegArgs& a, uint32_t c, RedSm
 #pragma unroll
       for (int g = 0; g < kGroup; ++g) {
         const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
-        if (p[g].loss == 0) apply_op<kClass>(op, p[g], i, b.mass, b.rmass, b.charge, xa, ya);
+        if (p[g].loss == 0)
+          apply_op<Usual, kClass>(op, p[g], i, b.mass, b.rmass, b.charge, xa, ya);
       }
     }
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g)
+      redo<kClass, kBatch>(c * kChunk + (j0 + g) * kBlock + t, p[g]);
 #pragma unroll
     for (int g = 0; g < kGroup; ++g) {
       const uint32_t i = c * kChunk + (j0 + g) * kBlock + t;
@@ -707,12 +806,13 @@ __device__ __forceinline__ void segment_body_live(const SegArgs& a, uint32_t c, 
       const ScDev* scp = a.sc;
       const hps_beam_stats* stp = a.st;
       asm volatile("" : "+s"(scp), "+s"(stp));
-      const KickConst k = kick_const(scp, stp, a.kick_len);
-      if (p.lloss == 0 && (i & a.kick_mask) != 0) kick(p, k, a.fld2, b.mass, b.rmass);
+      const KickConst k = kick_const<Usual>(scp, stp, a.kick_len);
+      if (p.lloss == 0 && (i & a.kick_mask) != 0)
+        kick<Usual>(p, k, a.fld2, b.mass, b.rmass);
     }
     for (int o = a.op_begin; o < a.op_end; ++o) {
       const OpConst& op = ((const OpConst*)a.ops)[o];
-      if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
+      if (p.loss == 0) apply_op<Usual, kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
     }
     store_particle(b, i, p);
     if (a.stats == STAT_SC) {
@@ -773,7 +873,7 @@ template <int kClass, int kGroup>
 __global__ __launch_bounds__(kBlock) void k_segment(SegArgs a)
 {
   __shared__ RedSmem sm;
-  segment_body<kClass, kGroup>(a, blockIdx.x, sm);
+  segment_body<kClass, kGroup, false>(a, blockIdx.x, sm);
 }
 
 // The same over the chunks of several simulations: map[block] packs the
@@ -786,10 +886,16 @@ __device__ __forceinline__ const T* period_recs(const T* recs, const uint64_t* r
   return (const T*)((const char*)recs + roff[0]);
 }
 
+// Waves per SIMD: the classes without RF gaps need 66 VGPRs with the second
+// pass of redo, two more than eight waves leave (seven members on 32 x 128:
+// 59.5 us a launch at seven waves, 56.0 at eight).
+template <int kClass>
+constexpr int kBatchWaves = kBounded && kClass < OPC_GAP ? 8 : 1;
+
 template <int kClass, int kGroup>
-__global__ __launch_bounds__(kBlock) void k_segment_batch(const SegArgs* __restrict__ recs,
-                                                          const uint32_t* __restrict__ map,
-                                                          const uint64_t* __restrict__ roff)
+__global__ __launch_bounds__(kBlock, kBatchWaves<kClass>) void k_segment_batch(
+    const SegArgs* __restrict__ recs, const uint32_t* __restrict__ map,
+    const uint64_t* __restrict__ roff)
 {
   __shared__ RedSmem sm;
   const uint32_t e = map[blockIdx.x];
@@ -798,7 +904,7 @@ __global__ __launch_bounds__(kBlock) void k_segment_batch(const SegArgs* __restr
   __shared__ LiveSmem ls;
   segment_body_live<kClass>(a, e & kBatchLocalMask, sm, ls);
 #else
-  segment_body<kClass, kGroup>(a, e & kBatchLocalMask, sm);
+  segment_body<kClass, kGroup, true>(a, e & kBatchLocalMask, sm);
 #endif
 }
 
@@ -832,17 +938,18 @@ __device__ __forceinline__ void segment_body_wide(const SegArgs& a, uint32_t c, 
   const int t = threadIdx.x;
   const BeamArrays& b = a.b;
   const uint32_t i = c * kChunk + (uint32_t)t;
-  Particle p = load_particle(b, i);
+  Particle p = load_particle(b, i, a.mark);
   const bool alive_in = i < b.n && p.loss == 0;
   if (a.kick && alive_in && p.lloss == 0 && (i & a.kick_mask) != 0) {
-    const KickConst k = kick_const(a.sc, a.st, a.kick_len);
-    kick(p, k, a.fld2, b.mass, b.rmass);
+    const KickConst k = kick_const<Usual>(a.sc, a.st, a.kick_len);
+    kick<Usual>(p, k, a.fld2, b.mass, b.rmass);
   }
   const double xa = a.st->x_avg, ya = a.st->y_avg;
   for (int o = a.op_begin; o < a.op_end; ++o) {
     const OpConst& op = ((const OpConst*)a.ops)[o];
-    if (p.loss == 0) apply_op<kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
+    if (p.loss == 0) apply_op<Usual, kClass>(op, p, i, b.mass, b.rmass, b.charge, xa, ya);
   }
+  redo<kClass, false>(i, p);
   const bool in = i < b.n;
   if (alive_in) store_particle(b, i, p);
   if (a.stats == STAT_NONE) return;
@@ -1261,6 +1368,7 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
   __shared__ int remesh;
   __shared__ uint32_t nbins;
   const int t = threadIdx.x;
+  uint32_t fld_off = 0;
   const BeamArrays& b = a.b;
   hps_beam_stats* st = a.st;
   ScDev* sc = a.sc;
@@ -1280,6 +1388,7 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
     ke = st->w_avg_good;
     phi_sig_good = st->phi_sig_good;
     ss = sc->st;
+    fld_off = sc->fld_off;
   }
   // waves 0..2: the relative-phase sums; wave 3: Beam::UpdateMaxRPhi
   // (beam.cu:829-851), the largest r^2 about the last all-particle centroid
@@ -1390,12 +1499,13 @@ __device__ __forceinline__ void phase_final_body(const PhaseArgs& a)
     sc->ratio_z = ratio_z;
     sc->ratio_q = ratio_q;
     sc->ratio_g = ratio_g;
-    sc->remesh = rm;
     sc->adj_eff = adj;
     if (rm) sc->valid = 1;
-    kick_prepare(sc, beta, a.freq, a.current * a.frac, x_avg_good, y_avg_good, x_sig_good,
+    const bool usual =
+        kick_prepare(sc, beta, a.freq, a.current * a.frac, x_avg_good, y_avg_good, x_sig_good,
                  y_sig_good, ss.dr, ss.dz, ss.nz, ratio_r, ratio_z, ratio_q, ratio_g, b.n,
-                 b.mass);
+                 b.mass, rm != 0, fld_off);
+    sc->remesh = rm ? (usual ? kRemeshQuick : kRemesh) : 0;
   }
 }
 
@@ -1413,6 +1523,7 @@ __global__ __launch_bounds__(kPhaseFinalBlock) void k_phase_final_batch(const Ph
 // One entry of the ring Green's table, UpdateFldTbl1Kernel
 // (space_charge_kernel.cu:38-100), stored [rp][dz][rs] so that the field sum
 // reads consecutive rs.
+template <class A>
 __device__ __forceinline__ void greens_entry(const ScDev* sc, double* fld1, uint32_t nr,
                                              uint32_t nz, uint32_t r_num_part, double mass,
                                              uint32_t idx)
@@ -1440,7 +1551,7 @@ __device__ __forceinline__ void greens_entry(const ScDev* sc, double* fld1, uint
   const double rp = rpi * dr;
   const double d = zp - zs;
   double er1, ez1;
-  ring_green(rs, rp, d, er1, ez1);
+  ring_green<A>(rs, rp, d, er1, ez1);
   // image rings of the neighbouring bunches, one RF period apart in the
   // bunch frame (space_charge_kernel.cu:74-94)
   const uint32_t adj = sc->adj_eff;
@@ -1451,7 +1562,7 @@ __device__ __forceinline__ void greens_entry(const ScDev* sc, double* fld1, uint
       double xi = (double)i;
       for (int j = 0; j < 2; ++j) {
         double er, ez;
-        ring_green(rs, rp, d - xi * pl, er, ez);
+        ring_green<A>(rs, rp, d - xi * pl, er, ez);
         if (rp != 0.0) er1 += er;
         ez1 += ez;
         xi = -xi;
@@ -1493,25 +1604,35 @@ __device__ __forceinline__ DepConst dep_const(const hps_beam_stats* st, const Sc
   d.hl = d.nz * 0.5 * d.dzg;
   d.c2 = r_beta * gm * wave_len / TWOPI;
   d.drdr = d.dr * d.dr;
-  d.repsq = recip(d.epsq);
-  d.rdr = recip(d.dr);
-  d.rdzg = recip(d.dzg);
-  d.rdrdr = recip(d.drdr);
+  if constexpr (kBounded) {
+    d.repsq = recip(d.epsq);
+    d.rdr = recip(d.dr);
+    d.rdzg = recip(d.dzg);
+    d.rdrdr = recip(d.drdr);
+  }
   return d;
+}
+
+// The squared radius of a particle scaled to the round beam.
+template <class A>
+__device__ __forceinline__ double deposit_r2(double x, double y, const DepConst& d)
+{
+  return A::div_by((x - d.xbar) * (x - d.xbar), d.epsq, d.repsq) +
+         (y - d.ybar) * (y - d.ybar) * d.epsq;
 }
 
 // One good particle's charge into the LDS histogram: the area weights in r,
 // the linear weights in z, as 2^-36 fixed point (DistributeParticleKernel's
 // body, space_charge_kernel.cu:151-218); returns whether it landed on the
-// mesh.
-__device__ __forceinline__ bool deposit_one(double x, double y, double phi, const DepConst& d,
+// mesh.  rsq_sh: the squared radius (deposit_r2).
+template <class A>
+__device__ __forceinline__ bool deposit_one(double rsq_sh, double phi, const DepConst& d,
                                             unsigned long long* hist)
 {
   const uint32_t nx = d.nx, nz = d.nz;
   const double dr = d.dr, dzg = d.dzg, drdr = d.drdr, hl = d.hl;
   double z = relative_phi(phi, d.ref);
-  const double rsq_sh = div_by((x - d.xbar) * (x - d.xbar), d.epsq, d.repsq) + (y - d.ybar) * (y - d.ybar) * d.epsq;
-  const int i = to_int(div_by(psqrt(rsq_sh), dr, d.rdr) + 1);
+  const int i = to_int(A::div_by(A::sqrt(rsq_sh), dr, d.rdr) + 1);
   if (i < 1 || i > (int)nx) return false;
   double ddz = z - d.phimc;
   for (int guard = 0; (ddz > PI || ddz < -PI) && guard < 4096; ++guard) {
@@ -1521,7 +1642,7 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
   z = -d.c2 * ddz;
   if (!(__builtin_fabs(z) < hl)) return false;
   const double zz = z + hl;
-  const int jm1 = to_int(div_by(zz, dzg, d.rdzg) + 1);
+  const int jm1 = to_int(A::div_by(zz, dzg, d.rdzg) + 1);
   int i1 = i + 1;
   if (rsq_sh < 0.5 * drdr * (double)(i * i + (i - 1) * (i - 1))) i1 = i - 1;
   if (i1 < 1) i1 = 1;
@@ -1534,14 +1655,14 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
   if (i1 == i) {
     a = 1.0;
   } else {
-    const double sqrtmp = psqrt(div_by(4.0 * rsq_sh, drdr, d.rdrdr) - 1.0);
+    const double sqrtmp = A::sqrt(A::div_by(4.0 * rsq_sh, drdr, d.rdrdr) - 1.0);
     const double rminsq = 0.25 * drdr * (sqrtmp - 1.0) * (sqrtmp - 1.0);
     const double rmaxsq = rminsq + sqrtmp * drdr;
-    if (i1 < i) a = pdiv(rmaxsq - (i - 1) * (i - 1) * drdr, rmaxsq - rminsq);
-    else a = pdiv((i1 - 1) * (i1 - 1) * drdr - rminsq, rmaxsq - rminsq);
+    if (i1 < i) a = A::div(rmaxsq - (i - 1) * (i - 1) * drdr, rmaxsq - rminsq);
+    else a = A::div((i1 - 1) * (i1 - 1) * drdr - rminsq, rmaxsq - rminsq);
   }
   double cc = 1.0;
-  if (j1 != jm1) cc = pdiv(zz - (j1 - 1 + 0.5) * dzg, (jm1 - j1) * dzg);
+  if (j1 != jm1) cc = A::div(zz - (j1 - 1 + 0.5) * dzg, (jm1 - j1) * dzg);
   const double bb = 1.0 - a;
   const double dd = 1.0 - cc;
   if (jm1 < 1 || jm1 > (int)nz) return false;
@@ -1565,8 +1686,8 @@ __device__ __forceinline__ bool deposit_one(double x, double y, double phi, cons
 // of 4,194,304 particles on 64 x 256: 226 -> 185 ms per 160-element step).
 __device__ __forceinline__ void deposit_block(const BeamArrays& b, const hps_beam_stats* st,
                                               ScDev* sc, int64_t* bins, uint32_t blk,
-                                              uint32_t nblk, unsigned long long* hist,
-                                              uint32_t* ured)
+                                              uint32_t nblk, bool usual,
+                                              unsigned long long* hist, uint32_t* ured)
 {
   const int t = threadIdx.x;
   const DepConst d = dep_const(st, sc);
@@ -1575,6 +1696,7 @@ __device__ __forceinline__ void deposit_block(const BeamArrays& b, const hps_bea
   if (t == 0) ured[0] = 0;
   __syncthreads();
   uint32_t count = 0;
+  bool again = false;
   const uint32_t stride = nblk * kDepositBlock;
   uint32_t np = blk * kDepositBlock + t;
   bool have = np < b.n;
@@ -1593,7 +1715,22 @@ __device__ __forceinline__ void deposit_block(const BeamArrays& b, const hps_bea
       lo = gld(b.loss, np); ll = gld(b.lloss, np);
       x = gld(b.x, np); y = gld(b.y, np); ph = gld(b.phi, np);
     }
-    if (clo == 0 && cll == 0 && deposit_one(cx, cy, cph, d, hist)) ++count;
+    if (clo == 0 && cll == 0) {
+      const double r2 = deposit_r2<Usual>(cx, cy, d);
+      if (!usual || Usual::off(Usual::mark(r2))) again = true;
+      else if (deposit_one<Usual>(r2, cph, d, hist)) ++count;
+    }
+  }
+  if constexpr (kBounded) {
+    // the particles that Quick does not cover, in a sweep of their own
+    if (__builtin_expect(again, 0)) {
+      for (uint32_t i = blk * kDepositBlock + t; i < b.n; i += stride) {
+        if (gld(b.loss, i) != 0 || gld(b.lloss, i) != 0) continue;
+        const double px = gld(b.x, i), py = gld(b.y, i);
+        if (usual && in_range(deposit_r2<Quick>(px, py, d))) continue;
+        if (deposit_one<Any>(deposit_r2<Any>(px, py, d), gld(b.phi, i), d, hist)) ++count;
+      }
+    }
   }
   __syncthreads();
   for (uint32_t i = t; i < nb; i += kDepositBlock) {
@@ -1619,16 +1756,30 @@ __device__ __forceinline__ void sc_build_body(const BuildArgs& a, uint32_t nr, u
                                               uint32_t blk, unsigned long long* hist,
                                               uint32_t* ured)
 {
-  if (!a.sc->remesh) return;
-  if (blk < a.greens_wgs) {
-    const uint32_t total = (nr + 1) * nz * nr;
-    for (uint32_t i = blk * kDepositBlock + threadIdx.x; i < total;
-         i += a.greens_wgs * kDepositBlock)
-      greens_entry(a.sc, a.fld1, nr, nz, a.b.n, a.b.mass, i);
-    if (a.side) return;
+  const int remesh = a.sc->remesh;
+  if (!remesh) return;
+  const bool usual = !kBounded || __builtin_expect(remesh == kRemeshQuick, 1);
+  const bool table = blk < a.greens_wgs;
+  const uint32_t total = (nr + 1) * nz * nr;
+  const uint32_t first = blk * kDepositBlock + threadIdx.x, step = a.greens_wgs * kDepositBlock;
+  if (table && usual)
+    for (uint32_t i = first; i < total; i += step)
+      greens_entry<Usual>(a.sc, a.fld1, nr, nz, a.b.n, a.b.mass, i);
+  if (!(table && a.side))
+    deposit_block(a.b, a.st, a.sc, a.bins, a.side ? blk - a.greens_wgs : blk, a.dep_blocks, usual,
+                  hist, ured);
+  // a mesh that Quick does not cover; here, where its loop keeps no register
+  // of the usual one's
+  if constexpr (kBounded) {
+    if (table && !usual) {
+      const ScDev* sc = a.sc;
+#ifdef __HIP_DEVICE_COMPILE__
+      asm volatile("" : "+s"(sc));
+#endif
+      for (uint32_t i = first; i < total; i += step)
+        greens_entry<Any>(sc, a.fld1, nr, nz, a.b.n, a.b.mass, i);
+    }
   }
-  deposit_block(a.b, a.st, a.sc, a.bins, a.side ? blk - a.greens_wgs : blk, a.dep_blocks, hist,
-                ured);
 }
 
 __global__ __launch_bounds__(kDepositBlock) void k_sc_build(BuildArgs a, uint32_t nr, uint32_t nz)
@@ -1984,6 +2135,7 @@ __global__ void k_probe(int fn, const double* x, const double* y, double* out, u
     case 16: psinhcosh(v, &s, &c); r = c; break;
     case 17: r = pdiv(v, y[i]); break;
     case 18: r = div_by(v, y[i], 1.0 / y[i]); break;
+    case 19: r = sqrt_unscaled(v); break;
     default: break;
   }
   out[i] = r;

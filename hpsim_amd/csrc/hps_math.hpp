@@ -24,6 +24,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define HPS_HD __host__ __device__ __forceinline__
 
 namespace hps {
@@ -42,22 +44,17 @@ HPS_HD uint64_t bits_of(double v) { return __builtin_bit_cast(uint64_t, v); }
 HPS_HD double double_of(uint64_t u) { return __builtin_bit_cast(double, u); }
 HPS_HD double pow2i(int k) { return double_of((uint64_t)(k + 1023) << 52); }
 
-// Quotients and square roots of the per-particle maps, the kick, the deposit
-// and the Green's table.  The tracking kernels are bound by vector
-// instructions (k_segment 88 % of its waves' time), and the compiler spends
-// eleven on a quotient and twenty-one on a root, several of which only scale
-// operands near the ends of the exponent range.  These are its sequences
-// without the scaling: the reciprocal of v_rcp_f64 with two Newton steps,
-// one corrected quotient (the residual is exact), v_div_fixup for zeros,
-// infinities and NaN; the root of v_rsq_f64 with one Goldschmidt step and
-// two corrections.  Where neither operand nor result comes within 2^54 of
-// the ends of the normal range (numerators from 2^-968, denominators between
-// 2^-1000 and 2^1000, roots of 2^-960 and up) every step rounds the same, so
-// the result is the correctly rounded one.  Quotients by one denominator
-// share its reciprocal: four instructions for each further one.
-// 1,048,576 particles on 32 x 128, 800 elements: k_segment 36.7 -> 33.3 us a
-// kick point, k_sc_build 15.2 -> 14.3; 500,009 particles without space charge,
-// 400 elements: 3.13 -> 2.70 ms (with the coefficients of uconst).
+// Quotients without exponent scaling.  The compiler spends eleven vector
+// instructions on an FP64 quotient, several of which only scale operands near
+// the ends of the exponent range.  This is its sequence without them: the
+// reciprocal of v_rcp_f64 with two Newton steps, one corrected quotient (the
+// residual is exact), v_div_fixup for zeros, infinities and NaN.  For a
+// numerator that is 0 or of 2^-968 and up, a denominator between 2^-1000 and
+// 2^1000 and a quotient between 2^-1000 and 2^1000 every step rounds the
+// same, so the result is the correctly rounded one.  Past that it is not (a
+// subnormal denominator gives NaN), so callers keep their operands in range:
+// see Quick below.  Quotients by one denominator share its reciprocal: four
+// instructions for each further one.
 // The build of hps_push_fast.hip and host code divide as they are compiled.
 static HPS_HD double recip(double d)
 {
@@ -375,8 +372,8 @@ static __device__ __forceinline__ void psinhcosh(double x, double* shp, double* 
 #endif
 }
 
-// The square root of the per-particle maps, the kick and the deposit (see
-// recip above), or sqrt_rsq in the build of hps_push_fast.hip,
+// The square root of the per-particle maps, the kick and the deposit: the
+// correctly rounded ::sqrt, or sqrt_rsq in the build of hps_push_fast.hip,
 // which serves batches whose results are held to error bounds, not to the
 // oracle's bits.  Internal to each translation unit, so the two builds keep
 // their own.
@@ -385,16 +382,116 @@ static __device__ __forceinline__ double psqrt(double x)
 #ifdef HPS_FAST_PUSH
   return sqrt_rsq(x);
 #else
+  return ::sqrt(x);
+#endif
+}
+
+// The root of v_rsq_f64 with one Goldschmidt step and two corrections, ten
+// instructions where ::sqrt takes twenty-one: correctly rounded from 2^-960 to
+// 2^1000, NaN for 0 and infinity.
+static __device__ __forceinline__ double sqrt_unscaled(double x)
+{
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = ::fma(-h, g, 0.5);
   g = ::fma(g, r, g);
   h = ::fma(h, r, h);
   g = ::fma(::fma(-g, g, x), h, g);
-  g = ::fma(::fma(-g, g, x), h, g);
-  return (x == 0.0 || x == kInf) ? x : g;
-#endif
+  return ::fma(::fma(-g, g, x), h, g);
 }
+
+// Quotients and roots of the maps, the kick, the deposit and the Green's
+// table, which take one of these as a template argument.
+//
+// Any takes every operand: the compiler's own sequences.
+//
+// Quick leaves out the exponent scaling (recip, div_by, sqrt_unscaled) and
+// gives the same bits while all operands stay in the range stated there.  A
+// function that takes it marks the few values of the particle that every
+// quotient and root of it follows from; where one of them lies outside
+// 2^-64 .. 2^64 or is 0, infinite or NaN (off), the particle goes through Any
+// instead.  The element's or mesh's constants are held to the same range (or
+// 0 where they are only numerators) once, before the particles (usual).  A sum
+// of such values is 0 or at least an ulp of the smaller one, so cancellation
+// stays far above 2^-968.
+// The tracking kernels are bound by vector instructions (k_segment 88 % of its
+// waves' time); a mark costs two, the zero and infinity cases that its roots
+// need not treat three each.  1,048,576 particles on 32 x 128, 800 elements,
+// a step: 60.8 ms, with Any alone 65.7.
+#if defined(HPS_FAST_PUSH) || !defined(__HIP_DEVICE_COMPILE__)
+constexpr bool kBounded = false;
+#else
+constexpr bool kBounded = true;
+#endif
+
+namespace {
+
+struct Any {
+  // Its quotients are not moved past each other: it is seldom run, and side by
+  // side they would take the kernels from 65 to 79 VGPRs.
+  static HPS_HD void order()
+  {
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HPS_FAST_PUSH)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+  }
+  static HPS_HD double recip(double) { return 0.0; }
+  static HPS_HD double div(double n, double d)
+  {
+    order();
+    const double q = n / d;
+    order();
+    return q;
+  }
+  static HPS_HD double div_by(double n, double d, double) { return div(n, d); }
+  static __device__ __forceinline__ double sqrt(double x)
+  {
+    order();
+    const double q = psqrt(x);
+    order();
+    return q;
+  }
+  static __device__ __forceinline__ double sqrt0(double x) { return psqrt(x); }
+  static HPS_HD uint32_t mark(double) { return 0; }
+  static HPS_HD uint32_t mark0(double) { return 0; }
+  static HPS_HD bool off(uint32_t) { return false; }
+};
+
+struct Quick {
+  static HPS_HD double recip(double d) { return hps::recip(d); }
+  static HPS_HD double div(double n, double d) { return hps::pdiv(n, d); }
+  static HPS_HD double div_by(double n, double d, double y) { return hps::div_by(n, d, y); }
+  static __device__ __forceinline__ double sqrt(double x) { return sqrt_unscaled(x); }
+  static __device__ __forceinline__ double sqrt0(double x) { return x > 0.0 ? sqrt(x) : x; }
+  // bits 27 to 30 of a mark are 0 if and only if |v| is in [2^-64, 2^64):
+  // the biased exponent less that of 2^-64, modulo 2^11.  Marks are or'ed.
+  static HPS_HD uint32_t mark(double v) { return (uint32_t)(bits_of(v) >> 32) - 0x3bf00000u; }
+  // The same with 0 in range (a particle on the axis).  Infinities and NaN
+  // pass too: for the RF gap, which loses such a particle in either form.
+  static __device__ __forceinline__ uint32_t mark0(double v)
+  {
+#ifdef __HIP_DEVICE_COMPILE__
+    return (uint32_t)(__builtin_amdgcn_frexp_exp(v) + 63) << 20;
+#else
+    return 0;
+#endif
+  }
+  static constexpr uint32_t kOff = 0x78000000u;
+  static HPS_HD bool off(uint32_t m) { return (m & kOff) != 0; }
+};
+
+typedef std::conditional<kBounded, Quick, Any>::type Usual;
+
+// |v| in [2^-64, 2^64)
+HPS_HD bool in_range(double v) { return !Quick::off(Quick::mark(v)); }
+// |v| < 2^64
+HPS_HD bool below_range_end(double v)
+{
+  return (uint32_t)(bits_of(v) >> 32 & 0x7fffffffu) < 0x43f00000u;
+}
+HPS_HD bool zero_or_in_range(double v) { return bits_of(v) << 1 == 0 || in_range(v); }
+
+}  // namespace
 
 // Remainder of x >= 0 by y > 0 (finite), exact.
 HPS_HD double fmod_pos(double x, double y)

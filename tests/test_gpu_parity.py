@@ -3,6 +3,7 @@ seeded inputs.  Coordinates and loss flags must match bit for bit."""
 import numpy as np
 import pytest
 
+from hpsim_amd import configs as cfg
 from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +68,107 @@ def test_unscaled_quotients_and_roots_are_ieee(fn, span):
     g = HPSim.probe_math(fn, x, None if fn == "psqrt" else y)
     same = (g.view(np.uint64) == ref.view(np.uint64)) | (np.isnan(g) & np.isnan(ref))
     assert same.all(), (fn, x[~same][:4], g[~same][:4], ref[~same][:4])
+
+
+def test_unscaled_quotients_and_roots_at_the_ends_of_their_range():
+    """pdiv, div_by and sqrt_unscaled round correctly up to the limits that
+    hps_math.hpp states for them; psqrt does for every double."""
+    from hpsim_amd import HPSim
+    rng = np.random.default_rng(8)
+
+    def some(lo, hi, n=200000):
+        """Either sign, exponents in [lo, hi], a quarter of them at the ends;
+        a fifth of the significands all ones but the last few bits."""
+        e = rng.integers(lo, hi + 1, n)
+        e[: n // 8], e[n // 8: n // 4] = lo, hi
+        m = rng.integers(0, 1 << 52, n, dtype=np.uint64)
+        m[::5] |= np.uint64((1 << 52) - 16)
+        u = (rng.integers(0, 2, n).astype(np.uint64) << np.uint64(63)) | (
+            (e + 1023).astype(np.uint64) << np.uint64(52)) | m
+        return u.view(np.float64)
+
+    n, d = some(-968, 999), rng.permutation(some(-1000, 999))
+    with np.errstate(all="ignore"):
+        ref = n / d
+    keep = (np.abs(ref) >= 2.0 ** -1000) & (np.abs(ref) <= 2.0 ** 1000)
+    assert keep.sum() > 50000
+    for fn in ("pdiv", "div_by"):
+        g = HPSim.probe_math(fn, n[keep], d[keep])
+        assert np.array_equal(g.view(np.uint64), ref[keep].view(np.uint64)), fn
+    x = np.abs(some(-960, 999))
+    g = HPSim.probe_math("sqrt_unscaled", x)
+    assert np.array_equal(g.view(np.uint64), np.sqrt(x).view(np.uint64))
+    x = rng.integers(0, 1 << 64, 400000, dtype=np.uint64)
+    x[::4] &= np.uint64((1 << 53) - 1)   # subnormals and the smallest normals
+    x = x.view(np.float64)
+    g = HPSim.probe_math("psqrt", x)
+    with np.errstate(all="ignore"):
+        ref = np.sqrt(x)
+    assert ((g.view(np.uint64) == ref.view(np.uint64)) | (np.isnan(g) & np.isnan(ref))).all()
+
+
+def _extreme_beam(num, sc, thin, tiny_elements):
+    """A workload whose particles, among ordinary ones, have coordinates and
+    energies anywhere down to the smallest subnormals; thin: a sheet, so that
+    every mesh constant in x is tiny; tiny_elements: lengths and gradients far
+    below any real one."""
+    wl = H.workload(0, num=num, periods=2, sc=sc)
+    elems = cfg.build_lattice(wl.lattice)
+    extra = [cfg.Element("ROT", "Rotation", angle=0.3),
+             cfg.Element("ST", "Steerer", bl_h=2e-4, bl_v=1e-4)]
+    elems = elems[:4] + extra + elems[4:]
+    if tiny_elements:
+        elems[2:2] = [cfg.Element("DT", "Drift", length=1e-300),
+                      cfg.Element("QT", "Quad", length=0.02, gradient=1e-290)]
+    dist = [np.array(v) for v in cfg.make_distribution(wl.beam)]
+    rng = np.random.default_rng(12)
+    if thin:
+        dist[0] *= 1e-150
+        dist[1] *= 1e-150
+    else:
+        for k in (0, 1, 2, 3) if sc else (0, 1, 2, 3, 5):
+            some = rng.random(num) < 0.3
+            dist[k][some] *= 10.0 ** rng.uniform(-320, 0, int(some.sum()))
+        axis = rng.random(num) < 0.1     # on the axis but for the last bits
+        dist[0][axis] = 10.0 ** rng.uniform(-323, -140, int(axis.sum()))
+        dist[2][axis] = 0.0
+    return wl, elems, dist
+
+
+@pytest.mark.parametrize("num,sc,thin,tiny_elements", [
+    # one and four particles per thread, without and with kicks and deposits
+    (4096, False, False, False), (600000, False, False, False),
+    (4096, True, False, False), (600000, True, False, False),
+    (4096, False, False, True), (4096, True, True, False)])
+def test_extreme_coordinates_bit_exact(num, sc, thin, tiny_elements):
+    """The maps, the kick and the deposit hold to the oracle's bits over the
+    whole range of doubles, not only where Quick covers them."""
+    wl, elems, dist = _extreme_beam(num, sc, thin, tiny_elements)
+    ob, _, _ = H.run_oracle(wl, elems=elems, dist=dist)
+    gb, _, _ = H.run_gpu(wl, elems=elems, dist=dist)
+    err = H.compare_arrays(gb.arrays(), ob.arrays())
+    assert err is None, err
+
+
+@pytest.mark.parametrize("sc,thin", [(False, False), (True, False), (True, True)])
+def test_extreme_coordinates_bit_exact_in_a_batch(sc, thin):
+    from hpsim_amd import HPSim
+    wl, elems, dist = _extreme_beam(4096, sc, thin, not sc)
+    ob, _, _ = H.run_oracle(wl, elems=elems, dist=dist)
+    sims = []
+    for _ in range(2):
+        b = HPSim.Beam(mass=wl.beam.mass, charge=wl.beam.charge, current=wl.beam.current,
+                       num=wl.beam.num)
+        b.set_distribution(*dist)
+        b.set_frequency(wl.beam.freq)
+        b.set_ref_w(wl.beam.w0)
+        sims.append(HPSim.Simulator(b, HPSim.BeamLine(elements=elems),
+                                    HPSim.SpaceCharge(nr=wl.nr, nz=wl.nz, interval=wl.interval)
+                                    if sc else None))
+    HPSim.Batch(sims).simulate()
+    for s in sims:
+        err = H.compare_arrays(s.beam.arrays(), ob.arrays())
+        assert err is None, err
 
 
 @pytest.mark.parametrize("num,periods", [(1000, 3), (4096, 4)])
