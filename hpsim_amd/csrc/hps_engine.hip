@@ -141,7 +141,7 @@ class PinnedLease {
     }
     if (p_) (void)hipHostFree(p_);
   }
-  Pinned* get() const { return p_; }
+  Pinned* get() const { return p_; }   // null where there is no pinned memory to be had
   hipError_t wait(hipStream_t s)
   {
     const hipError_t e = hipStreamSynchronize(s);
@@ -169,15 +169,28 @@ struct Pair {
 int read_sums(hps_beam* b, const Pair* p, int n, hps_beam_stats* s)
 {
   PinnedLease pin;
-  if (!pin.get()) return fail("pinned host allocation failed");
-  Readout* const ro = &pin.get()->ro;
+  Readout* ro = pin.get() ? &pin.get()->ro : nullptr;
+  // without pinned memory: a device block, and a copy
+  struct Block {
+    Readout* p = nullptr;
+    ~Block() { if (p) (void)hipFree(p); }
+  } dev;
+  if (!ro) {
+    HPS_CHECK(hipMalloc(&dev.p, sizeof(Readout)));
+    ro = dev.p;
+  }
   for (int k = 0; k < n; ++k) {
     HPS_CHECK(launch_sums(b->d, p[k].a, p[k].bb, p[k].filter, b->pr, b->stream, p[k].rel_ref,
                           &ro->sums[k], s && k == n - 1 ? ro : nullptr, b->st));
   }
-  HPS_CHECK(pin.wait(b->stream));
-  b->ro = *ro;
-  if (s) *s = ro->st;
+  if (dev.p) {
+    HPS_CHECK(hipMemcpyAsync(&b->ro, ro, sizeof(Readout), hipMemcpyDeviceToHost, b->stream));
+    HPS_CHECK(hipStreamSynchronize(b->stream));
+  } else {
+    HPS_CHECK(pin.wait(b->stream));
+    b->ro = *ro;
+  }
+  if (s) *s = b->ro.st;
   return 0;
 }
 
@@ -581,19 +594,20 @@ int hps_beam_download(hps_beam* b, double* x, double* xp, double* y, double* yp,
     // a small beam: one kernel writes the arrays into pinned memory, one wait
     // (eight copies of 16 KB, each with its own wait: 160 us; so 25)
     PinnedLease pin;
-    if (!pin.get()) return fail("pinned host allocation failed");
-    BeamArrays dst = b->d;
-    uint8_t* at = pin.get()->stage;
-    double** dd[6] = {&dst.x, &dst.xp, &dst.y, &dst.yp, &dst.phi, &dst.w};
-    for (double** d : dd) { *d = (double*)at; at += nd; }
-    dst.loss = (uint32_t*)at; dst.lloss = (uint32_t*)(at + nu);
-    HPS_CHECK(launch_copy_beam(b->d, dst, b->stream));
-    HPS_CHECK(pin.wait(b->stream));
-    for (int k = 0; k < 6; ++k)
-      if (out[k]) std::memcpy(out[k], *dd[k], nd);
-    if (loss) std::memcpy(loss, dst.loss, nu);
-    if (lloss) std::memcpy(lloss, dst.lloss, nu);
-    return 0;
+    if (pin.get()) {
+      BeamArrays dst = b->d;
+      uint8_t* at = pin.get()->stage;
+      double** dd[6] = {&dst.x, &dst.xp, &dst.y, &dst.yp, &dst.phi, &dst.w};
+      for (double** d : dd) { *d = (double*)at; at += nd; }
+      dst.loss = (uint32_t*)at; dst.lloss = (uint32_t*)(at + nu);
+      HPS_CHECK(launch_copy_beam(b->d, dst, b->stream));
+      HPS_CHECK(pin.wait(b->stream));
+      for (int k = 0; k < 6; ++k)
+        if (out[k]) std::memcpy(out[k], *dd[k], nd);
+      if (loss) std::memcpy(loss, dst.loss, nu);
+      if (lloss) std::memcpy(lloss, dst.lloss, nu);
+      return 0;
+    }
   }
   HPS_CHECK(hipStreamSynchronize(b->stream));
   for (int k = 0; k < 6; ++k)

@@ -5,12 +5,15 @@ The reference writes the header values at the stream's default precision
 (6 significant digits) and the particle rows at 15; reading back sets the
 reference particle's transverse coordinates to 0 and the design energy to
 its w."""
+import os
+
 import numpy as np
 import pytest
 
 from hpsim_amd import configs as cfg
 from hpsim_amd.HPSim import read_beam_file, write_beam_file
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 COORDS = ("x", "xp", "y", "yp", "phi", "w")
 
 
@@ -95,3 +98,44 @@ def test_print_to_and_beam_from_file_on_the_engine(tmp_path):
     assert nb.get_frequency() == wl.beam.freq
     assert nb.get_mass() == wl.beam.mass and nb.get_charge() == wl.beam.charge
     assert nb.get_ref_w() == e["w"][0]
+
+
+@pytest.mark.gpu
+def test_getters_without_pinned_memory(tmp_path):
+    """Where no pinned host memory can be had the getters, a restore and a
+    small beam's arrays are read through device memory: the same values."""
+    import json
+    import subprocess
+    import sys
+    src = tmp_path / "none.c"
+    src.write_text("#include <stddef.h>\n"
+                   "int calls;\n"
+                   "int hipHostMalloc(void** p, size_t n, unsigned f)\n"
+                   "{ (void)n; (void)f; *p = NULL; ++calls; return 2; }   // out of memory\n")
+    lib = tmp_path / "none.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    prog = """
+import ctypes, json, sys
+none = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL) if len(sys.argv) > 1 else None
+import numpy as np
+from hpsim_amd import HPSim
+rng = np.random.default_rng(3)
+b = HPSim.Beam(mass=939.294, charge=-1.0, current=0.01, num=3000)
+b.set_distribution(*rng.normal(0, 1e-3, (4, 3000)), rng.normal(-0.5, 0.3, 3000),
+                   0.75 + rng.normal(0, 1e-3, 3000))
+b.set_frequency(201.25)
+b.save_initial_beam()
+b.apply_cut("x", 1e-3, 1.0)
+v = [b.get_loss_num("t"), b.get_loss_num("l"), b.get_loss_num("all"), b.get_avg_x(),
+     b.get_sig_phi("longitudinal_good"), b.get_emittance_x(), b.get_emittance_z(), b.get_current()]
+v += [float(x) for x in b.get_x("good")[:9]] + [int(x) for x in b.get_losses()[:9]]
+b.restore_initial_beam()
+v += [b.get_loss_num("t"), b.get_avg_phi("relative")] + [float(x) for x in b.arrays()["w"][:9]]
+calls = ctypes.c_int.in_dll(none, "calls").value if none else 0
+print(json.dumps([v, calls]))
+"""
+    out = [json.loads(subprocess.run([sys.executable, "-c", prog, *a], check=True, timeout=100,
+                                     cwd=ROOT, capture_output=True, text=True).stdout)
+           for a in ([], [str(lib)])]
+    assert out[1][1] > 0, "the library allocated past the failing function"
+    assert out[0][0] == out[1][0]
