@@ -123,8 +123,10 @@ class PinnedLease {
         return;
       }
     }
-    if (hipHostMalloc((void**)&p_, sizeof(Pinned), hipHostMallocPortable) != hipSuccess)
+    if (hipHostMalloc((void**)&p_, sizeof(Pinned), hipHostMallocPortable) != hipSuccess) {
       p_ = nullptr;
+      (void)hipGetLastError();   // the caller does without
+    }
   }
   PinnedLease(const PinnedLease&) = delete;
   PinnedLease& operator=(const PinnedLease&) = delete;
@@ -1580,7 +1582,6 @@ extern "C" int hps_sim_simulate(hps_sim* m, int32_t start, int32_t end)
         put(ptrs, sizeof ptrs);
         put(&sc->cfg.nx, sizeof sc->cfg.nx);
         put(&sc->cfg.nz, sizeof sc->cfg.nz);
-        put(&sc->max_lds, sizeof sc->max_lds);
       }
       if (!m->graph_exec || sig != m->graph_sig) {
         if (m->graph_exec) { (void)hipGraphExecDestroy(m->graph_exec); m->graph_exec = nullptr; }
@@ -1750,8 +1751,11 @@ static std::vector<uint32_t> xcd_chunk_map(const std::vector<uint32_t>& nch)
   return map;
 }
 
+// A captured period graph holds these buffers, so it goes with them (their
+// successors may come to lie at the same addresses).
 static void free_gemm(hps_batch* bt)
 {
+  if (bt->pgraph_exec) { (void)hipGraphExecDestroy(bt->pgraph_exec); bt->pgraph_exec = nullptr; }
   (void)hipFree(bt->d_mem); (void)hipFree(bt->d_gs); (void)hipFree(bt->d_perm);
   (void)hipFree(bt->d_tables); (void)hipFree(bt->d_q); (void)hipFree(bt->d_w);
   (void)hipFree(bt->mm.pos_exact); (void)hipFree(bt->mm.pos_nn); (void)hipFree(bt->mm.fallback);
@@ -2514,15 +2518,16 @@ extern "C" int hps_batch_simulate(hps_batch* bt, int32_t start, int32_t end)
     for (size_t j = run.a; j < run.a + run.p; ++j) put(&launches[j], sizeof(BLaunch));
     const void* ptrs[] = {bt->d_rec, d_chunk_map, d_build, d_build_map, d_field, bt->d_mem,
                           bt->d_gs, bt->d_perm, bt->d_tables, bt->d_q, bt->d_w, bt->d_ctl,
-                          bt->sur, bt->capture, bt->d_sur, bt->d_xinf, cap_data.x,
-                          bt->mm.pos_exact, bt->fft.shat, bt->fft.qhat, bt->fft.what};
+                          bt->sur, bt->capture, bt->d_sur, bt->d_xinf, cap_data.x, cap_data.y,
+                          cap_data.u, cap_data.count};
     put(ptrs, sizeof ptrs);
     const uint32_t dims[] = {(uint32_t)B, nr, nz, total_chunks, build_blocks, bt->field_shape,
                              bt->gemm_shape, bt->cus, gemm ? 1u : 0u};
     put(dims, sizeof dims);
     put(&bt->aspect_lnr, sizeof bt->aspect_lnr);
-    const size_t max_lds = sc_on ? m0->sc->max_lds : 0;
-    put(&max_lds, sizeof max_lds);
+    // the network's inference buffers, which another batch may make it replace
+    const uint64_t infer = bt->sur ? net_infer_id(net_of(bt->sur)) : 0;
+    put(&infer, sizeof infer);
     if (!bt->pgraph_exec || sig != bt->pgraph_sig) {
       if (bt->pgraph_exec) { (void)hipGraphExecDestroy(bt->pgraph_exec); bt->pgraph_exec = nullptr; }
       HPS_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeGlobal));

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -85,6 +86,7 @@ struct NetImpl {
   int hist_cap = 0;
   // inference buffers (the batch engine) for inf_b samples
   int inf_b = 0;
+  uint64_t inf_id = 0;
   std::vector<float*> iout;
   float* iscale = nullptr;
   // dataset
@@ -324,6 +326,8 @@ int net_reserve_infer(NetImpl* n, int B)
   (void)hipFree(n->iscale);
   n->iscale = nullptr;
   n->inf_b = B;
+  static std::atomic<uint64_t> last_id{0};
+  n->inf_id = ++last_id;
   for (const Layer& l : n->layers) {
     float* p = nullptr;
     NN_CHECK(hipMalloc(&p, act_size(l, B) * 4));
@@ -333,6 +337,8 @@ int net_reserve_infer(NetImpl* n, int B)
   int held = 0;
   return upload_film(n, B, n->d_film_inf, &held);
 }
+
+uint64_t net_infer_id(const NetImpl* n) { return n->inf_id; }
 
 int net_data(NetImpl* n, NetData* out)
 {

@@ -103,6 +103,9 @@ int net_infer(NetImpl* n, const float* x, const float* u, const uint32_t* dyn_b,
               float** y, hipStream_t s);
 // inference buffers for up to B samples (allocates; call before capture)
 int net_reserve_infer(NetImpl* n, int B);
+// of the present inference buffers: another number for every reservation
+// that replaced them, and for every network
+uint64_t net_infer_id(const NetImpl* n);
 // device dataset the batch appends (charge, field) pairs to
 struct NetData {
   float *x, *y, *u;          // [cap][nz][cin], [cap][zn][cout], [cap] (log aspect)

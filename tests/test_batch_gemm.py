@@ -383,3 +383,50 @@ def test_deposit_shares_give_the_same_bits(nr, nz, num):
         assert np.array_equal(bins, ref[1])
         for k in ref[0]:
             assert np.array_equal(a[k].view(np.uint32), ref[0][k].view(np.uint32)), (n, k)
+
+
+def test_period_graph_follows_replaced_buffers():
+    """A captured lattice period is not replayed past its buffers: another
+    batch with more members makes a shared network replace its inference
+    buffers, a run on another mesh those of the grouped solve.  Every run gives
+    the bits of eager launches."""
+    from hpsim_amd import surrogate as S
+
+    def runs(graph):
+        wl = cfg.config(0, num=2000, periods=6)
+        lat = cfg.build_lattice(wl.lattice)
+        net = S.Network(nr=32, nz=128, widths=(16, 16, 32, 32), nbot=1, max_batch=4, seed=2)
+        net.set_norm(1e-9, 0.0, 1.0)
+        made = [S.make_batch(cfg.BatchWorkload(wl.name, [wl.beam] * n, [lat] * n, nr=32, nz=128,
+                                               interval=wl.interval)) for n in (1, 3)]
+        out = []
+
+        def go(k, on=graph):
+            batch, objs = made[k]
+            for b, _, m in objs:
+                b.restore_initial_beam()
+                m.reset()
+            batch.set_graph(on)
+            batch.simulate()
+            out.extend(b.arrays() for b, _, _ in objs)
+
+        for batch, objs in made:
+            batch.set_gemm_shape(8)
+            S.attach(batch, net, audit_every=3)
+            for b, _, _ in objs:
+                b.save_initial_beam()
+        go(0), go(0), go(1), go(0)
+        batch, objs = made[0]
+        S.attach(batch, None)
+        objs[0][1].set_mesh_size(16, 64)
+        go(0, False)
+        objs[0][1].set_mesh_size(32, 128)
+        S.attach(batch, net, audit_every=3)
+        go(0), go(0)
+        return out, batch.graph_info()[0]
+
+    (eager, none), (replayed, some) = runs(False), runs(True)
+    assert none == 0 and some > 0
+    for k, (a, b) in enumerate(zip(eager, replayed)):
+        assert np.isfinite(a["x"]).all()
+        assert H.compare_arrays(b, a, f"run {k}: ") is None
