@@ -203,6 +203,8 @@ int pull(hps_beam* b, hps_beam_stats* s)
   return 0;
 }
 
+// Enqueues the write and returns: whatever reads the statistics next is on the
+// beam's stream too (one per device), so it comes after.
 int push(hps_beam* b, const hps_beam_stats& s)
 {
   HPS_CHECK(launch_set_stats(b->st, s, b->stream));

@@ -132,6 +132,11 @@ int hps_beam_set_dc(hps_beam* b, double ax, double bx, double ex, double ay, dou
  * of log and cos).  No reference counterpart (the reference samples on the
  * host, beam.cpp:391-537). */
 int hps_beam_sample_gaussian(hps_beam* b, uint32_t seed, const double* center, const double* sigma);
+/* The calls of a beam run in order on its device's one stream.  A getter
+ * returns when its value is there, hps_beam_restore when the particles have
+ * been read back; the statistics they update may still be on their way to the
+ * device.  Calls that follow see them; an error in that write is reported by
+ * the next call that waits. */
 /* Copy coordinates to host; any pointer may be NULL.  Replaces the array
  * part of get_x/get_xp/.../get_losses, wrap_beam.cpp:440-912. */
 int hps_beam_download(hps_beam* b, double* x, double* xp, double* y, double* yp,
