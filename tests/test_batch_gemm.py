@@ -137,6 +137,67 @@ def test_spectral_product_equals_direct_product_at_64x256():
         assert err < 1e-5, (k, err)
 
 
+@pytest.mark.parametrize("nr,nz", [(8, 1024), (8, 2048)])
+def test_spectral_product_of_one_row_per_workgroup(nr, nz):
+    """Transforms of 2,048 and 4,096 entries: one row fills a workgroup, and
+    the longer one takes every thread more than one turn.  Spectral against
+    direct product, with the bound of the test above (as many bins)."""
+    bw = cfg.combined_stress(nbeams=2, num=20000, periods=1)
+    bw.nr, bw.nz = nr, nz
+    fields = []
+    for shape in (0, 8):
+        objs = _members(bw, range(2))
+        bt = _gemm_batch(objs, shape)
+        bt.simulate(0, 0)
+        assert bt.gemm_info()["shape"] == shape
+        fields.append([s.tables()[1] for _, s, _ in objs])
+        del bt, objs
+    for k, (d, f) in enumerate(zip(*fields)):
+        err = np.linalg.norm(f - d) / np.linalg.norm(d)
+        print(f"{nr} x {nz}, beam {k}: spectral vs direct relative L2 {err:.2e}", flush=True)
+        assert err < 1e-5, (k, err)
+
+
+def test_schedule_of_the_largest_batch():
+    """4,095 members, the most a batch takes (the schedule of a kick point holds
+    66 KB of LDS): each gives the bits it gives in a batch of three."""
+    from hpsim_amd import HPSim
+    wl = cfg.config(0, num=200, periods=1)
+    line = HPSim.BeamLine(elements=cfg.build_lattice(wl.lattice)[:4])
+    dists = []
+    for k in range(3):
+        d = [np.array(v) for v in cfg.make_distribution(wl.beam)]
+        for q in (0, 2):
+            d[q] *= 1.0 + 0.4 * k
+        dists.append(d)
+
+    def run(n):
+        sims = []
+        for k in range(n):
+            b = HPSim.Beam(mass=wl.beam.mass, charge=wl.beam.charge, current=wl.beam.current,
+                           num=wl.beam.num)
+            b.set_distribution(*dists[k % 3])
+            b.set_frequency(wl.beam.freq)
+            b.set_ref_w(wl.beam.w0)
+            sims.append(HPSim.Simulator(b, line, HPSim.SpaceCharge(nr=4, nz=64,
+                                                                   interval=wl.interval)))
+        batch = HPSim.Batch(sims)
+        batch.set_field_mode("gemm", STEP)
+        batch.set_gemm_shape(8)
+        batch.simulate()
+        assert batch.gemm_info()["conflicts"] == 0
+        return sims
+
+    ref = [(s.beam.arrays(), s.spch.tables()[1]) for s in run(3)]
+    print("three members done", flush=True)
+    sims = run(4095)
+    print("4,095 members done", flush=True)
+    for k in [*range(6), 255, 256, 2048, 4093, 4094]:
+        a, f = sims[k].beam.arrays(), sims[k].spch.tables()[1]
+        assert H.compare_arrays(a, ref[k % 3][0], f"member {k}: ") is None
+        assert np.array_equal(f.view(np.uint64), ref[k % 3][1].view(np.uint64)), k
+
+
 def test_spectral_shape_needs_a_power_of_two_mesh(oracle_lib):
     """On a 16 x 192 mesh (nz a multiple of 64 but not a power of two) the
     frequency-domain shape is not available: asking for it fails with an

@@ -263,10 +263,9 @@ def test_graph_replay_same_simulator():
 @pytest.mark.parametrize("num", [5000, 150000, 600000])
 def test_longitudinal_loss_rescan_bit_exact(num):
     """A 70-degree phase spread pushes particles out of the bucket, so the
-    lloss flags and the chunk rescan path are exercised: 5 chunks (one per
-    wavefront of the rescanning workgroup, one wave taking two), 147 chunks
-    (more than the 64 one rescan round lists) and 586 chunks (the
-    four-particles-per-thread segment kernel)."""
+    lloss flags and the chunk rescan path are exercised: 5 and 147 chunks (one
+    rescan round) and 586 chunks (the four-particles-per-thread segment
+    kernel)."""
     import math
     wl = H.workload(0, num=num, periods=6, sc=True)
     wl.beam.sig_phi = math.radians(70.0)
@@ -278,12 +277,36 @@ def test_longitudinal_loss_rescan_bit_exact(num):
     assert err is None, err
 
 
+@pytest.mark.parametrize("flagged", [17, 40, 256, 257, 310])
+def test_longitudinal_loss_rescan_rounds_bit_exact(flagged):
+    """310 chunks with a particle past the loss threshold in `flagged` of them
+    at the first kick: a rescan round lists 256 on sixteen wavefronts, so from
+    17 on a wavefront takes several and from 257 on there is a second round."""
+    wl = H.workload(0, num=310 * 1024, periods=1, sc=True)
+    dist = [np.array(v) for v in cfg.make_distribution(wl.beam)]
+    phi = dist[4]
+    far = np.arange(flagged) * (310 // flagged if flagged < 256 else 1)
+    phi[far * 1024 + 5 + far % 900] += 20.0
+    # before the first kick every phase advances alike, but for the energy
+    # spread: well inside the distance kept to the threshold here
+    thr = phi.mean() + 3 * np.pi
+    assert (np.abs(phi - thr) > 2.0).all()
+    assert (phi.reshape(310, 1024) > thr).any(axis=1).sum() == flagged
+    ob, osc, _ = H.run_oracle(wl, dist=dist)
+    gb, gsc, _ = H.run_gpu(wl, dist=dist)
+    oa = ob.arrays()
+    assert (oa["lloss"] != 0).sum() >= flagged
+    err = H.compare_arrays(gb.arrays(), oa)
+    assert err is None, err
+
+
 @pytest.mark.parametrize("num", [400_000, 1_500_000, 2_500_000])
 def test_cross_chunk_tree_widths_bit_exact(num):
     """Beams of 391, 1,465 and 2,442 chunks: the cross-chunk trees run with
-    2, 8 and 16 entries per thread (chunk partials padded to 512, 2,048 and
-    4,096), each a specialised load-then-fold path, with the 70-degree phase
-    spread so the chunk maxima of the longitudinal-loss test are live."""
+    8, 32 and 64 entries per lane (chunk partials padded to 512, 2,048 and
+    4,096; the last two in two and four batches of loads), each a specialised
+    load-then-fold path, with the 70-degree phase spread so the chunk maxima of
+    the longitudinal-loss test are live."""
     import math
     wl = H.workload(0, num=num, periods=2, sc=True)
     wl.beam.sig_phi = math.radians(70.0)
@@ -404,7 +427,7 @@ def test_waterbag_and_dc_beams_match_oracle_then_track(oracle_lib):
 @pytest.mark.parametrize("nr,nz", [(32, 128), (16, 64), (7, 33), (64, 256)])
 def test_space_charge_tables_bit_exact(nr, nz):
     """Green's table, charge histogram and field table of the last remesh,
-    for several mesh shapes (the LDS-staged and the direct field kernel)."""
+    for several mesh shapes (four and nine waves a workgroup, few rings)."""
     wl = H.workload(0, num=8192, periods=2, sc=True)
     wl.nr, wl.nz = nr, nz
     ob, osc, _ = H.run_oracle(wl)
@@ -412,6 +435,23 @@ def test_space_charge_tables_bit_exact(nr, nz):
     assert gsc.state()["remesh_count"] == osc.state()["remesh_count"] > 0
     for name, g, o in zip(("greens", "field", "bins"), gsc.tables(), osc.tables()):
         assert g.shape == o.shape, name
+        assert np.array_equal(g.view(np.uint64), o.view(np.uint64)), name
+    err = H.compare_arrays(gb.arrays(), ob.arrays())
+    assert err is None, err
+
+
+@pytest.mark.parametrize("nr,nz", [
+    (70, 3),      # more rings than a wave's partials (a second turn of its lanes), one row block
+    (70, 40),     # the same over several row blocks
+    (4, 8)])      # fewer rows than the window holds: the tail alone
+def test_field_window_edges_bit_exact(nr, nz):
+    """The field sum where its window of row blocks is not filled, or refilled."""
+    wl = H.workload(0, num=8192, periods=1, sc=True)
+    wl.nr, wl.nz = nr, nz
+    ob, osc, _ = H.run_oracle(wl)
+    gb, gsc, _ = H.run_gpu(wl)
+    assert gsc.state()["remesh_count"] == osc.state()["remesh_count"] > 0
+    for name, g, o in zip(("greens", "field", "bins"), gsc.tables(), osc.tables()):
         assert np.array_equal(g.view(np.uint64), o.view(np.uint64)), name
     err = H.compare_arrays(gb.arrays(), ob.arrays())
     assert err is None, err
