@@ -6,21 +6,26 @@
 //
 // Built with -fapprox-func and -freciprocal-math, an FP64 quotient x / y
 // becomes v_rcp_f64(y), two Newton steps, x times the refined reciprocal and
-// one FMA correction (7 instructions instead of 11).  It skips the
-// v_div_scale / v_div_fmas / v_div_fixup steps of the correctly rounded
-// sequence, and quotients by one denominator share its reciprocal (x times
-// the rounded 1 / y).  With HPS_FAST_PUSH defined, the square roots of the
-// maps, the kick and the deposit (psqrt, hps_math.hpp) come from v_rsq_f64
-// with one Goldschmidt step and one Newton correction (12 instructions
-// instead of 21).  Measured on the device, both gave the correctly rounded
-// result for every one of 400,000 random quotients and roots between
-// 10^-200 and 10^200.  A zero or infinite denominator gives NaN instead of
-// an infinity or zero.  The push guards the denominators that can be zero:
-// r and the gap radius on the axis, and bgzf <= 0 is a loss.  Every other
-// denominator is a mass, a mesh spacing, or a velocity or energy that is
-// positive for any particle still alive.  Static VALU instruction counts of
-// the batched push drop by 12 % (quad class) and 15 % (RF-gap class), and
-// by 10 % in the batched deposit.
+// one FMA correction (7 instructions; the compiler's correctly rounded
+// sequence takes 11, the exact build's Quick 9, see hps_math.hpp), and
+// quotients by one denominator share its reciprocal (x times the rounded
+// 1 / y).  With HPS_FAST_PUSH defined, the square roots of the maps, the kick
+// and the deposit (psqrt) come from v_rsq_f64 with one Goldschmidt step and
+// one Newton correction (12 instructions instead of 21; Quick 10).  Measured
+// on the device, both gave the correctly rounded result for every one of
+// 400,000 random quotients and roots between 10^-200 and 10^200.  A zero or
+// infinite denominator gives NaN instead of an infinity or zero.  The push
+// guards the denominators that can be zero: r and the gap radius on the axis,
+// and bgzf <= 0 is a loss.  Every other denominator is a mass, a mesh spacing,
+// or a velocity or energy that is positive for any particle still alive.
+//
+// Against the same file built with correctly rounded quotients and roots and
+// the full polynomials (Any, hps_math.hpp; the live-particle push in both),
+// static VALU instruction counts of the batched push drop by 12 % (quad class)
+// and 17 % (RF-gap class), and by 11 % in the batched deposit.  Four members of
+// 2,097,152 particles on 64 x 256: push 251 -> 247 us (quad) and 260 -> 249 us
+// (RF gap) a launch, rebuild 96 -> 77.  So the push, bound by its memory
+// accesses, gains little by now; the deposit is what the second build pays for.
 //
 // The batched push of this build visits only the live particles of each
 // chunk (segment_body_live in hps_kernels.hip).  It adds each chunk's sums
