@@ -249,10 +249,11 @@ __global__ __launch_bounds__(kFftThreads) void k_fft_forward(
 //
 // A slot of at most kProdVec columns takes the vector form: the product is
 // then bound by reading S^ (17 MB a slot at 64 x 256), and a matrix tile
-// would multiply 28 to 31 empty columns for it (four members on 64 x 256:
-// 111 -> 38 us a kick point; seven on 32 x 128: 32 -> 17 us).  One lane per (f, row), S^ coalesced along row,
-// kRing rings in flight; the charges of a frequency are the same address for
-// its lanes.  VALU and matrix cores break even at about six columns of 16.
+// would multiply 12 to 15 empty columns for it (four members on 64 x 256:
+// 111 -> 48 us a kick point; seven on 32 x 128: 32 -> 17 us).  One lane per
+// (f, row), S^ coalesced along row, kRing rings in flight; the charges of a
+// frequency are the same address for its lanes.  kProdVec of 2 / 4 / 6 / 8: 57 /
+// 48 / 54 / 59 us for the former, 17.8 / 16.6 / 16.6 / 16.6 for the latter.
 template <int NC>
 __device__ __forceinline__ void product_rows(const float2* __restrict__ S,
                                              const float2* __restrict__ qhat,
@@ -474,6 +475,11 @@ bool fft_product_supported(uint32_t nr, uint32_t nz)
          L <= (uint32_t)kFftMaxL && 2 * nr <= (uint32_t)kProdMaxK;
 }
 
+// Workgroups a CU: the transforms' 52 KB of LDS leave room for three, the
+// product's 17 KB for nine.  Four members on 64 x 256, us a kick point: the
+// forward transforms 14.3 / 11.7 / 11.5 with one / two / four, the product 57 /
+// 48 / 48 with four / eight / sixteen; seven members on 32 x 128 differ by less
+// than the runs.
 hipError_t launch_fft_product(const GemmMember* mem, uint32_t nmem, const GemmState* gs,
                               const uint32_t* perm, const int32_t* pos_exact,
                               const float* tables, float* w, const FftBufs& fb, uint32_t nr,

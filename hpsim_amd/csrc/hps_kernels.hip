@@ -2405,8 +2405,9 @@ uint32_t field_batch_shapes() { return kFieldShapes; }
 // more than half of the LDS a CU holds one workgroup, so it takes nine waves,
 // as many as its registers allow (64 x 256, 2,145 waves on 239 workgroups:
 // 109 us a kick point; eight waves are a second round of workgroups, 127;
-// four 130); otherwise several small ones (four waves; nine 163, two 156 on
-// the seven members).
+// four 130; the sum alone, nine and four waves: 44.0 and 64.4 us there, 39.8
+// and 42.9 on 48 x 256, 35.4 and 39.8 on 128 x 100); otherwise several small
+// ones (four waves; nine 163, two 156 on the seven members).
 uint32_t field_batch_default_shape(uint32_t nr, uint32_t nz, uint32_t nmem)
 {
   const uint32_t k = field_shape(nr, nz, 8, 1).g.units * (uint64_t)nmem >= 1024 ? 0 : 1;

@@ -52,8 +52,14 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;
 constexpr int kMaxFrag = kMaxCout / 16;
-// output positions from which a conv workgroup takes two position tiles (each
-// weight fragment then serves two products)
+// Output positions from which a conv workgroup takes two position tiles: each
+// weight fragment then serves two products, but the workgroups are half as
+// many.  The line was set without a sweep and lies lower than the sizes below
+// ask for: two tiles pay only on a device that is full either way.  The same
+// run with two tiles from 4,096 positions on, one tile always, and two from
+// 20,000 on: training, 64 samples on 32 x 128 (at most 8,704 positions) 7.8 /
+// 7.0 / 7.0 ms, on 64 x 256 (16,896) 9.5 / 8.5 / 8.5; 160 beams of 32 x 128 with
+// surrogate fields (21,760) 5.1 / 4.9 / 4.8.  The bits are the same either way.
 constexpr int kConvTwoTiles = 4096;
 
 __host__ __device__ inline int cdiv(int a, int b) { return (a + b - 1) / b; }

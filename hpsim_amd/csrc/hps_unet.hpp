@@ -38,7 +38,10 @@ struct WgradArgs {
   int B, Zin, Zout, Cin, Cout, taps, dil, mode;
 };
 
-// rows of z in one slab of the FiLM gradient, and the slabs of Z rows
+// Rows of z in one slab of the FiLM gradient, and the slabs of Z rows.  A
+// layer of k_film_bwd at 64 samples of up to 136 rows: 3.5 us with 17, 3.7 with
+// 34, 3.8 with 68 (runs of one differ by 0.1); fewer slabs are fewer sums to
+// store and add up.
 constexpr int kFilmSlab = 34;
 inline int film_slabs(int Z) { return (Z + kFilmSlab - 1) / kFilmSlab; }
 
